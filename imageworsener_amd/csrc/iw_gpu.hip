@@ -15,7 +15,9 @@
 //                   band products with FP32 sums, the per-pixel work in FP64.
 //   errdiff      -- one workgroup per error-diffused plane walking the
 //                   reference's serpentine order (src/imagew-main.c:497-567,
-//                   1072-1136).
+//                   1072-1136): errdiff_rows_kernel with the rows in registers
+//                   (its codes gathered into pixels by edr_interleave_kernel),
+//                   errdiff_kernel for wider rows and more levels.
 // Batches and the request loop run the same kernels over a descriptor table
 // of many plans (persistent band kernels, hipGraph replay).
 //
@@ -122,6 +124,7 @@ struct DevPlan {
 	double *ed_err;
 	int n_ed;
 	int ed_seg;             // fewest pixels per error-diffusion segment
+	int ed_shift;           // layout of the samples (ed_sample_at); nonzero: diffused by errdiff_rows_kernel
 	// Per-request completion (request loop only; null otherwise): the last
 	// error-diffusion plane of a request to finish copies the output image to
 	// host memory and raises the flag there.
@@ -141,6 +144,16 @@ struct DevPlan {
 	const int4 *h4i;
 	const float *h4w;
 };
+
+// Where row pixel x of W lies in a plane's row of error-diffusion samples.
+// shift 0: by x.  Else by segments of 2^shift pixels, the segments' first
+// pixels first, then their second ones, ...: errdiff_rows_kernel's lanes hold
+// one segment each, so their loads are consecutive.
+__device__ __forceinline__ int ed_sample_at(int x, int W, int shift)
+{
+	const int r = x & ((1 << shift) - 1);
+	return r * (W >> shift) + min(r, W & ((1 << shift) - 1)) + (x >> shift);
+}
 
 // ---- input sampling (src/imagew-main.c:129-276) ---------------------------
 
@@ -430,6 +443,7 @@ struct EmitCtx {
 	size_t out_bpr;
 	uint8_t *out;
 	double *ed_samples;
+	int ed_shift;
 	int c[IWAMD_MAX_CH], o[IWAMD_MAX_CH], unassoc[IWAMD_MAX_CH], is_alpha[IWAMD_MAX_CH];
 	DevOChan q[IWAMD_MAX_CH];
 };
@@ -454,6 +468,7 @@ __device__ __forceinline__ void emit_ctx(const DevPlan &P, EmitCtx &E)
 	E.out_bpr = P.out_bpr;
 	E.out = P.out;
 	E.ed_samples = P.ed_samples;
+	E.ed_shift = P.ed_shift;
 #pragma unroll
 	for (int idx = 0; idx < IWAMD_MAX_CH; idx++) {
 		const int c = idx < P.inter_nch ? P.order[idx] : 0;
@@ -476,7 +491,7 @@ __device__ __forceinline__ void emit_ctx(const DevPlan &P, EmitCtx &E)
 // bin-index log2 (9-13).  n: searched entries, or the plane index for error
 // diffusion.
 struct EmitSimple {
-	int nch, intclamp, out_depth, out_nch, out_w, out_h;
+	int nch, intclamp, out_depth, out_nch, out_w, out_h, ed_shift;
 	int pack4;  // 8-bit, four output channels, each written once, none diffused: one 32-bit store per pixel
 	size_t out_bpr;
 	uint8_t *out;
@@ -498,6 +513,7 @@ __host__ __device__ inline bool emit_simple_ctx(const DevPlan &P, EmitSimple &E)
 	E.out_bpr = P.out_bpr;
 	E.out = P.out;
 	E.ed_samples = P.ed_samples;
+	E.ed_shift = P.ed_shift;
 	bool ok = true;
 #pragma unroll
 	for (int idx = 0; idx < IWAMD_MAX_CH; idx++) {
@@ -583,7 +599,8 @@ __device__ __forceinline__ void emit_px(const EmitCtx &E, int i, int j, Gather g
 		}
 		v = clamp01(v);
 		if (q.family == IW_DITHERFAMILY_ERRDIFF) {
-			((__attribute__((address_space(1))) double *)E.ed_samples)[((size_t)q.ed_index * E.out_h + j) * E.out_w + i] = v;
+			((__attribute__((address_space(1))) double *)E.ed_samples)[((size_t)q.ed_index * E.out_h + j) * E.out_w +
+				ed_sample_at(i, E.out_w, E.ed_shift)] = v;
 			continue;
 		}
 		emit_store(E, i, j, o, quantize(q, v, i, j));
@@ -680,7 +697,7 @@ __device__ __forceinline__ void emit_px_simple(const EmitSimple &E, const int (&
 			const double x = v[idx][n];
 			if (f & (1 << 7)) {
 				((__attribute__((address_space(1))) double *)E.ed_samples)[((size_t)E.n[idx] * E.out_h + pj[n]) *
-					E.out_w + pi[n]] = x;
+					E.out_w + ed_sample_at(pi[n], E.out_w, E.ed_shift)] = x;
 				continue;
 			}
 			const int l = lo[idx][n], m = hi[idx][n] - l;
@@ -2237,6 +2254,107 @@ __device__ __forceinline__ void ed_resolve(const EdCtx &c, Lds &S, unsigned shor
 	}
 }
 
+// Pixels x .. x+3 of row j: the codes of the error-diffused channels into
+// their bytes of the output.
+__device__ __forceinline__ void edr_interleave4(const DevPlan &P, int j, int x)
+{
+	const int W = P.out_w, n = min(4, W - x), nc = P.out_nch;
+	const size_t plane = (size_t)P.out_h * W * 8, at = (size_t)j * W * 8;
+	const uint8_t *src = (const uint8_t *)P.ed_samples;
+	g_u8 *dst = (g_u8 *)P.out + (size_t)j * P.out_bpr;
+	if (P.out_depth != 8) {
+		for (int o = 0; o < nc; o++) {
+			if (P.oc[o].family != IW_DITHERFAMILY_ERRDIFF) continue;
+			const g_cu16 *s = (const g_cu16 *)(src + P.oc[o].ed_index * plane + at) + x;
+			for (int i = 0; i < n; i++) {
+				const unsigned int v = s[i];
+				dst[(size_t)(nc * (x + i) + o) * 2] = (uint8_t)(v >> 8);
+				dst[(size_t)(nc * (x + i) + o) * 2 + 1] = (uint8_t)v;
+			}
+		}
+		return;
+	}
+	unsigned int c[IWAMD_MAX_CH];
+	bool ed[IWAMD_MAX_CH];
+#pragma unroll
+	for (int o = 0; o < IWAMD_MAX_CH; o++) {
+		ed[o] = o < nc && P.oc[o].family == IW_DITHERFAMILY_ERRDIFF;
+		c[o] = ed[o] ? *(const __attribute__((address_space(1))) unsigned int *)(src + P.oc[o].ed_index * plane + at + x) : 0u;
+	}
+	if (n == 4 && P.n_ed == nc) {
+		// Every channel of four pixels: whole words.
+		unsigned int w[4];
+		if (nc == 4) {
+#pragma unroll
+			for (int i = 0; i < 4; i++)
+				w[i] = (c[0] >> (8 * i) & 0xffu) | (c[1] >> (8 * i) & 0xffu) << 8 | (c[2] >> (8 * i) & 0xffu) << 16 |
+					(c[3] >> (8 * i) & 0xffu) << 24;
+			__builtin_memcpy(dst + (size_t)4 * x, w, 16);
+			return;
+		}
+		if (nc == 3) {
+			auto b = [&](int k) { return c[k % 3] >> (8 * (k / 3)) & 0xffu; };
+#pragma unroll
+			for (int i = 0; i < 3; i++) w[i] = b(4 * i) | b(4 * i + 1) << 8 | b(4 * i + 2) << 16 | b(4 * i + 3) << 24;
+			__builtin_memcpy(dst + (size_t)3 * x, w, 12);
+			return;
+		}
+		if (nc == 1) {
+			__builtin_memcpy(dst + x, c, 4);
+			return;
+		}
+	}
+#pragma unroll
+	for (int o = 0; o < IWAMD_MAX_CH; o++)
+#pragma unroll
+		for (int i = 0; i < 4; i++)
+			if (ed[o] && i < n) dst[(size_t)nc * (x + i) + o] = (uint8_t)(c[o] >> (8 * i));
+}
+
+// Completion of a request (request loop): the last of its planes to finish
+// copies the whole output to the host and raises the flag.  All nt threads
+// of the workgroup call it, after its last store and a barrier.
+__device__ __forceinline__ void ed_complete(const DevPlan &P, int tid, int nt)
+{
+	if (!P.ed_done) return;
+	__shared__ int last;
+	if (tid == 0) {
+		__threadfence();
+		last = atomicAdd(P.ed_done, 1) == P.n_ed - 1;
+		__threadfence();
+	}
+	__syncthreads();
+	if (!last) return;
+	if (P.ed_shift) {
+		const int q = (P.out_w + 3) >> 2;
+		for (int j = 0; j < P.out_h; j++)
+			for (int t = tid; t < q; t += nt) edr_interleave4(P, j, 4 * t);
+		__syncthreads();
+	}
+	// 8 words per thread in flight: one workgroup's copy is bound by the
+	// latency of its loads.
+	typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+	const size_t n16 = P.out_bytes / 16;
+	const __attribute__((address_space(1))) u32x4 *src = (const __attribute__((address_space(1))) u32x4 *)P.out;
+	__attribute__((address_space(1))) u32x4 *dst = (__attribute__((address_space(1))) u32x4 *)P.host_out;
+	size_t k = tid;
+	for (; k + 7 * (size_t)nt < n16; k += 8 * (size_t)nt) {
+		u32x4 v[8];
+#pragma unroll
+		for (int u = 0; u < 8; u++) v[u] = src[k + u * (size_t)nt];
+#pragma unroll
+		for (int u = 0; u < 8; u++) dst[k + u * (size_t)nt] = v[u];
+	}
+	for (; k < n16; k += nt) dst[k] = src[k];
+	for (size_t k = n16 * 16 + tid; k < P.out_bytes; k += nt) P.host_out[k] = P.out[k];
+	__threadfence_system();
+	__syncthreads();
+	if (tid == 0) {
+		__threadfence_system();
+		__hip_atomic_store(P.host_flag, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+	}
+}
+
 // One workgroup per plane: planes[b] = (plan, output channel).  Per row:
 // waves 0-3 walk the segments while waves 4-7 store the previous row's codes
 // and load the next row's samples; wave 0 checks the boundaries and walks
@@ -2344,30 +2462,505 @@ __global__ void __launch_bounds__(ED_THREADS) errdiff_kernel(const DevPlan *__re
 	}
 	ed_store_row(c, lvl_of(H - 1), H - 1, tid, ED_THREADS);
 	__syncthreads();
-	if (P.ed_done) {
-		// Completion of the request: the last of its planes to finish copies
-		// the whole output to the host and raises the flag.
-		__shared__ int last;
-		if (tid == 0) {
-			__threadfence();
-			last = atomicAdd(P.ed_done, 1) == P.n_ed - 1;
-			__threadfence();
+	ed_complete(P, tid, ED_THREADS);
+}
+
+// ---- error diffusion with the rows in registers -----------------------------
+//
+// The same speculation for rows of up to EDR_MAX_W pixels and up to 257
+// levels, with everything a row needs in registers: lane L of the workgroup
+// keeps pixels x = L*SEG .. L*SEG+SEG-1 of every row (walked upwards on even
+// rows, downwards on odd ones -- the serpentine), so the errors carried to
+// the next rows are formed in place, from the lane's own errors and its
+// neighbours' nearest two (lane shifts; between waves through LDS).
+//
+// A row is a fixed point: each segment's start state is its predecessor's
+// end state.  Every round walks all segments from the start states the last
+// round left (the first from zero) and passes the new end states on; a wave
+// has settled when none of its start states changed, bit for bit.  The row's
+// first segment starts from zero in the reference too, so at the fixed point
+// every segment is the true chain, by induction, and each round makes at
+// least one more segment true; two walks' states meet within a few dozen
+// pixels, so the rounds are few.  Waves read their predecessor's end state as
+// it stands when a round begins, without waiting for it.  One barrier ends
+// the row: after it every wave compares all waves' start states with their
+// predecessors' end states, and all of them go on if any differs.
+//
+// Decision (as ed_decide): the level is #{D <= s} with the folded boundaries
+// D[k] = min(T[k], max(T[k-1], U[k], M[k])) (QuantTable::D), the error
+// s - lin[level], or 0 where s is exact (T[level-1] <= s < U[level]).  Each
+// pixel keeps one boundary D[b] and its two levels, so a walk's step is a
+// product, two sums (the second with the clamp), a compare, a select and a
+// difference.  That decides right for s in [D[b-1], D[b+1]).  The boundary is
+// looked up once per row, for the sample without its in-row carry; samples
+// outside their range are looked up again after each of the first rounds and
+// when a wave has settled, and the walks go on.  So are exact samples found:
+// they lie within `eps` of their level, and one keeps its own value as both
+// levels, which makes its error 0.
+//
+// Bound: one wave's issue of a dependent chain (4 clocks an instruction, 9 a
+// step, about 55 steps to settle a Floyd-Steinberg row) on one workgroup per
+// plane, then the votes and exchanges between rounds.  So a row is spread
+// over as many waves as give each its own SIMD: segments of 4 pixels up to
+// 1024 wide, of 8 beyond (16 pixels on 4 waves do not fit the registers:
+// 3072-wide rows 10.0 us against 8.7).  Measured per row, errdiff_kernel ->
+// this kernel: Floyd-Steinberg 1000 pixels 16.7 -> 4.0 us, 2500 pixels
+// 22.2 -> 5.6 us, 200 pixels 12.7 -> 2.9 us; Jarvis-Judice-Ninke to 4 levels,
+// 3072 pixels, 23.1 -> 8.7 us.
+//
+// The samples come segment-transposed (ed_sample_at), so that a wave's loads
+// are consecutive, and the codes go out planar over the samples already
+// read; edr_interleave_kernel forms the pixels (byte stores at the pixels'
+// stride held up the rows: 2500-wide RGB 12 us a row with them).
+
+#define EDR_MAX_W 4096   // 8 waves of 64 segments of 8 pixels
+
+// One wave's row as its neighbours see it: its first and last two errors (by
+// x: the end state of a walk downwards or upwards) and the start state its
+// walks used at the end they start from.
+struct EdrEdge {
+	double first[2], last[2], used[2];
+};
+
+// D[0] = -1, D[1 + k] = boundary k, then 4.0: every sample lies in some range.
+template <int NW>
+struct EdrLds {
+	double D[ED_LDS_TABLE + 4];
+	double lin[ED_LDS_TABLE + 2];
+	double lo[ED_LDS_TABLE + 1], hi[ED_LDS_TABLE + 1];  // level k's exact samples: [lo[k], hi[k])
+	unsigned short Q[ED_NB];                 // first guess of b by s * ED_NB
+	unsigned short code[ED_LDS_TABLE + 1];   // output code per level
+	unsigned long long eps;                  // bits of the widest distance of an exact sample from its level
+	EdrEdge edge[2][NW];
+	double hold[NW + 1][2];  // a wave's predecessor's state once it is fixed; [NW]: zero
+};
+
+template <bool M1, int SEG>
+struct EdrRow {
+	double X[SEG], Y[SEG];      // samples; errors carried from the rows above
+	double S[SEG], E[SEG];      // the walks' clamped sums and errors
+	double R1[M1 ? SEG : 1];    // the previous row's share for the row after next
+	double Dm[SEG], D[SEG], Dp[SEG], A[SEG], B[SEG];  // D[b-1], D[b], D[b+1], lin[b], lin[b+1]
+	int b[SEG];
+	unsigned int ex;            // pixels whose sample is exact
+};
+
+// Lane i gets lane i-1's value (UP) or lane i+1's; the end lane, which has no
+// neighbour there, gets its own `edge`.
+template <bool UP>
+__device__ __forceinline__ double edr_shift(double v, double edge)
+{
+	constexpr int ctrl = UP ? 0x138 : 0x130;  // wave_shr:1, wave_shl:1
+	const long long a = __double_as_longlong(v), e = __double_as_longlong(edge);
+	const int lo = __builtin_amdgcn_update_dpp((int)e, (int)a, ctrl, 0xf, 0xf, false);
+	const int hi = __builtin_amdgcn_update_dpp((int)(e >> 32), (int)(a >> 32), ctrl, 0xf, 0xf, false);
+	return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+
+__device__ __forceinline__ double edr_get(const double *p)
+{
+	return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+__device__ __forceinline__ void edr_put(double *p, double v)
+{
+	__hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+// Pixel i's boundary for sample s: the index's guess; SETTLE: stepped until
+// s lies in its range.
+template <bool SETTLE, bool M1, int SEG, class Lds>
+__device__ __forceinline__ void edr_lookup(EdrRow<M1, SEG> &r, const Lds &S, int i, double s)
+{
+	int b = S.Q[min((int)(s * ED_NB), ED_NB - 1)];
+	if (SETTLE) {
+		while (s < S.D[b]) b--;
+		while (s >= S.D[b + 2]) b++;
+	}
+	r.b[i] = b;
+	r.Dm[i] = S.D[b];
+	r.D[i] = S.D[b + 1];
+	r.Dp[i] = S.D[b + 2];
+	r.A[i] = S.lin[b];
+	r.B[i] = S.lin[b + 1];
+}
+
+// a where d < 0, else b (d is not -0.0): by the sign bit, since a compare's
+// result is not ready for the select for two instructions (the empty asm
+// keeps the compiler from making a compare of it).
+__device__ __forceinline__ double edr_select(double d, double a, double b)
+{
+	const long long m = __double_as_longlong(d), x = __double_as_longlong(a), y = __double_as_longlong(b);
+	unsigned int k = (unsigned int)((int)(m >> 32) >> 31);
+	asm("" : "+v"(k));
+	const unsigned int lo = ((unsigned int)x & k) | ((unsigned int)y & ~k);
+	const unsigned int hi = ((unsigned int)(x >> 32) & k) | ((unsigned int)(y >> 32) & ~k);
+	return __longlong_as_double(((long long)hi << 32) | lo);
+}
+
+// One walk of the lane's segment from state (p1, p2), in the row's direction;
+// the state after it comes back in (p1, p2).  The terms are added in the
+// reference's order (ed_step).
+template <bool REV, bool M1, int SEG>
+__device__ __forceinline__ void edr_walk(EdrRow<M1, SEG> &r, double m0, double m1, double &p1, double &p2)
+{
+#pragma unroll
+	for (int k = 0; k < SEG; k++) {
+		const int i = REV ? SEG - 1 - k : k;
+		const double cell = M1 ? (r.Y[i] + p2 * m1) + p1 * m0 : r.Y[i] + p1 * m0;
+		const double s = fmin(fmax(r.X[i] + cell, 0.0), 1.0);
+		const double e = s - edr_select(s - r.D[i], r.A[i], r.B[i]);
+		r.S[i] = s;
+		r.E[i] = e;
+		p2 = p1;
+		p1 = e;
+	}
+}
+
+__device__ __forceinline__ bool edr_any(bool v)
+{
+	return __builtin_amdgcn_ballot_w64(v) != 0;
+}
+
+// Whether a sample of the lane's n pixels is outside its range.
+template <bool M1, int SEG>
+__device__ __forceinline__ bool edr_outside(const EdrRow<M1, SEG> &r, int n)
+{
+	bool any = false;
+#pragma unroll
+	for (int i = 0; i < SEG; i++) any |= (i < n) & ((r.S[i] < r.Dm[i]) | (r.S[i] >= r.Dp[i]));
+	return any;
+}
+
+// Whether one of the lane's errors is nonzero and at most about eps: high
+// word - 1 below eps_hi (0 wraps round, and so is not near).
+template <bool M1, int SEG>
+__device__ __forceinline__ bool edr_near(const EdrRow<M1, SEG> &r, unsigned int eps_hi)
+{
+	unsigned int near = 0xffffffffu;
+#pragma unroll
+	for (int i = 0; i < SEG; i++)
+		near = min(near, ((unsigned int)(__double_as_longlong(r.E[i]) >> 32) & 0x7fffffffu) - 1u);
+	return near < eps_hi;
+}
+
+// New boundaries for those of the lane's n pixels whose sample is outside its
+// range; EXACT: then marks those whose sample has become exact and unmarks
+// those whose sample has changed.  True where anything did.
+template <bool EXACT, bool M1, int SEG, class Lds>
+__device__ __forceinline__ bool edr_repair(EdrRow<M1, SEG> &r, const Lds &S, int n)
+{
+	bool changed = false;
+#pragma unroll
+	for (int i = 0; i < SEG; i++) {
+		const double s = r.S[i];
+		const bool stale = EXACT && (r.ex >> i & 1u) && r.E[i] != 0.0;
+		if ((i < n) & ((s < r.Dm[i]) | (s >= r.Dp[i]) | stale)) {
+			edr_lookup<true>(r, S, i, s);
+			r.ex &= ~(1u << i);
+			changed = true;
 		}
-		__syncthreads();
-		if (last) {
-			const size_t n16 = P.out_bytes / 16;
-			const uint4 *src = (const uint4 *)P.out;
-			uint4 *dst = (uint4 *)P.host_out;
-			for (size_t k = tid; k < n16; k += ED_THREADS) dst[k] = src[k];
-			for (size_t k = n16 * 16 + tid; k < P.out_bytes; k += ED_THREADS) P.host_out[k] = P.out[k];
-			__threadfence_system();
-			__syncthreads();
-			if (tid == 0) {
-				__threadfence_system();
-				__hip_atomic_store(P.host_flag, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+		if (EXACT && i < n && r.E[i] != 0.0) {
+			const int k = r.b[i] + (s >= r.D[i] ? 1 : 0);
+			if (s >= S.lo[k] && s < S.hi[k]) {
+				r.A[i] = r.B[i] = s;
+				r.ex |= 1u << i;
+				changed = true;
 			}
 		}
 	}
+	return changed;
+}
+
+struct EdrCtx {
+	double *samp;             // the plane's clamped samples [H][W] (ed_sample_at), then its codes
+	const double *m;          // the matrix
+	double m0, m1;
+	unsigned int eps_hi;
+	int W, H;
+	int x0, n;                // the lane's first pixel and how many it has
+	int out_depth, code_is_level;
+	int par;                  // LDS slot of the current row (alternates at each barrier)
+};
+
+// The lane's samples of row j, 0.0 past the row's end.
+template <int SEG>
+__device__ __forceinline__ void edr_load(const EdrCtx &c, int j, double (&v)[SEG])
+{
+	g_cf64 *row = (g_cf64 *)c.samp + (size_t)min(j, c.H - 1) * c.W;
+#pragma unroll
+	for (int i = 0; i < SEG; i++) {
+		const double s = row[ed_sample_at(min(c.x0 + i, c.W - 1), c.W, SEG == 8 ? 3 : 2)];
+		v[i] = i < c.n ? s : 0.0;
+	}
+}
+
+template <bool REV, bool M1, int SEG, int NW>
+__device__ __forceinline__ void edr_row(EdrCtx &c, EdrRow<M1, SEG> &r, double (&nx)[SEG], EdrLds<NW> &S, int j)
+{
+	const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const int from = REV ? 63 : 0, prev = REV ? wave + 1 : wave - 1;
+	const bool has_prev = prev >= 0 && prev < NW;
+	// Errors carried from the rows above: what row j-2 left in R1, then row
+	// j-1's sources in its scan order (that row ran the other way).  R1 takes
+	// row j-1's share for row j+1.  Floyd-Steinberg and Sierra 4-2-1 reach one
+	// pixel and one row.
+	{
+		double l1 = 0.0, l2 = 0.0, n1 = 0.0, n2 = 0.0;
+		if (NW > 1) {
+			// Lane 0 and lane 63 take the neighbouring waves' errors.
+			if (wave > 0) {
+				l1 = edr_get(&S.edge[c.par ^ 1][wave - 1].last[0]);
+				if (M1) l2 = edr_get(&S.edge[c.par ^ 1][wave - 1].last[1]);
+			}
+			if (wave < NW - 1) {
+				n1 = edr_get(&S.edge[c.par ^ 1][wave + 1].first[0]);
+				if (M1) n2 = edr_get(&S.edge[c.par ^ 1][wave + 1].first[1]);
+			}
+		}
+		double E[SEG + 4];
+		E[0] = M1 ? edr_shift<true>(r.E[SEG - 2], l2) : 0.0;
+		E[1] = edr_shift<true>(r.E[SEG - 1], l1);
+#pragma unroll
+		for (int i = 0; i < SEG; i++) E[2 + i] = r.E[i];
+		E[SEG + 2] = edr_shift<false>(r.E[0], n1);
+		E[SEG + 3] = M1 ? edr_shift<false>(r.E[1], n2) : 0.0;
+#pragma unroll
+		for (int i = 0; i < SEG; i++) {
+			double e = M1 ? r.R1[i] : 0.0, a2 = 0.0;
+#pragma unroll
+			for (int dd = M1 ? -2 : -1; dd <= (M1 ? 2 : 1); dd++) {
+				// The source dd places on in row j-1's scan.
+				const double er = E[2 + i + (REV ? dd : -dd)];
+				e = e + er * c.m[4 - dd];
+				if (M1) a2 = a2 + er * c.m[9 - dd];
+			}
+			r.Y[i] = i < c.n ? e : 0.0;
+			if (M1) r.R1[i] = a2;
+		}
+	}
+#pragma unroll
+	for (int i = 0; i < SEG; i++) edr_lookup<false>(r, S, i, fmin(fmax(r.X[i] + r.Y[i], 0.0), 1.0));
+	r.ex = 0;
+
+	// (u1, u2): the state the last walk started from; pend: the predecessor
+	// wave's end state, for the lane next to it.
+	const double *pend = !has_prev ? S.hold[NW] : (REV ? S.edge[c.par][prev].first : S.edge[c.par][prev].last);
+	const bool busy = edr_any(c.n > 0);
+	double u1 = 0.0, u2 = 0.0;
+	bool go = busy, live = true;
+	// One round; true in lanes whose start state changes by it.
+	auto round = [&]() {
+		// Until the row's first barrier the predecessor's state is read as it
+		// stands; after one, as it stood there, so every barrier settles one
+		// more wave for good.
+		double w1 = 0.0, w2 = 0.0;
+		if (NW > 1) {
+			w1 = edr_get(pend);
+			if (M1) w2 = edr_get(pend + 1);
+		}
+		double e1 = u1, e2 = u2;
+		edr_walk<REV>(r, c.m0, c.m1, e1, e2);
+		const double s1 = edr_shift<!REV>(e1, w1), s2 = M1 ? edr_shift<!REV>(e2, w2) : 0.0;
+		// (After the shift: LDS operations return in order, so a write before
+		// it would be waited for with the read.)
+		if (NW > 1 && live && lane == 63 - from) {
+			double *p = REV ? S.edge[c.par][wave].first : S.edge[c.par][wave].last;
+			edr_put(p, e1);
+			if (M1) edr_put(p + 1, e2);
+		}
+		const bool changed = (c.n > 0) & ((s1 != u1) | (M1 && s2 != u2));
+		u1 = s1;
+		u2 = s2;
+		return changed;
+	};
+	// The passes end by the induction above, one per wave at most; the count
+	// only bounds them.
+	int budget = 1 << 16;
+	for (int pass = 0; pass <= 2 * NW; pass++) {
+		const bool walked = go;
+		if (go) {
+			if (live) {
+				// Samples outside their ranges are looked up again after 8 and
+				// 16 pixels' walks; and no wave settles within about
+				// 40, so the rounds up to there are not asked.
+				for (int k = 0; k < 2; k++) {
+#pragma unroll
+					for (int t = 0; t < 8 / SEG; t++) (void)round();
+					if (__builtin_expect(edr_any(edr_outside(r, c.n)), 0)) (void)edr_repair<false>(r, S, c.n);
+				}
+				for (int k = 0; k < 24 / SEG; k++) (void)round();
+			}
+			// A round makes one more segment true (64 * NW at most, following
+			// the predecessors), a repair one more pixel: the budget, far
+			// above that, only bounds the loop.
+			while (budget > 0) {
+				do {
+#pragma unroll
+					for (int k2 = SEG; k2 < 8; k2 += SEG) (void)round();
+					budget--;
+				} while (edr_any(round()) && budget > 0);
+				// (`|`: one vote for the three.)
+				if (!edr_any(edr_outside(r, c.n) | edr_near(r, c.eps_hi) | (r.ex != 0))) break;
+				if (!edr_any(edr_repair<true>(r, S, c.n))) break;
+			}
+		}
+		if (walked) {
+#pragma unroll
+			for (int i = 0; i < SEG; i++)
+				if (i >= c.n) r.E[i] = 0.0;
+		}
+		if (NW == 1) break;
+		EdrEdge &g = S.edge[c.par][wave];
+		if (lane == 0) {
+			edr_put(&g.first[0], r.E[0]);
+			edr_put(&g.first[1], r.E[1]);
+		}
+		if (lane == 63) {
+			edr_put(&g.last[0], r.E[SEG - 1]);
+			edr_put(&g.last[1], r.E[SEG - 2]);
+		}
+		if (lane == from) {
+			edr_put(&g.used[0], u1);
+			edr_put(&g.used[1], u2);
+		}
+		__syncthreads();
+		// Every wave's start against its predecessor's end, one wave per lane.
+		const int before = REV ? lane + 1 : lane - 1;
+		bool off = false;
+		if (lane < NW && before >= 0 && before < NW && lane * 64 * SEG < c.W) {
+			const double *used = S.edge[c.par][lane].used;
+			const double *p = REV ? S.edge[c.par][before].first : S.edge[c.par][before].last;
+			off = edr_get(p) != edr_get(used) || (M1 && edr_get(p + 1) != edr_get(used + 1));
+		}
+		double w1 = 0.0, w2 = 0.0;
+		if (has_prev) {
+			const double *p = REV ? S.edge[c.par][prev].first : S.edge[c.par][prev].last;
+			w1 = edr_get(p);
+			if (M1) w2 = edr_get(p + 1);
+		}
+		c.par ^= 1;
+		if (!edr_any(off)) break;
+		live = false;
+		if (has_prev) {
+			pend = S.hold[wave];
+			if (lane == 0) {
+				edr_put(&S.hold[wave][0], w1);
+				edr_put(&S.hold[wave][1], w2);
+			}
+		}
+		const bool changed = lane == from && c.n > 0 && (w1 != u1 || (M1 && w2 != u2));
+		if (lane == from) {
+			u1 = w1;
+			u2 = w2;
+		}
+		go = busy && edr_any(changed);
+	}
+
+	// The next row's samples, then this row's codes, then the loads for the
+	// row after: loads and stores share one counter, so waiting for loads
+	// issued before a store would wait for the store too.
+#pragma unroll
+	for (int i = 0; i < SEG; i++) r.X[i] = nx[i];
+	// The codes lie by x over the row's samples, which every wave has had
+	// since before the last barrier.
+	if (c.n > 0) {
+		uint8_t *row = (uint8_t *)(c.samp + (size_t)j * c.W);
+		unsigned int pack[SEG / 4] = {};
+#pragma unroll
+		for (int i = 0; i < SEG; i++) {
+			const int k = r.b[i] + (r.S[i] >= r.D[i] ? 1 : 0);
+			const unsigned int v = c.code_is_level ? (unsigned int)k : S.code[k];
+			if (c.out_depth == 8) pack[i / 4] |= v << (8 * (i % 4));
+			else if (i < c.n) ((__attribute__((address_space(1))) unsigned short *)row)[c.x0 + i] = (unsigned short)v;
+		}
+		// SEG bytes per lane stay inside the row's 8 * W.
+		if (c.out_depth == 8) __builtin_memcpy((g_u8 *)row + (size_t)SEG * threadIdx.x, pack, SEG);
+	}
+	edr_load<SEG>(c, j + 2, nx);
+}
+
+// The codes of plans diffused by errdiff_rows_kernel into their outputs:
+// items[blockIdx.x] = (plan, first row), EDR_ILV_ROWS rows each.
+#define EDR_ILV_ROWS 8
+__global__ void __launch_bounds__(256) edr_interleave_kernel(const DevPlan *__restrict__ plans,
+	const int2 *__restrict__ items)
+{
+	const int2 it = items[blockIdx.x];
+	const DevPlan &P = plans[it.x];
+	const int q = (P.out_w + 3) >> 2, rows = min(EDR_ILV_ROWS, P.out_h - it.y);
+	for (int t = threadIdx.x; t < q * rows; t += 256) edr_interleave4(P, it.y + t / q, (t % q) * 4);
+}
+
+// One workgroup per plane: planes[b] = (plan, output channel), rows of at
+// most 64 * NW * SEG pixels.
+template <bool M1, int SEG, int NW>
+__global__ void __launch_bounds__(64 * NW) errdiff_rows_kernel(const DevPlan *__restrict__ plans,
+	const int2 *__restrict__ planes)
+{
+	static_assert(SEG == 4 || SEG == 8, "a lane's 8-bit codes are whole words");
+	__shared__ EdrLds<NW> S;
+	constexpr int NT = 64 * NW;
+	const int tid = threadIdx.x;
+	const int2 pl = planes[blockIdx.x];
+	const DevPlan &P = plans[pl.x];
+	const DevOChan &q = P.oc[pl.y];
+	const int Pq = q.P;
+	g_cf64 *T = (g_cf64 *)q.T, *U = (g_cf64 *)q.U, *M = (g_cf64 *)q.M, *lin = (g_cf64 *)q.lin;
+
+	EdrCtx c;
+	c.m = c_ed_matrix[(q.subtype >= 0 && q.subtype <= 7) ? q.subtype : 0];
+	c.m0 = c.m[0];
+	c.m1 = c.m[1];
+	c.W = P.out_w;
+	c.H = P.out_h;
+	c.samp = P.ed_samples + (size_t)q.ed_index * c.H * c.W;
+	c.out_depth = P.out_depth;
+	c.code_is_level = q.code_is_level;
+	c.x0 = tid * SEG;
+	c.n = max(0, min(SEG, c.W - c.x0));
+	c.par = 0;
+
+	if (tid == 0) S.eps = 0;
+	if (tid < 2) S.hold[NW][tid] = 0.0;
+	for (int t = tid; t < (int)(sizeof(S.edge) / sizeof(double)); t += NT) (&S.edge[0][0].first[0])[t] = 0.0;
+	__syncthreads();
+	double eps = 0.0;
+	for (int k = tid; k <= Pq; k += NT) {
+		// The top level's exact samples end at 1.0 (U[P] is infinite).
+		S.lo[k] = k ? T[k - 1] : 0.0;
+		S.hi[k] = U[k];
+		S.lin[k] = lin[k];
+		eps = fmax(eps, fmax(fabs(S.lo[k] - lin[k]), fabs((k < Pq ? U[k] : 1.0) - lin[k])));
+		S.code[k] = (unsigned short)(0.5 + ((g_cf64 *)q.code)[k]);
+	}
+	atomicMax(&S.eps, (unsigned long long)__double_as_longlong(eps));
+	for (int k = tid; k < Pq + 3; k += NT) {
+		double d = k == 0 ? -1.0 : 4.0;
+		if (k > 0 && k <= Pq) d = fmin(T[k - 1], fmax(k > 1 ? T[k - 2] : 0.0, fmax(U[k - 1], M[k - 1])));
+		S.D[k] = d;
+	}
+	// The level below the bin's middle: its upper boundary is the nearest.
+	for (int k = tid; k < ED_NB; k += NT)
+		S.Q[k] = (unsigned short)(level_in(q.lin, 1, Pq, (k + 0.5) / (double)ED_NB) - 1);
+	__syncthreads();
+	c.eps_hi = (unsigned int)(S.eps >> 32) + 1u;
+
+	EdrRow<M1, SEG> r;
+#pragma unroll
+	for (int i = 0; i < SEG; i++) {
+		r.S[i] = r.E[i] = 0.0;
+		if (M1) r.R1[i] = 0.0;
+	}
+	double nx[SEG];
+	edr_load<SEG>(c, 0, r.X);
+	edr_load<SEG>(c, 1, nx);
+	for (int j = 0; j < c.H; j += 2) {
+		edr_row<false>(c, r, nx, S, j);
+		if (j + 1 < c.H) edr_row<true>(c, r, nx, S, j + 1);
+	}
+	__syncthreads();
+	ed_complete(P, tid, NT);
 }
 
 // ---- device memory and stream -------------------------------------------
@@ -3311,6 +3904,8 @@ int ed_warm(const iwamd_ochan &o, int P)
 	return m1 ? 96 : 64;
 }
 
+int ed_rows_shift(const Staged &S, const iwamd_plan &p);
+
 void fill_dev_plan(const Staged &S, const iwamd_plan &p, char *base, DevPlan &D)
 {
 	memset(&D, 0, sizeof(D));
@@ -3430,6 +4025,7 @@ void fill_dev_plan(const Staged &S, const iwamd_plan &p, char *base, DevPlan &D)
 	D.ed_err = (double *)(base + S.o_ede);
 	D.n_ed = S.n_ed;
 	D.ed_seg = S.ed_seg;
+	D.ed_shift = ed_rows_shift(S, p);
 	D.apply_bkgd = p.apply_bkgd;
 	D.late = p.bkgd_strategy_late;
 	D.checker = p.bkgd_checkerboard;
@@ -3466,29 +4062,56 @@ int lds_class(size_t bytes)
 	return q;
 }
 
-typedef void (*EdKernel)(const DevPlan *, const int2 *);
-constexpr int kEdVariants = 12;
-const EdKernel kEdKernels[kEdVariants] = {
-	errdiff_kernel<0, false, false>, errdiff_kernel<0, false, true>,
-	errdiff_kernel<0, true, false>, errdiff_kernel<0, true, true>,
-	errdiff_kernel<1, false, false>, errdiff_kernel<1, false, true>,
-	errdiff_kernel<1, true, false>, errdiff_kernel<1, true, true>,
-	errdiff_kernel<2, false, false>, errdiff_kernel<2, false, true>,
-	errdiff_kernel<2, true, false>, errdiff_kernel<2, true, true>};
+struct EdVariant {
+	void (*kernel)(const DevPlan *, const int2 *);
+	int threads;
+};
+// Row shapes of errdiff_rows_kernel: (pixels per segment, waves), by width.
+#define EDR_SHAPES(M1) \
+	{errdiff_rows_kernel<M1, 4, 1>, 64}, {errdiff_rows_kernel<M1, 4, 2>, 128}, {errdiff_rows_kernel<M1, 4, 4>, 256}, \
+	{errdiff_rows_kernel<M1, 8, 4>, 256}, {errdiff_rows_kernel<M1, 8, 8>, 512}
+constexpr int kEdrShapes = 5;
+constexpr int kEdrWidth[kEdrShapes] = {256, 512, 1024, 2048, EDR_MAX_W};
+constexpr int kEdRowsVariant = 8;  // the first variant of errdiff_rows_kernel
+constexpr int kEdVariants = kEdRowsVariant + 2 * kEdrShapes;
+const EdVariant kEdKernels[kEdVariants] = {
+	{errdiff_kernel<0, false, false>, ED_THREADS}, {errdiff_kernel<0, false, true>, ED_THREADS},
+	{errdiff_kernel<0, true, false>, ED_THREADS}, {errdiff_kernel<0, true, true>, ED_THREADS},
+	{errdiff_kernel<1, false, false>, ED_THREADS}, {errdiff_kernel<1, true, false>, ED_THREADS},
+	{errdiff_kernel<2, false, false>, ED_THREADS}, {errdiff_kernel<2, true, false>, ED_THREADS},
+	EDR_SHAPES(false), EDR_SHAPES(true)};
+#undef EDR_SHAPES
 
-// Kernel variant of one error-diffusion plane: decision records in registers
-// for at most ED_SMALL_P + 1 levels, in LDS for up to 257, the x+2 carry only
-// where its weight is nonzero (not Floyd-Steinberg or Sierra 4-2-1), working
-// rows in LDS up to ED_ROWS_LDS wide.
-int ed_variant(const Staged &S, const iwamd_plan &p, int o)
+// Kernel variant of one error-diffusion plane.  rows: the job runs
+// errdiff_rows_kernel (ed_rows_shift).  Else errdiff_kernel: decision records
+// in registers for at most ED_SMALL_P + 1 levels, in LDS for up to 257, its
+// working rows in LDS up to ED_ROWS_LDS wide for more levels.  The x+2 carry
+// only where its weight is nonzero (not Floyd-Steinberg or Sierra 4-2-1).
+int ed_variant(const Staged &S, const iwamd_plan &p, int o, bool rows)
 {
 	const int subtype = p.och[o].dithersubtype;
 	const int sub = (subtype >= 0 && subtype <= 7) ? subtype : 0;
-	const bool m1 = sub != 0 && sub != 6;
-	const bool rows = p.out_width <= ED_ROWS_LDS && ed_cap(p.out_width, S.ed_seg) <= ED_CAP_LDS;
+	const int m1 = sub != 0 && sub != 6;
+	if (rows) {
+		int shape = 0;
+		while (p.out_width > kEdrWidth[shape]) shape++;
+		return kEdRowsVariant + kEdrShapes * m1 + shape;
+	}
 	const int P = S.qt[o].P;
 	const int tabm = P <= ED_SMALL_P ? 2 : (P <= ED_LDS_TABLE ? 1 : 0);
-	return 4 * tabm + (m1 ? 2 : 0) + (rows ? 1 : 0);
+	if (tabm) return 2 + 2 * tabm + m1;
+	return 2 * m1 + (p.out_width <= ED_ROWS_LDS && ed_cap(p.out_width, S.ed_seg) <= ED_CAP_LDS ? 1 : 0);
+}
+
+// The sample layout of a job whose planes run errdiff_rows_kernel (log2 of
+// its pixels per segment), or 0: rows of up to EDR_MAX_W pixels and at most
+// 257 levels in every error-diffused channel.
+int ed_rows_shift(const Staged &S, const iwamd_plan &p)
+{
+	if (!S.n_ed || p.out_width > EDR_MAX_W) return 0;
+	for (int e = 0; e < S.n_ed; e++)
+		if (S.qt[S.ed_list[e]].P > ED_LDS_TABLE) return 0;
+	return p.out_width <= 1024 ? 2 : 3;
 }
 
 struct WorkSet {
@@ -3496,6 +4119,7 @@ struct WorkSet {
 	std::vector<int2> bands[3][kLdsClasses];  // (plan, first row), by band height kBandR and LDS class
 	size_t band_lds[3][kLdsClasses] = {};      // largest LDS of a band in each list
 	std::vector<int2> planes[kEdVariants];  // (plan, output channel), by ed_variant
+	std::vector<int2> ilv;            // (plan, first row) of the outputs edr_interleave_kernel forms
 	std::vector<int> twopass;         // plans resampled by vpass + hpass
 	// Chosen-precision tiles, and work items over them: runs of one band's
 	// tiles (first tile, count), by kernel variant.
@@ -3504,7 +4128,7 @@ struct WorkSet {
 	std::vector<int2> fast[FAST_NVAR];
 	int fast_chunks[FAST_NVAR][XCD_COUNT + 1] = {};  // each chosen-form list's chunks, one per XCD
 	size_t o_plans = 0, o_bands[3][kLdsClasses] = {}, o_planes[kEdVariants] = {0}, o_counters = 0, o_fast[FAST_NVAR] = {},
-		o_chunks = 0, o_done = 0;
+		o_chunks = 0, o_done = 0, o_ilv = 0;
 	size_t bytes = 0;
 	const FastItem *d_fast_tiles = nullptr;
 	const int2 *d_fast[FAST_NVAR] = {};
@@ -3513,6 +4137,7 @@ struct WorkSet {
 	const DevPlan *d_plans = nullptr;
 	const int2 *d_bands[3][kLdsClasses] = {};
 	const int2 *d_planes[kEdVariants] = {nullptr};
+	const int2 *d_ilv = nullptr;
 	const int *d_chunks = nullptr;
 	int *d_counters = nullptr;
 };
@@ -3565,10 +4190,13 @@ int ws_add(WorkSet &W, const Staged &S, const iwamd_plan &p)
 	} else {
 		W.twopass.push_back(jx);
 	}
+	const bool rows = ed_rows_shift(S, p) != 0;
 	for (int e = 0; e < S.n_ed; e++) {
 		const int o = S.ed_list[e];
-		W.planes[ed_variant(S, p, o)].push_back(make_int2(jx, o));
+		W.planes[ed_variant(S, p, o, rows)].push_back(make_int2(jx, o));
 	}
+	if (rows)
+		for (int j0 = 0; j0 < p.out_height; j0 += EDR_ILV_ROWS) W.ilv.push_back(make_int2(jx, j0));
 	return jx;
 }
 
@@ -3608,6 +4236,7 @@ void ws_layout(WorkSet &W)
 	for (int r = 0; r < 3; r++)
 		for (int q = 0; q < kLdsClasses; q++) W.o_bands[r][q] = L.add<int2>(W.bands[r][q].size());
 	for (int v = 0; v < kEdVariants; v++) W.o_planes[v] = L.add<int2>(W.planes[v].size());
+	W.o_ilv = L.add<int2>(W.ilv.size());
 	W.o_counters = L.add<int>(kCounters);
 	W.o_fast_tiles = L.add<FastItem>(W.fast_tiles.size());
 	for (int v = 0; v < FAST_NVAR; v++) W.o_fast[v] = L.add<int2>(W.fast[v].size());
@@ -3636,6 +4265,8 @@ bool ws_upload(WorkSet &W, char *base, hipStream_t st)
 		W.d_planes[v] = (const int2 *)(base + W.o_planes[v]);
 		up(W.o_planes[v], W.planes[v].data(), W.planes[v].size() * sizeof(int2));
 	}
+	W.d_ilv = (const int2 *)(base + W.o_ilv);
+	up(W.o_ilv, W.ilv.data(), W.ilv.size() * sizeof(int2));
 	W.d_counters = (int *)(base + W.o_counters);
 	W.d_fast_tiles = (const FastItem *)(base + W.o_fast_tiles);
 	up(W.o_fast_tiles, W.fast_tiles.data(), W.fast_tiles.size() * sizeof(FastItem));
@@ -3724,12 +4355,16 @@ void ws_enqueue_resample(const WorkSet &W, hipStream_t st, bool persistent)
 	}
 }
 
-void ws_enqueue_errdiff(const WorkSet &W, hipStream_t st)
+// interleave: form the outputs of the planes errdiff_rows_kernel has diffused
+// (in the request loop each request's last plane does).
+void ws_enqueue_errdiff(const WorkSet &W, hipStream_t st, bool interleave = true)
 {
 	for (int v = 0; v < kEdVariants; v++) {
 		const int n = (int)W.planes[v].size();
-		if (n) hipLaunchKernelGGL(kEdKernels[v], dim3(n), dim3(ED_THREADS), 0, st, W.d_plans, W.d_planes[v]);
+		if (n) hipLaunchKernelGGL(kEdKernels[v].kernel, dim3(n), dim3(kEdKernels[v].threads), 0, st, W.d_plans, W.d_planes[v]);
 	}
+	if (interleave && !W.ilv.empty())
+		hipLaunchKernelGGL(edr_interleave_kernel, dim3((unsigned int)W.ilv.size()), dim3(256), 0, st, W.d_plans, W.d_ilv);
 }
 
 // Useful floating-point operations of a plan's resampling: a multiply and an
@@ -4847,7 +5482,7 @@ bool ServerExec::launch(Loop::Flight &F, int slot)
 	}
 	if (ok) {
 		ws_enqueue_resample(D.W, st, true);
-		ws_enqueue_errdiff(D.W, st);
+		ws_enqueue_errdiff(D.W, st, false);
 		// The optimiser's scans of the outputs that complete with the
 		// flight (one that completes on its own has been copied already).
 		char *sreg = (char *)D.block + D.scan_dev;
