@@ -230,9 +230,36 @@ struct iwx_opt_scan {
 	unsigned long long pal[IWX_SCAN_PAL_SLOTS];
 };
 
-// iw_finish.cpp
-int iwx_finish(iw_context *ctx, const iwx_opt_scan *scan = nullptr);
-void iwx_optimize_image(iw_context *ctx, const iwx_opt_scan *scan = nullptr);
+// How the optimised image is formed from the finished one, pixel by pixel,
+// where the pixels are still on the device: 16-bit samples reduced to their
+// high byte, then channels picked, then either palette indices or a colour
+// key in place of fully transparent pixels (src/imagew-opt.c:243-360,
+// :418-683, :906-1004).
+struct iwx_out_conv {
+	int any = 0;                    // 0: the image stays as it is
+	int to8 = 0;
+	int nch = 0, src[4] = {0, 1, 2, 3};  // channels, each from this one of the image
+	int pal_n = 0;                  // entries of a palette image, else 0
+	unsigned int pal[256] = {};     // r | g<<8 | b<<16 | a<<24, the image's pixel as the palette sees it
+	int pal_key = -1;               // index of fully transparent pixels, where a grey palette has a colour key
+	int key = 0;                    // fully transparent pixels become key_px
+	int key_alpha = 0;              // the image's alpha channel
+	unsigned char key_px[8] = {};
+};
+
+// iw_finish.cpp.  conv: the image is not in ctx->img2.pixels; conv tells how
+// to form the optimised one (needs a valid scan).
+int iwx_finish(iw_context *ctx, const iwx_opt_scan *scan = nullptr, iwx_out_conv *conv = nullptr);
+void iwx_optimize_image(iw_context *ctx, const iwx_opt_scan *scan = nullptr, iwx_out_conv *conv = nullptr);
+
+// iw_prepare.cpp.  A prepared context whose image is on the device:
+// iwx_finish_decide() decides its output from the scan, then
+// iwx_finish_pixels() gives the memory that its pixels (conv's) are to be
+// copied to.  iwx_finish_begin() gives the memory of the unchanged image, for
+// iwx_finish() to follow.
+int iwx_finish_decide(struct iw_context *ctx, const struct iwx_opt_scan *scan, iwx_out_conv *conv);
+iw_byte *iwx_finish_pixels(struct iw_context *ctx, const iwx_out_conv &conv, size_t *bytes);
+iw_byte *iwx_finish_begin(struct iw_context *ctx);
 
 // iw_gpu.hip
 int iwx_gpu_process(iw_context *ctx);

@@ -182,16 +182,21 @@ void attach_pixels(iw_context *ctx, iwx_opt_ctx &o, iw_byte *np, size_t nbpr)
 }
 
 // Keep the high byte of every sample (src/imagew-opt.c:243-283).
-void reduce_16_to_8(iw_context *ctx, iwx_opt_ctx &o, int spp)
+void reduce_16_to_8(iw_context *ctx, iwx_opt_ctx &o, int spp, iwx_out_conv *conv)
 {
 	if (!ctx->opt_16_to_8) return;
 	size_t nbpr = iw_calc_bytesperrow(o.width, 8 * spp);
-	iw_byte *np = (iw_byte *)iw_malloc_large(ctx, nbpr, o.height);
-	if (!np) return;
-	for (int j = 0; j < o.height; j++)
-		for (int i = 0; i < spp * o.width; i++)
-			np[(size_t)j * nbpr + i] = o.pixelsptr[(size_t)j * o.bpr + (size_t)i * 2];
-	attach_pixels(ctx, o, np, nbpr);
+	if (conv) {
+		conv->any = conv->to8 = 1;
+		o.bpr = nbpr;
+	} else {
+		iw_byte *np = (iw_byte *)iw_malloc_large(ctx, nbpr, o.height);
+		if (!np) return;
+		for (int j = 0; j < o.height; j++)
+			for (int i = 0; i < spp * o.width; i++)
+				np[(size_t)j * nbpr + i] = o.pixelsptr[(size_t)j * o.bpr + (size_t)i * 2];
+		attach_pixels(ctx, o, np, nbpr);
+	}
 	o.bit_depth = 8;
 	if (o.has_bkgdlabel)
 		for (int k = 0; k < 4; k++) o.bkgdlabel[k] >>= 8;
@@ -199,14 +204,24 @@ void reduce_16_to_8(iw_context *ctx, iwx_opt_ctx &o, int spp)
 
 // New image from up to three channels of the current one
 // (src/imagew-opt.c:286-360).
-void copy_channels(iw_context *ctx, iwx_opt_ctx &o, int new_type, int c0, int c1, int c2)
+void copy_channels(iw_context *ctx, iwx_opt_ctx &o, int new_type, int c0, int c1, int c2, iwx_out_conv *conv)
 {
 	const int oldnc = iw_imgtype_num_channels(o.imgtype), newnc = iw_imgtype_num_channels(new_type);
 	const int bps = o.bit_depth / 8;
 	size_t nbpr = iw_calc_bytesperrow(o.width, o.bit_depth * newnc);
+	const int src[3] = {c0, c1, c2};
+	if (conv) {
+		int was[4];
+		memcpy(was, conv->src, sizeof(was));
+		for (int k = 0; k < newnc; k++) conv->src[k] = was[src[k]];
+		conv->nch = newnc;
+		conv->any = 1;
+		o.bpr = nbpr;
+		o.imgtype = new_type;
+		return;
+	}
 	iw_byte *np = (iw_byte *)iw_malloc_large(ctx, nbpr, o.height);
 	if (!np) return;
-	const int src[3] = {c0, c1, c2};
 	for (int j = 0; j < o.height; j++)
 		for (int i = 0; i < o.width; i++)
 			for (int k = 0; k < newnc; k++)
@@ -237,7 +252,7 @@ int find_unused(const iw_byte *flags, int count, iw_byte *out)
 // RGBA/GA with only fully opaque or fully transparent pixels becomes RGB/G
 // plus a colour key chosen among values the image does not use
 // (src/imagew-opt.c:418-683).
-void try_binary_trns(iw_context *ctx, iwx_opt_ctx &o, const iwx_opt_scan *scan)
+void try_binary_trns(iw_context *ctx, iwx_opt_ctx &o, const iwx_opt_scan *scan, iwx_out_conv *conv)
 {
 	if (!(ctx->output_profile & IW_PROFILE_BINARYTRNS)) return;
 	if (!ctx->opt_binary_trns) return;
@@ -252,9 +267,12 @@ void try_binary_trns(iw_context *ctx, iwx_opt_ctx &o, const iwx_opt_scan *scan)
 		const int key = rgb ? (b16 ? IWX_KEY_RGB16 : IWX_KEY_RGB8) : (b16 ? IWX_KEY_GRAY16 : IWX_KEY_GRAY8);
 		for (int v = 0; v < 256; v++) used[v] = (scan->used[key][v >> 5] >> (v & 31)) & 1u;
 	}
-	iw_byte *mask = (iw_byte *)iw_malloc_large(ctx, o.width, o.height);
-	if (!mask) return;
-	for (int j = 0; j < o.height; j++) {
+	iw_byte *mask = nullptr;
+	if (!conv) {
+		mask = (iw_byte *)iw_malloc_large(ctx, o.width, o.height);
+		if (!mask) return;
+	}
+	for (int j = 0; j < o.height && !conv; j++) {
 		for (int i = 0; i < o.width; i++) {
 			const unsigned int a = sample_at(o, nc, i, j, nc - 1);
 			mask[(size_t)j * o.width + i] = (a != 0);
@@ -282,10 +300,16 @@ void try_binary_trns(iw_context *ctx, iwx_opt_ctx &o, const iwx_opt_scan *scan)
 	}
 	iw_byte key = 0;
 	if (find_unused(used, 256, &key)) {
-		copy_channels(ctx, o, rgb ? IW_IMGTYPE_RGB : IW_IMGTYPE_GRAY, 0, rgb ? 1 : 0, rgb ? 2 : 0);
-		if (o.tmp_pixels) {
+		if (conv) conv->key_alpha = conv->src[nc - 1];
+		copy_channels(ctx, o, rgb ? IW_IMGTYPE_RGB : IW_IMGTYPE_GRAY, 0, rgb ? 1 : 0, rgb ? 2 : 0, conv);
+		if (o.tmp_pixels || conv) {
 			const int nnc = rgb ? 3 : 1;
-			for (int j = 0; j < o.height; j++) {
+			if (conv) {
+				conv->key = 1;
+				memset(conv->key_px, 192, sizeof(conv->key_px));
+				conv->key_px[b16 ? 1 : 0] = key;
+			}
+			for (int j = 0; j < o.height && !conv; j++) {
 				for (int i = 0; i < o.width; i++) {
 					if (mask[(size_t)j * o.width + i]) continue;
 					iw_byte *q = o.tmp_pixels + (size_t)j * o.bpr + (size_t)i * nnc * (b16 ? 2 : 1);
@@ -306,7 +330,7 @@ void try_binary_trns(iw_context *ctx, iwx_opt_ctx &o, const iwx_opt_scan *scan)
 			o.colorkey[IW_CHANNELTYPE_BLUE] = kgb;
 		}
 	}
-	iw_free(ctx, mask);
+	if (mask) iw_free(ctx, mask);
 }
 
 // ---- palettes (src/imagew-opt.c:678-1094) --------------------------------
@@ -494,9 +518,19 @@ struct PaletteIndex {
 	}
 };
 
-void convert_to_palette(iw_context *ctx, iwx_opt_ctx &o)
+void convert_to_palette(iw_context *ctx, iwx_opt_ctx &o, iwx_out_conv *conv)
 {
 	size_t nbpr = o.width;
+	if (conv) {
+		conv->any = 1;
+		conv->pal_n = o.palette->num_entries;
+		for (int i = 0; i < conv->pal_n; i++) conv->pal[i] = PaletteIndex::pack(o.palette->entry[i]);
+		if (o.has_colorkey_trns) conv->pal_key = (iw_byte)o.colorkey[IW_CHANNELTYPE_RED];
+		o.bpr = nbpr;
+		o.bit_depth = 8;
+		o.imgtype = IW_IMGTYPE_PALETTE;
+		return;
+	}
 	iw_byte *np = (iw_byte *)iw_malloc_large(ctx, nbpr, o.height);
 	if (!np) return;
 	const PaletteIndex index(o.palette);
@@ -519,7 +553,7 @@ void convert_to_palette(iw_context *ctx, iwx_opt_ctx &o)
 
 // Preference gray1, pal1, gray2, pal2, gray4, pal4, (gray8: leave), pal8
 // (src/imagew-opt.c:1010-1094).
-void try_palette(iw_context *ctx, iwx_opt_ctx &o, const iwx_opt_scan *scan)
+void try_palette(iw_context *ctx, iwx_opt_ctx &o, const iwx_opt_scan *scan, iwx_out_conv *conv)
 {
 	const unsigned int p = ctx->output_profile;
 	if (!(p & (IW_PROFILE_PAL1 | IW_PROFILE_PAL2 | IW_PROFILE_PAL4 | IW_PROFILE_PAL8 |
@@ -558,7 +592,7 @@ void try_palette(iw_context *ctx, iwx_opt_ctx &o, const iwx_opt_scan *scan)
 		if (chosen) {
 			if (!o.palette_is_grayscale)
 				qsort(o.palette->entry, o.palette->num_entries, sizeof(struct iw_rgba8color), palette_order);
-			convert_to_palette(ctx, o);
+			convert_to_palette(ctx, o, conv);
 		}
 	}
 	if (o.imgtype != IW_IMGTYPE_PALETTE) {
@@ -584,8 +618,9 @@ void make_transparent_pixels_black(iw_image &im)
 
 }  // namespace
 
-void iwx_optimize_image(iw_context *ctx, const iwx_opt_scan *scan)
+void iwx_optimize_image(iw_context *ctx, const iwx_opt_scan *scan, iwx_out_conv *conv)
 {
+	if (conv) conv->nch = ctx->img2_numchannels;
 	if (scan && !(scan->valid & IWX_SCAN_HAVE_FLAGS)) scan = nullptr;
 	iwx_opt_ctx &o = ctx->optctx;
 	o.width = ctx->img2.width;
@@ -618,25 +653,25 @@ void iwx_optimize_image(iw_context *ctx, const iwx_opt_scan *scan)
 			if (scan->flags & IWX_SCAN_16BIT) o.has_16bit_precision = 1;
 		}
 		const int t0 = o.imgtype;
-		if (o.bit_depth == 16 && !o.has_16bit_precision) reduce_16_to_8(ctx, o, iw_imgtype_num_channels(t0));
+		if (o.bit_depth == 16 && !o.has_16bit_precision) reduce_16_to_8(ctx, o, iw_imgtype_num_channels(t0), conv);
 		if (!o.has_transparency && ctx->opt_strip_alpha) {
-			if (o.imgtype == IW_IMGTYPE_RGBA) copy_channels(ctx, o, IW_IMGTYPE_RGB, 0, 1, 2);
-			else if (o.imgtype == IW_IMGTYPE_GRAYA) copy_channels(ctx, o, IW_IMGTYPE_GRAY, 0, 0, 0);
+			if (o.imgtype == IW_IMGTYPE_RGBA) copy_channels(ctx, o, IW_IMGTYPE_RGB, 0, 1, 2, conv);
+			else if (o.imgtype == IW_IMGTYPE_GRAYA) copy_channels(ctx, o, IW_IMGTYPE_GRAY, 0, 0, 0, conv);
 		}
 		if (!o.has_color && (ctx->output_profile & IW_PROFILE_GRAYSCALE) && ctx->opt_grayscale) {
-			if (o.imgtype == IW_IMGTYPE_RGB) copy_channels(ctx, o, IW_IMGTYPE_GRAY, 0, 0, 0);
-			else if (o.imgtype == IW_IMGTYPE_RGBA) copy_channels(ctx, o, IW_IMGTYPE_GRAYA, 0, 3, 0);
+			if (o.imgtype == IW_IMGTYPE_RGB) copy_channels(ctx, o, IW_IMGTYPE_GRAY, 0, 0, 0, conv);
+			else if (o.imgtype == IW_IMGTYPE_RGBA) copy_channels(ctx, o, IW_IMGTYPE_GRAYA, 0, 3, 0, conv);
 		}
 	}
 
-	try_palette(ctx, o, scan);
+	try_palette(ctx, o, scan, conv);
 
 	if ((o.imgtype == IW_IMGTYPE_RGBA || o.imgtype == IW_IMGTYPE_GRAYA) && !o.has_partial_transparency &&
 		(o.bit_depth == 8 || o.bit_depth == 16))
-		try_binary_trns(ctx, o, scan);
+		try_binary_trns(ctx, o, scan, conv);
 }
 
-int iwx_finish(iw_context *ctx, const iwx_opt_scan *scan)
+int iwx_finish(iw_context *ctx, const iwx_opt_scan *scan, iwx_out_conv *conv)
 {
 	process_bkgd_label(ctx);
 	// The device scans only images that are not negated afterwards.
@@ -644,6 +679,6 @@ int iwx_finish(iw_context *ctx, const iwx_opt_scan *scan)
 		negate_target_image(ctx);
 		scan = nullptr;
 	}
-	iwx_optimize_image(ctx, scan);
+	iwx_optimize_image(ctx, scan, conv);
 	return 1;
 }

@@ -57,6 +57,7 @@ typedef __attribute__((address_space(1))) unsigned char g_u8;
 typedef const __attribute__((address_space(1))) double g_cf64;
 typedef const __attribute__((address_space(1))) unsigned short g_cu16;
 typedef const __attribute__((address_space(1))) int g_cint;
+typedef __attribute__((address_space(1), aligned(1))) unsigned int g_u32u;  // at any byte
 
 // ---- device-side plan ----------------------------------------------------
 
@@ -3315,6 +3316,153 @@ __global__ void opt_clear_kernel(uint4 *p, size_t n)
 		p[i] = make_uint4(0u, 0u, 0u, 0u);
 }
 
+// ---- the optimised image (iwx_out_conv) ---------------------------------------
+// The image that the optimiser decided on, formed from the finished one
+// before it is copied back: each pixel is read once and its new bytes
+// written.  HBM-bound by size, though at these sizes mostly a launch: 3072^2
+// grey to palette indices 12 us, where the host took 25-40 ms.  A palette's
+// colours are looked up in an LDS hash set whose slots hold the first entry
+// with that colour.
+
+#define CONV_PPT 4       // consecutive pixels per thread
+#define CONV_SLOTS 1024
+
+struct ConvArgs {
+	const unsigned char *src;
+	unsigned char *dst;
+	unsigned long long npx;
+	iwx_out_conv c;
+};
+
+template <int NC, int B16>
+__device__ void conv_pixels(const ConvArgs &A, const unsigned long long *tab, const int *idx)
+{
+	constexpr int PB = NC * (B16 ? 2 : 1);
+	const iwx_out_conv &c = A.c;
+	const bool wide = B16 && !c.to8;
+	const int ob = c.pal_n ? 1 : c.nch * (wide ? 2 : 1);
+	const unsigned long long p0 = ((unsigned long long)blockIdx.x * blockDim.x + threadIdx.x) * CONV_PPT;
+	if (p0 >= A.npx) return;
+	const int n = (int)(A.npx - p0 < CONV_PPT ? A.npx - p0 : CONV_PPT);
+	unsigned long long v[CONV_PPT];
+#pragma unroll
+	for (int t = 0; t < CONV_PPT; t++) {
+		unsigned int s[4];
+		const OptRaw<NC, B16> raw = opt_raw<NC, B16>((const g_u8 *)A.src + (p0 + (t < n ? t : 0)) * PB);
+		opt_decode<NC, B16>(raw, s);
+		auto pick = [&](int k) {
+			unsigned int x = s[0];
+#pragma unroll
+			for (int i = 1; i < NC; i++)
+				if (k == i) x = s[i];
+			return x;
+		};
+		unsigned int d[4] = {0, 0, 0, 0};
+#pragma unroll
+		for (int k = 0; k < 4; k++)
+			if (k < c.nch) {
+				d[k] = pick(c.src[k]);
+				if (B16 && c.to8) d[k] >>= 8;
+			}
+		if (c.pal_n) {
+			// The pixel as the palette sees it.
+			const unsigned int a = c.nch == 4 ? d[3] : (c.nch == 2 ? d[1] : 255u);
+			unsigned int key = c.nch >= 3 ? d[0] | d[1] << 8 | d[2] << 16 : d[0] * 0x010101u;
+			key = a ? key | a << 24 : 0u;
+			int e = 0;
+			if (!a && c.pal_key >= 0) {
+				e = c.pal_key;
+			} else {
+				const unsigned long long want = (1ull << 32) | key;
+				unsigned int h = opt_hash(key, CONV_SLOTS);
+				while (tab[h] && tab[h] != want) h = (h + 1) & (CONV_SLOTS - 1);
+				if (tab[h]) e = idx[h];
+			}
+			v[t] = (unsigned int)e;
+			continue;
+		}
+		unsigned long long w = 0;
+#pragma unroll
+		for (int k = 0; k < 4; k++) {
+			if (k >= c.nch) continue;
+			// 16-bit samples are stored big-endian.
+			if (wide) w |= (unsigned long long)((d[k] >> 8 & 0xffu) | (d[k] & 0xffu) << 8) << (16 * k);
+			else w |= (unsigned long long)(d[k] & 0xffu) << (8 * k);
+		}
+		if (c.key && pick(c.key_alpha) == 0) {
+			w = 0;
+#pragma unroll
+			for (int k = 0; k < 8; k++) w |= (unsigned long long)c.key_px[k] << (8 * k);
+		}
+		v[t] = w;
+	}
+	g_u8 *q = (g_u8 *)A.dst + p0 * ob;
+	if (n == CONV_PPT && ob <= 4) {
+		// Whole words: four pixels of ob bytes are ob words.
+		unsigned int w[4];
+		if (ob == 1) {
+			w[0] = (unsigned int)(v[0] & 0xffu) | (unsigned int)(v[1] & 0xffu) << 8 | (unsigned int)(v[2] & 0xffu) << 16 |
+				(unsigned int)v[3] << 24;
+			*(g_u32u *)q = w[0];
+			return;
+		}
+		if (ob == 3) {
+			w[0] = (unsigned int)(v[0] & 0xffffffu) | (unsigned int)v[1] << 24;
+			w[1] = (unsigned int)(v[1] >> 8 & 0xffffu) | (unsigned int)v[2] << 16;
+			w[2] = (unsigned int)(v[2] >> 16 & 0xffu) | (unsigned int)v[3] << 8;
+			for (int k = 0; k < 3; k++) ((g_u32u *)q)[k] = w[k];
+			return;
+		}
+	}
+	for (int t = 0; t < n; t++) {
+		unsigned long long x = t == 0 ? v[0] : (t == 1 ? v[1] : (t == 2 ? v[2] : v[3]));
+		for (int b = 0; b < ob; b++) q[t * ob + b] = (uint8_t)(x >> (8 * b));
+	}
+}
+
+template <int NC, int B16>
+__global__ void __launch_bounds__(256) conv_kernel(ConvArgs A)
+{
+	__shared__ unsigned long long tab[CONV_SLOTS];
+	__shared__ int idx[CONV_SLOTS];
+	if (A.c.pal_n) {
+		for (int t = threadIdx.x; t < CONV_SLOTS; t += 256) {
+			tab[t] = 0;
+			idx[t] = 0x7fffffff;
+		}
+		__syncthreads();
+		for (int t = threadIdx.x; t < A.c.pal_n; t += 256) {
+			// At most 256 entries in 1024 slots: one is always free.
+			const unsigned long long want = (1ull << 32) | A.c.pal[t];
+			unsigned int h = opt_hash(A.c.pal[t], CONV_SLOTS);
+			for (;; h = (h + 1) & (CONV_SLOTS - 1)) {
+				const unsigned long long was = atomicCAS(&tab[h], 0ull, want);
+				if (was == 0 || was == want) break;
+			}
+			atomicMin(&idx[h], t);
+		}
+		__syncthreads();
+	}
+	conv_pixels<NC, B16>(A, tab, idx);
+}
+
+// Forms the optimised image of the finished one at src on st.
+bool conv_enqueue(const iwx_out_conv &conv, const iw_context *ctx, const void *src, void *dst, hipStream_t st)
+{
+	ConvArgs A;
+	A.src = (const unsigned char *)src;
+	A.dst = (unsigned char *)dst;
+	A.npx = (unsigned long long)ctx->img2.width * ctx->img2.height;
+	A.c = conv;
+	const unsigned int grid = (unsigned int)((A.npx + 256 * CONV_PPT - 1) / (256 * CONV_PPT));
+	const int nc = iw_imgtype_num_channels(ctx->img2.imgtype), b16 = ctx->img2.bit_depth == 16;
+	typedef void (*Kernel)(ConvArgs);
+	static const Kernel k[8] = {conv_kernel<1, 0>, conv_kernel<1, 1>, conv_kernel<2, 0>, conv_kernel<2, 1>,
+		conv_kernel<3, 0>, conv_kernel<3, 1>, conv_kernel<4, 0>, conv_kernel<4, 1>};
+	hipLaunchKernelGGL(k[2 * (nc - 1) + b16], dim3(grid), dim3(256), 0, st, A);
+	return hipGetLastError() == hipSuccess;
+}
+
 // Which of the optimiser's inputs the device forms for this prepared
 // context (IWX_SCAN_HAVE_*); 0: the host scans.  Negated output is scanned
 // by the host after the negation (src/imagew-main.c:1439-1440).
@@ -4711,37 +4859,79 @@ extern "C" double iwamd_job_flops(struct iwamd_job *J)
 	return J->flops;
 }
 
+// Outputs from this size on wait for their scan first, so that the optimised
+// image is formed on the device and copied straight to its place; smaller ones
+// come back with the scan, one wait in all, and the host forms them (a second
+// wait costs about 15 us, which the host forms some 10,000 pixels in).
+#define FINISH_ON_DEVICE ((size_t)128 << 10)
+
 extern "C" int iwamd_job_finish(struct iwamd_job *J)
 {
-	std::vector<uint8_t> host(J->out_bytes + 1, 0);
+	iw_context *ctx = J->ctx;
+	char *out = (char *)J->block + J->out_off;
 	// The optimiser's scans run on the output before it is copied back.
-	const unsigned int want = J->skip_pixels ? 0 : opt_scan_want(J->ctx);
+	const unsigned int want = J->skip_pixels ? 0 : opt_scan_want(ctx);
+	const bool large = J->out_bytes >= FINISH_ON_DEVICE && !J->skip_pixels;
 	const size_t sbytes = opt_scan_bytes(1);
-	void *sblk = want ? dev_alloc(sbytes) : nullptr;
+	size_t cbytes = 0;
+	void *sblk = want ? dev_alloc(sbytes) : nullptr, *cblk = nullptr;
 	std::vector<OptJob> scans;
 	std::unique_ptr<iwx_opt_scan> scan(want ? new iwx_opt_scan() : nullptr);
 	bool ok = !want || sblk;
 	if (ok && want) {
 		iwx_opt_scan *res = (iwx_opt_scan *)((char *)sblk + opt_scan_bytes(1) - sizeof(iwx_opt_scan));
-		scans.push_back(opt_job(J->ctx, (char *)J->block + J->out_off, res, want));
+		scans.push_back(opt_job(ctx, out, res, want));
 		ok = opt_scan_enqueue(scans, sblk, 1, J->stream) &&
 			hipMemcpyAsync(scan.get(), res, sizeof(iwx_opt_scan), hipMemcpyDeviceToHost, J->stream) == hipSuccess;
 	}
-	if (ok && !J->skip_pixels)
-		ok = hipMemcpyAsync(host.data(), (char *)J->block + J->out_off, J->out_bytes, hipMemcpyDeviceToHost,
-			J->stream) == hipSuccess;
-	ok = ok && iwamd_job_sync(J);
+	auto back = [&](void *dst, const void *src, size_t bytes) {
+		return hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, J->stream) == hipSuccess && iwamd_job_sync(J);
+	};
+	int done = 1;
+	if (ok && large && want) {
+		ok = iwamd_job_sync(J);
+		if (ok) {
+			scan->valid = want;
+			iwx_out_conv conv;
+			done = iwx_finish_decide(ctx, scan.get(), &conv);
+			size_t bytes = 0;
+			iw_byte *dst = done ? iwx_finish_pixels(ctx, conv, &bytes) : nullptr;
+			if (!dst) {
+				done = 0;
+			} else if (conv.any) {
+				cbytes = bytes;
+				cblk = dev_alloc(cbytes);
+				ok = cblk && conv_enqueue(conv, ctx, out, cblk, J->stream) && back(dst, cblk, bytes);
+			} else {
+				ok = back(dst, out, bytes);
+			}
+		}
+	} else if (ok && large) {
+		iw_byte *dst = iwx_finish_begin(ctx);
+		done = dst != nullptr;
+		if (dst) {
+			ok = back(dst, out, J->out_bytes);
+			if (ok) done = iwx_finish(ctx);
+		} else {
+			ok = iwamd_job_sync(J);
+		}
+	} else if (ok) {
+		std::vector<uint8_t> host(J->out_bytes + 1, 0);
+		ok = J->skip_pixels ? iwamd_job_sync(J) : back(host.data(), out, J->out_bytes);
+		if (scan) scan->valid = want;
+		if (ok) done = iwx_finish_image(ctx, host.data(), scan.get());
+	}
 	if (sblk) dev_release(sblk, sbytes);
+	if (cblk) dev_release(cblk, cbytes);
 	if (!ok) {
-		iw_set_error(J->ctx, "Device-to-host copy failed");
+		iw_set_error(ctx, "Device-to-host copy failed");
 		return 0;
 	}
-	if (scan) scan->valid = want;
 	double ms[3];
 	int k = iwamd_job_kernel_ms(J, ms, 3);
-	J->ctx->num_last_timings = k;
-	for (int i = 0; i < k; i++) J->ctx->last_timings_ms[i] = ms[i];
-	return iwx_finish_image(J->ctx, host.data(), scan.get());
+	ctx->num_last_timings = k;
+	for (int i = 0; i < k; i++) ctx->last_timings_ms[i] = ms[i];
+	return done;
 }
 
 extern "C" void iwamd_job_destroy(struct iwamd_job *J)

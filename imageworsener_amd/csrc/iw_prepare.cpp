@@ -701,15 +701,46 @@ extern "C" int iwamd_prepare(struct iw_context *ctx, struct iwamd_plan *plan)
 // optimiser scan when there is one.
 int iwx_finish_image(struct iw_context *ctx, const uint8_t *img2, const iwx_opt_scan *scan)
 {
-	if (!ctx->prepared) {
-		iw_set_error(ctx, "Internal: finish without prepare");
-		return 0;
-	}
-	ctx->img2.pixels = (iw_byte *)iw_malloc_large(ctx, ctx->img2.bpr, ctx->img2.height);
-	if (!ctx->img2.pixels) return 0;
+	if (!iwx_finish_begin(ctx)) return 0;
 	memcpy(ctx->img2.pixels, img2, ctx->img2.bpr * ctx->img2.height);
-	ctx->prepared = 0;
 	return iwx_finish(ctx, scan);
+}
+
+static int finish_check(struct iw_context *ctx)
+{
+	if (ctx->prepared) return 1;
+	iw_set_error(ctx, "Internal: finish without prepare");
+	return 0;
+}
+
+iw_byte *iwx_finish_begin(struct iw_context *ctx)
+{
+	if (!finish_check(ctx)) return nullptr;
+	ctx->img2.pixels = (iw_byte *)iw_malloc_large(ctx, ctx->img2.bpr, ctx->img2.height);
+	if (!ctx->img2.pixels) return nullptr;
+	ctx->prepared = 0;
+	return ctx->img2.pixels;
+}
+
+// The unchanged image's size is held to the allocation limit here too, so
+// what was refused with it in host memory stays refused.
+int iwx_finish_decide(struct iw_context *ctx, const iwx_opt_scan *scan, iwx_out_conv *conv)
+{
+	if (!finish_check(ctx) || !iwx_alloc_check(ctx, ctx->img2.bpr, ctx->img2.height)) return 0;
+	ctx->prepared = 0;
+	return iwx_finish(ctx, scan, conv);
+}
+
+iw_byte *iwx_finish_pixels(struct iw_context *ctx, const iwx_out_conv &conv, size_t *bytes)
+{
+	iwx_opt_ctx &o = ctx->optctx;
+	iw_byte *p = (iw_byte *)iw_malloc_large(ctx, o.bpr, o.height);
+	if (!p) return nullptr;
+	if (conv.any) o.tmp_pixels = p;
+	else ctx->img2.pixels = p;
+	o.pixelsptr = p;
+	*bytes = o.bpr * (size_t)o.height;
+	return p;
 }
 
 extern "C" int iwamd_finish(struct iw_context *ctx, const uint8_t *img2)
