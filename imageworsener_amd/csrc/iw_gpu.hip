@@ -3551,6 +3551,9 @@ struct iwamd_job {
 	int band_rows = 0;  // rows per band of the fused kernel; 0: two-pass kernels
 	bool ran = false;
 	bool skip_pixels = false;  // unknown filter: the reference reports and outputs zeros
+	int device = 0;
+	std::vector<uint8_t> host_tables;  // being uploaded (a job made without waiting)
+	std::vector<double> host_input;
 	void *ws = nullptr;        // the job's work set (WorkSet)
 };
 
@@ -3562,14 +3565,24 @@ struct WOff { size_t start, src, w, copy, dfirst, dcount, doff, dw; };
 struct QOff { size_t T, U, lin, code, nc, ix, D, prow, pcol, M; };
 
 struct Staged {
-	std::vector<iwx::WeightList> wv, wh;
-	std::vector<iwx::DenseWeights> dv, dh;
+	// The different weight lists of each dimension -- one, unless channels are
+	// offset -- and which of them each channel has.
+	struct List {
+		iwx::WeightList wl;
+		iwx::DenseWeights d;
+		int channeltype = 0;
+	};
+	std::vector<List> lists[2];  // by IW_DIMENSION_*
+	int list_of[2][IWAMD_MAX_CH] = {};
+	const iwx::WeightList &wv(int c) const { return lists[IW_DIMENSION_V][list_of[IW_DIMENSION_V][c]].wl; }
+	const iwx::WeightList &wh(int c) const { return lists[IW_DIMENSION_H][list_of[IW_DIMENSION_H][c]].wl; }
+	const iwx::DenseWeights &dv(int c) const { return lists[IW_DIMENSION_V][list_of[IW_DIMENSION_V][c]].d; }
+	const iwx::DenseWeights &dh(int c) const { return lists[IW_DIMENSION_H][list_of[IW_DIMENSION_H][c]].d; }
 	std::vector<FastItem> fast;  // chosen-precision tiles (job index set when placed); empty: plain
-	std::vector<std::vector<double>> luts;
+	std::vector<std::shared_ptr<const std::vector<double>>> luts;
 	int ic_lut[4][3];
 	int alpha_lut = -1;
-	std::vector<iwx::QuantTable> qt;
-	std::vector<iwx::EdTables> et;
+	std::vector<std::shared_ptr<const iwx::QuantTable>> qt;  // by output channel
 	std::vector<iwx::PrngTables> pt;
 	int ed_of[4] = {-1, -1, -1, -1};
 	int n_ed = 0;
@@ -3590,7 +3603,7 @@ struct Staged {
 	size_t in_bytes = 0, out_bytes = 0;
 	size_t o_in = 0, o_inter = 0, o_out = 0, o_eds = 0, o_ede = 0;
 	std::vector<size_t> o_lut;
-	std::vector<WOff> ov, oh;
+	std::vector<WOff> o_list[2];  // by dimension, for each of its lists
 	std::vector<QOff> oq;
 	size_t bytes = 0;          // size of the job's part of a block
 	size_t o_tables = 0;       // start of the host-built tables (through the end of the part)
@@ -3604,11 +3617,11 @@ size_t band_lds_bytes(int R, int C, int W)
 
 // Whether bands of R output rows fit the band kernel: LDS for the rows and
 // input spans of at most BAND_MAX_K positions.
-bool band_fits(const iwamd_plan &p, const std::vector<iwx::DenseWeights> &dv, int R)
+bool band_fits(const iwamd_plan &p, const Staged &S, int R)
 {
 	if (band_lds_bytes(R, p.inter_nch, p.inter_width) > rt().band_lds_max) return false;
-	for (int c = 0; c < p.inter_nch; c++) {
-		const iwx::DenseWeights &d = dv[c];
+	for (const Staged::List &l : S.lists[IW_DIMENSION_V]) {
+		const iwx::DenseWeights &d = l.d;
 		for (int j0 = 0; j0 < p.inter_height; j0 += R) {
 			int lo = 0x7fffffff, hi = -0x7fffffff;
 			for (int r = 0; r < R && j0 + r < p.inter_height; r++) {
@@ -3623,16 +3636,22 @@ bool band_fits(const iwamd_plan &p, const std::vector<iwx::DenseWeights> &dv, in
 }
 
 // The tallest band that fits (0: none).
-int choose_band_rows(const iwamd_plan &p, const std::vector<iwx::DenseWeights> &dv)
+int choose_band_rows(const iwamd_plan &p, const Staged &S)
 {
 	for (int R : {4, 2, 1})
-		if (band_fits(p, dv, R)) return R;
+		if (band_fits(p, S, R)) return R;
 	return 0;
 }
 
-bool same_dense(const iwx::DenseWeights &a, const iwx::DenseWeights &b)
+// Whether every channel has the same weights in this dimension.
+bool one_list(const Staged &S, int dim)
 {
-	return a.first == b.first && a.count == b.count && a.off == b.off && a.w == b.w;
+	const std::vector<Staged::List> &l = S.lists[dim];
+	for (size_t k = 1; k < l.size(); k++) {
+		const iwx::DenseWeights &a = l[0].d, &b = l[k].d;
+		if (!(a.first == b.first && a.count == b.count && a.off == b.off && a.w == b.w)) return false;
+	}
+	return true;
 }
 
 // Positions [lo, lo + cnt) that rows a..a+n-1 of d reach (cnt 0: none).
@@ -3674,11 +3693,10 @@ void plan_fast(const iwamd_plan &p, Staged &S, int want_ti = 0)
 	if (p.out_sampletype == IW_SAMPLETYPE_FLOATINGPOINT || p.out_bit_depth > 16) return;
 	// Floating-point inputs can hold values past the form's range.
 	if (p.in_sampletype == IW_SAMPLETYPE_FLOATINGPOINT) return;
-	for (int c = 1; c < p.inter_nch; c++) {
-		if (!same_dense(S.dv[c], S.dv[0]) || !same_dense(S.dh[c], S.dh[0])) return;
-		if (S.wv[c].edge_value != S.wv[0].edge_value) return;
-	}
-	const iwx::DenseWeights &dv = S.dv[0], &dh = S.dh[0];
+	if (!one_list(S, IW_DIMENSION_V) || !one_list(S, IW_DIMENSION_H)) return;
+	for (int c = 1; c < p.inter_nch; c++)
+		if (p.ich[c].edge_sample_value[IW_DIMENSION_V] != p.ich[0].edge_sample_value[IW_DIMENSION_V]) return;
+	const iwx::DenseWeights &dv = S.dv(0), &dh = S.dh(0);
 	for (int j0 = 0; j0 < p.inter_height; j0 += FAST_ROWS) {
 		int lo, n;
 		dense_span(dv, j0, std::min(FAST_ROWS, p.inter_height - j0), lo, n);
@@ -3759,6 +3777,8 @@ bool build_f64_input(iw_context *ctx, const iwamd_plan &p, Staged &S, bool in_el
 	return true;
 }
 
+int ed_rows_shift(const Staged &S, const iwamd_plan &p);
+
 // Build the host tables of a plan, choose its path and lay out its device
 // data (offsets from the job's base).  path: "band", "twopass" or null.
 bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path, bool out_elsewhere = false,
@@ -3778,21 +3798,29 @@ bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path
 		for (int c = 0; c < p.inter_nch; c++) nonlinear |= p.ich[c].in_cs.cstype != IW_CSTYPE_LINEAR;
 		if (nonlinear && !build_f64_input(ctx, p, S, in_elsewhere)) return false;
 	}
-	S.wv.resize(p.inter_nch);
-	S.wh.resize(p.inter_nch);
-	S.dv.resize(p.inter_nch);
-	S.dh.resize(p.inter_nch);
+	for (int dim = 0; dim < 2; dim++) {
+		for (int c = 0; c < p.inter_nch; c++) {
+			// A list depends on the channel by its offset only.
+			const int type = p.rs[dim].use_offset ? p.ich[c].channeltype : 0;
+			std::vector<Staged::List> &l = S.lists[dim];
+			size_t k = 0;
+			while (k < l.size() && l[k].channeltype != type) k++;
+			if (k == l.size()) {
+				l.emplace_back();
+				l[k].channeltype = type;
+				l[k].wl = build_weight_list(p.rs[dim], type, 0.0);
+				l[k].d = dense_weights(l[k].wl);
+			}
+			S.list_of[dim][c] = (int)k;
+		}
+	}
 	for (int c = 0; c < p.inter_nch; c++) {
-		S.wv[c] = build_weight_list(p.rs[IW_DIMENSION_V], p.ich[c].channeltype, p.ich[c].edge_sample_value[IW_DIMENSION_V]);
-		S.wh[c] = build_weight_list(p.rs[IW_DIMENSION_H], p.ich[c].channeltype, p.ich[c].edge_sample_value[IW_DIMENSION_H]);
-		if (!S.wv[c].ok || !S.wh[c].ok) {
+		if (!S.wv(c).ok || !S.wh(c).ok) {
 			// The reference reports the error and carries on
 			// (src/imagew-resize.c:512-515).
 			iw_set_error(ctx, "Internal: Unknown resize algorithm");
 			S.skip_pixels = true;
 		}
-		S.dv[c] = dense_weights(S.wv[c]);
-		S.dh[c] = dense_weights(S.wh[c]);
 	}
 	S.in_int = p.in_sampletype != IW_SAMPLETYPE_FLOATINGPOINT;
 	const int nvalues = S.in_int ? (1 << p.in_bit_depth) : 0;
@@ -3827,12 +3855,11 @@ bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path
 		}
 	}
 	S.qt.resize(p.out_nch);
-	S.et.resize(p.out_nch);
 	S.pt.resize(p.out_nch);
 	if (p.out_sampletype != IW_SAMPLETYPE_FLOATINGPOINT) {
 		for (int o = 0; o < p.out_nch; o++) {
 			S.qt[o] = build_quant_table(p.och[o], p.och[o].use_nc_table != 0,
-				p.och[o].ditherfamily == IW_DITHERFAMILY_NONE);
+				p.och[o].ditherfamily == IW_DITHERFAMILY_NONE, p.och[o].ditherfamily == IW_DITHERFAMILY_ERRDIFF);
 			if (p.och[o].ditherfamily == IW_DITHERFAMILY_RANDOM) {
 				S.pt[o] = build_prng_tables(p.och[o].random_seed, p.out_width, p.out_height);
 				if (!S.pt[o].ok) {
@@ -3841,8 +3868,7 @@ bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path
 				}
 			}
 			if (p.och[o].ditherfamily == IW_DITHERFAMILY_ERRDIFF) {
-				S.et[o] = build_ed_tables(S.qt[o]);
-				if (S.qt[o].P > 65535) {
+				if (S.qt[o]->P > 65535) {
 					iw_set_error(ctx, "Too many output levels for error diffusion on the GPU path");
 					return false;
 				}
@@ -3889,12 +3915,12 @@ bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path
 		plan_fast(p, S, (want_ti == 16 || want_ti == 32) ? want_ti : 0);
 	if (!S.fast.empty()) {
 		S.shape_forced = S.fast_ti == want_ti;
-		build_h4(S.dh[0], S);
+		build_h4(S.dh(0), S);
 	}
 	if (S.fast.empty()) {
-		S.band_rows = force_two ? 0 : choose_band_rows(p, S.dv);
+		S.band_rows = force_two ? 0 : choose_band_rows(p, S);
 		if (!force_band && S.band_rows && p.inter_width > 2048) S.band_rows = 0;
-		if (S.band_rows && (want_rows == 1 || want_rows == 2 || want_rows == 4) && band_fits(p, S.dv, want_rows)) {
+		if (S.band_rows && (want_rows == 1 || want_rows == 2 || want_rows == 4) && band_fits(p, S, want_rows)) {
 			S.band_rows = want_rows;
 			S.shape_forced = true;
 		}
@@ -3908,41 +3934,39 @@ bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path
 	S.out_bytes = p.out_bpr * (size_t)p.out_height;
 	S.o_out = out_elsewhere ? 0 : L.add<uint8_t>(S.out_bytes);
 	S.o_eds = L.add<double>((size_t)S.n_ed * p.out_height * p.out_width);
-	S.o_ede = L.add<double>((size_t)S.n_ed * ed_rows_off(p.out_width, S.ed_seg).total);
+	S.o_ede = L.add<double>(ed_rows_shift(S, p) ? 0 : (size_t)S.n_ed * ed_rows_off(p.out_width, S.ed_seg).total);
 	S.o_tables = L.add<uint8_t>(0);
 	S.o_lut.resize(S.luts.size());
-	for (size_t i = 0; i < S.luts.size(); i++) S.o_lut[i] = L.add<double>(S.luts[i].size());
-	S.ov.resize(p.inter_nch);
-	S.oh.resize(p.inter_nch);
-	auto place_w = [&](const WeightList &wl, WOff &o) {
-		o.start = L.add<int>(wl.start.size());
-		o.src = L.add<int>(wl.src.size());
-		o.w = L.add<double>(wl.w.size());
-		o.copy = L.add<int>(wl.copy_src.size());
-	};
-	for (int c = 0; c < p.inter_nch; c++) {
-		place_w(S.wv[c], S.ov[c]);
-		place_w(S.wh[c], S.oh[c]);
-		S.ov[c].dfirst = L.add<int>(S.dv[c].first.size());
-		S.ov[c].dcount = L.add<int>(S.dv[c].count.size());
-		S.ov[c].doff = L.add<int>(S.dv[c].off.size());
-		S.ov[c].dw = L.add<double>(S.dv[c].w.size());
-		S.oh[c].dfirst = L.add<int>(S.dh[c].first.size());
-		S.oh[c].dcount = L.add<int>(S.dh[c].count.size());
-		S.oh[c].doff = L.add<int>(S.dh[c].off.size());
-		S.oh[c].dw = L.add<double>(S.dh[c].w.size());
+	for (size_t i = 0; i < S.luts.size(); i++) S.o_lut[i] = L.add<double>(S.luts[i]->size());
+	for (int dim = 0; dim < 2; dim++) {
+		for (const Staged::List &l : S.lists[dim]) {
+			WOff o;
+			o.start = L.add<int>(l.wl.start.size());
+			o.src = L.add<int>(l.wl.src.size());
+			o.w = L.add<double>(l.wl.w.size());
+			o.copy = L.add<int>(l.wl.copy_src.size());
+			o.dfirst = L.add<int>(l.d.first.size());
+			o.dcount = L.add<int>(l.d.count.size());
+			o.doff = L.add<int>(l.d.off.size());
+			o.dw = L.add<double>(l.d.w.size());
+			S.o_list[dim].push_back(o);
+		}
 	}
 	S.o_h4i = L.add<int4>(S.h4i.size());
 	S.o_h4w = L.add<float>(S.h4w.size());
 	S.oq.resize(p.out_nch);
-	// Channels whose tables are the same (the host builds each once per
-	// process) share one device copy.
+	// Channels whose tables are the same share one device copy: the host holds
+	// one per process of each, and tables of different options can be equal.
 	auto same_tables = [&](int a, int b) {
-		const iwx::QuantTable &x = S.qt[a], &y = S.qt[b];
+		if (S.pt[a].row_q != S.pt[b].row_q || S.pt[a].col_mont != S.pt[b].col_mont) return false;
+		if (S.qt[a] == S.qt[b]) return true;
+		const iwx::QuantTable &x = *S.qt[a], &y = *S.qt[b];
 		return x.P == y.P && x.ix_log2 == y.ix_log2 && x.code_is_level == y.code_is_level && x.T == y.T &&
-			x.U == y.U && x.lin == y.lin && x.code == y.code && x.nc == y.nc && x.ix == y.ix && x.D == y.D &&
-			S.pt[a].row_q == S.pt[b].row_q && S.pt[a].col_mont == S.pt[b].col_mont && S.et[a].M == S.et[b].M;
+			x.U == y.U && x.lin == y.lin && x.code == y.code && x.nc == y.nc && x.ix == y.ix && x.D == y.D && x.M == y.M;
 	};
+	static const std::shared_ptr<const iwx::QuantTable> no_table = std::make_shared<iwx::QuantTable>();
+	for (auto &q : S.qt)
+		if (!q) q = no_table;  // floating-point output
 	for (int o = 0; o < (int)S.qt.size(); o++) {
 		QOff &q = S.oq[o];
 		int same = -1;
@@ -3952,16 +3976,16 @@ bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path
 			q = S.oq[same];
 			continue;
 		}
-		q.T = L.add<double>(S.qt[o].T.size());
-		q.U = L.add<double>(S.qt[o].U.size());
-		q.lin = L.add<double>(S.qt[o].lin.size());
-		q.code = L.add<double>(S.qt[o].code.size());
-		q.nc = L.add<double>(S.qt[o].nc.size());
-		q.ix = L.add<uint16_t>(S.qt[o].ix.size());
-		q.D = L.add<double>(S.qt[o].D.size());
+		q.T = L.add<double>(S.qt[o]->T.size());
+		q.U = L.add<double>(S.qt[o]->U.size());
+		q.lin = L.add<double>(S.qt[o]->lin.size());
+		q.code = L.add<double>(S.qt[o]->code.size());
+		q.nc = L.add<double>(S.qt[o]->nc.size());
+		q.ix = L.add<uint16_t>(S.qt[o]->ix.size());
+		q.D = L.add<double>(S.qt[o]->D.size());
 		q.prow = L.add<uint64_t>(S.pt[o].row_q.size());
 		q.pcol = L.add<uint64_t>(S.pt[o].col_mont.size());
-		q.M = L.add<double>(S.et[o].M.size());
+		q.M = L.add<double>(S.qt[o]->M.size());
 	}
 	S.bytes = (L.off + 255) & ~(size_t)255;
 	return true;
@@ -3969,52 +3993,55 @@ bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path
 
 // Queue the host-to-device copies of a staged job into its part of a block:
 // the input image, then every host-built table in one copy of the tables
-// region from a host image of it (S.pack).  S must live until the stream has
-// been synchronised.
-bool upload_job(Staged &S, const iwamd_plan &p, char *base, hipStream_t st)
+// region from a host image of it (S.pack).  lists: the host image of a work
+// set placed right after the job's part (ws_pack), sent with it.  S must live
+// until the stream has been synchronised.
+bool upload_job(Staged &S, const iwamd_plan &p, char *base, hipStream_t st, const std::vector<uint8_t> *lists = nullptr)
 {
 	bool ok = true;
 	if (S.in_bytes && !S.in_elsewhere)
 		ok &= hipMemcpyAsync(base + S.o_in, S.in_f64.empty() ? p.in_pixels : (const void *)S.in_f64.data(), S.in_bytes,
 			hipMemcpyHostToDevice, st) == hipSuccess;
 	const size_t t0 = S.o_tables;
-	S.pack.assign(S.bytes - t0, 0);
+	S.pack.assign(S.bytes - t0 + (lists ? lists->size() : 0), 0);
+	if (lists && !lists->empty()) memcpy(S.pack.data() + (S.bytes - t0), lists->data(), lists->size());
 	auto up = [&](size_t off, const void *src, size_t bytes) {
 		if (bytes) memcpy(S.pack.data() + (off - t0), src, bytes);
 	};
-	for (size_t i = 0; i < S.luts.size(); i++) up(S.o_lut[i], S.luts[i].data(), S.luts[i].size() * 8);
-	auto up_w = [&](const iwx::WeightList &wl, const WOff &o) {
-		up(o.start, wl.start.data(), wl.start.size() * 4);
-		up(o.src, wl.src.data(), wl.src.size() * 4);
-		up(o.w, wl.w.data(), wl.w.size() * 8);
-		up(o.copy, wl.copy_src.data(), wl.copy_src.size() * 4);
-	};
-	for (int c = 0; c < p.inter_nch; c++) {
-		up_w(S.wv[c], S.ov[c]);
-		up_w(S.wh[c], S.oh[c]);
-		up(S.ov[c].dfirst, S.dv[c].first.data(), S.dv[c].first.size() * 4);
-		up(S.ov[c].dcount, S.dv[c].count.data(), S.dv[c].count.size() * 4);
-		up(S.ov[c].doff, S.dv[c].off.data(), S.dv[c].off.size() * 4);
-		up(S.ov[c].dw, S.dv[c].w.data(), S.dv[c].w.size() * 8);
-		up(S.oh[c].dfirst, S.dh[c].first.data(), S.dh[c].first.size() * 4);
-		up(S.oh[c].dcount, S.dh[c].count.data(), S.dh[c].count.size() * 4);
-		up(S.oh[c].doff, S.dh[c].off.data(), S.dh[c].off.size() * 4);
-		up(S.oh[c].dw, S.dh[c].w.data(), S.dh[c].w.size() * 8);
+	for (size_t i = 0; i < S.luts.size(); i++) up(S.o_lut[i], S.luts[i]->data(), S.luts[i]->size() * 8);
+	for (int dim = 0; dim < 2; dim++) {
+		for (size_t k = 0; k < S.lists[dim].size(); k++) {
+			const iwx::WeightList &wl = S.lists[dim][k].wl;
+			const iwx::DenseWeights &d = S.lists[dim][k].d;
+			const WOff &o = S.o_list[dim][k];
+			up(o.start, wl.start.data(), wl.start.size() * 4);
+			up(o.src, wl.src.data(), wl.src.size() * 4);
+			up(o.w, wl.w.data(), wl.w.size() * 8);
+			up(o.copy, wl.copy_src.data(), wl.copy_src.size() * 4);
+			up(o.dfirst, d.first.data(), d.first.size() * 4);
+			up(o.dcount, d.count.data(), d.count.size() * 4);
+			up(o.doff, d.off.data(), d.off.size() * 4);
+			up(o.dw, d.w.data(), d.w.size() * 8);
+		}
 	}
 	up(S.o_h4i, S.h4i.data(), S.h4i.size() * sizeof(int4));
 	up(S.o_h4w, S.h4w.data(), S.h4w.size() * sizeof(float));
 	for (int o = 0; o < (int)S.qt.size(); o++) {
 		const QOff &q = S.oq[o];
-		up(q.T, S.qt[o].T.data(), S.qt[o].T.size() * 8);
-		up(q.U, S.qt[o].U.data(), S.qt[o].U.size() * 8);
-		up(q.lin, S.qt[o].lin.data(), S.qt[o].lin.size() * 8);
-		up(q.code, S.qt[o].code.data(), S.qt[o].code.size() * 8);
-		up(q.nc, S.qt[o].nc.data(), S.qt[o].nc.size() * 8);
-		up(q.ix, S.qt[o].ix.data(), S.qt[o].ix.size() * 2);
-		up(q.D, S.qt[o].D.data(), S.qt[o].D.size() * 8);
+		const iwx::QuantTable &t = *S.qt[o];
+		bool placed = false;
+		for (int k = 0; k < o && !placed; k++) placed = S.oq[k].T == q.T && S.oq[k].U == q.U;
+		if (placed && !t.T.empty()) continue;  // shares an earlier channel's copy
+		up(q.T, t.T.data(), t.T.size() * 8);
+		up(q.U, t.U.data(), t.U.size() * 8);
+		up(q.lin, t.lin.data(), t.lin.size() * 8);
+		up(q.code, t.code.data(), t.code.size() * 8);
+		up(q.nc, t.nc.data(), t.nc.size() * 8);
+		up(q.ix, t.ix.data(), t.ix.size() * 2);
+		up(q.D, t.D.data(), t.D.size() * 8);
 		up(q.prow, S.pt[o].row_q.data(), S.pt[o].row_q.size() * 8);
 		up(q.pcol, S.pt[o].col_mont.data(), S.pt[o].col_mont.size() * 8);
-		up(q.M, S.et[o].M.data(), S.et[o].M.size() * 8);
+		up(q.M, t.M.data(), t.M.size() * 8);
 	}
 	if (!S.pack.empty())
 		ok &= hipMemcpyAsync(base + t0, S.pack.data(), S.pack.size(), hipMemcpyHostToDevice, st) == hipSuccess;
@@ -4052,8 +4079,6 @@ int ed_warm(const iwamd_ochan &o, int P)
 	return m1 ? 96 : 64;
 }
 
-int ed_rows_shift(const Staged &S, const iwamd_plan &p);
-
 void fill_dev_plan(const Staged &S, const iwamd_plan &p, char *base, DevPlan &D)
 {
 	memset(&D, 0, sizeof(D));
@@ -4085,12 +4110,8 @@ void fill_dev_plan(const Staged &S, const iwamd_plan &p, char *base, DevPlan &D)
 	}
 	D.W = p.inter_width;
 	D.Hp = p.inter_height;
-	D.v_shared = (int)S.dv.size() == p.inter_nch && p.inter_nch > 0;
-	for (int c = 0; c < (int)S.dv.size() && D.v_shared; c++)
-		if (!same_dense(S.dv[c], S.dv[0]) || S.wv[c].mode != iwx::WeightList::WEIGHTS) D.v_shared = 0;
-	D.h_shared = (int)S.dh.size() == p.inter_nch && p.inter_nch > 0;
-	for (int c = 0; c < (int)S.dh.size() && D.h_shared; c++)
-		if (!same_dense(S.dh[c], S.dh[0]) || S.wh[c].mode != iwx::WeightList::WEIGHTS) D.h_shared = 0;
+	D.v_shared = p.inter_nch > 0 && one_list(S, IW_DIMENSION_V) && S.wv(0).mode == iwx::WeightList::WEIGHTS;
+	D.h_shared = p.inter_nch > 0 && one_list(S, IW_DIMENSION_H) && S.wh(0).mode == iwx::WeightList::WEIGHTS;
 	for (int c = 0; c < p.inter_nch; c++) {
 		const iwamd_ichan &s = p.ich[c];
 		DevIChan &d = D.ic[c];
@@ -4107,27 +4128,24 @@ void fill_dev_plan(const Staged &S, const iwamd_plan &p, char *base, DevPlan &D)
 		d.lut_lin_max = 0.0;
 		if (d.lut[0] && s.in_cs.cstype == IW_CSTYPE_LINEAR && s.input_channel < p.in_nch_physical)
 			d.lut_lin_max = p.in_ch_slow[s.input_channel] ? p.in_ch_maxcolorcode[s.input_channel] : p.in_maxcolorcode;
-		auto fill = [&](const iwx::WeightList &wl, const WOff &o, DevWeights &dw, int dim) {
-			dw.mode = wl.mode;
+		auto fill = [&](DevWeights &dw, int dim) {
+			const Staged::List &l = S.lists[dim][S.list_of[dim][c]];
+			const WOff &o = S.o_list[dim][S.list_of[dim][c]];
+			dw.mode = l.wl.mode;
 			dw.start = (const int *)(base + o.start);
 			dw.src = (const int *)(base + o.src);
 			dw.w = (const double *)(base + o.w);
 			dw.copy_src = (const int *)(base + o.copy);
-			dw.edge = wl.edge_value;
+			dw.edge = s.edge_sample_value[dim];
 			dw.edge_transparent = p.rs[dim].edge_policy == IW_EDGE_POLICY_TRANSPARENT;
+			dw.dfirst = (const int *)(base + o.dfirst);
+			dw.dcount = (const int *)(base + o.dcount);
+			dw.doff = (const int *)(base + o.doff);
+			dw.dw = (const double *)(base + o.dw);
+			dw.dmax = l.d.max_count;
 		};
-		fill(S.wv[c], S.ov[c], d.v, IW_DIMENSION_V);
-		fill(S.wh[c], S.oh[c], d.h, IW_DIMENSION_H);
-		d.v.dfirst = (const int *)(base + S.ov[c].dfirst);
-		d.v.dcount = (const int *)(base + S.ov[c].dcount);
-		d.v.doff = (const int *)(base + S.ov[c].doff);
-		d.v.dw = (const double *)(base + S.ov[c].dw);
-		d.v.dmax = S.dv[c].max_count;
-		d.h.dfirst = (const int *)(base + S.oh[c].dfirst);
-		d.h.dcount = (const int *)(base + S.oh[c].dcount);
-		d.h.doff = (const int *)(base + S.oh[c].doff);
-		d.h.dw = (const double *)(base + S.oh[c].dw);
-		d.h.dmax = S.dh[c].max_count;
+		fill(d.v, IW_DIMENSION_V);
+		fill(d.h, IW_DIMENSION_H);
 	}
 	D.inter = (float *)(base + S.o_inter);
 	D.h4i = S.h4i.empty() ? nullptr : (const int4 *)(base + S.o_h4i);
@@ -4152,21 +4170,21 @@ void fill_dev_plan(const Staged &S, const iwamd_plan &p, char *base, DevPlan &D)
 		if (!D.out_float) {
 			const QOff &q = S.oq[o];
 			d.qmode = s.use_nc_table ? Q_NC : Q_THRESH;
-			d.P = S.qt[o].P;
+			d.P = S.qt[o]->P;
 			d.T = (const double *)(base + q.T);
 			d.U = (const double *)(base + q.U);
 			d.lin = (const double *)(base + q.lin);
 			d.code = (const double *)(base + q.code);
 			d.nc = (const double *)(base + q.nc);
-			d.ix = S.qt[o].ix.empty() ? nullptr : (const unsigned short *)(base + q.ix);
-			d.D = S.qt[o].D.empty() ? nullptr : (const double *)(base + q.D);
-			d.code_is_level = S.qt[o].code_is_level ? 1 : 0;
-			d.ix_le2 = !S.qt[o].ix.empty() && S.qt[o].ix_max <= 2;
-			d.ix_log2 = S.qt[o].ix_log2;
+			d.ix = S.qt[o]->ix.empty() ? nullptr : (const unsigned short *)(base + q.ix);
+			d.D = S.qt[o]->D.empty() ? nullptr : (const double *)(base + q.D);
+			d.code_is_level = S.qt[o]->code_is_level ? 1 : 0;
+			d.ix_le2 = !S.qt[o]->ix.empty() && S.qt[o]->ix_max <= 2;
+			d.ix_log2 = S.qt[o]->ix_log2;
 			d.prng_row = (const uint64_t *)(base + q.prow);
 			d.prng_col = (const uint64_t *)(base + q.pcol);
 			d.M = (const double *)(base + q.M);
-			d.ed_warm = S.ed_warm > 0 ? S.ed_warm : ed_warm(s, S.qt[o].P);
+			d.ed_warm = S.ed_warm > 0 ? S.ed_warm : ed_warm(s, S.qt[o]->P);
 		}
 	}
 	D.ed_samples = (double *)(base + S.o_eds);
@@ -4185,7 +4203,7 @@ void fill_dev_plan(const Staged &S, const iwamd_plan &p, char *base, DevPlan &D)
 	D.bk2a = p.bkgd2alpha;
 	D.vband_r = 0;
 	FastCin F;
-	if (!S.band_rows && S.fast.empty() && D.v_shared && fast_cin_depth(D, F)) D.vband_r = vband_rows(p, S.dv[0]);
+	if (!S.band_rows && S.fast.empty() && D.v_shared && fast_cin_depth(D, F)) D.vband_r = vband_rows(p, S.dv(0));
 }
 
 // ---- work sets ---------------------------------------------------------------
@@ -4245,7 +4263,7 @@ int ed_variant(const Staged &S, const iwamd_plan &p, int o, bool rows)
 		while (p.out_width > kEdrWidth[shape]) shape++;
 		return kEdRowsVariant + kEdrShapes * m1 + shape;
 	}
-	const int P = S.qt[o].P;
+	const int P = S.qt[o]->P;
 	const int tabm = P <= ED_SMALL_P ? 2 : (P <= ED_LDS_TABLE ? 1 : 0);
 	if (tabm) return 2 + 2 * tabm + m1;
 	return 2 * m1 + (p.out_width <= ED_ROWS_LDS && ed_cap(p.out_width, S.ed_seg) <= ED_CAP_LDS ? 1 : 0);
@@ -4258,7 +4276,7 @@ int ed_rows_shift(const Staged &S, const iwamd_plan &p)
 {
 	if (!S.n_ed || p.out_width > EDR_MAX_W) return 0;
 	for (int e = 0; e < S.n_ed; e++)
-		if (S.qt[S.ed_list[e]].P > ED_LDS_TABLE) return 0;
+		if (S.qt[S.ed_list[e]]->P > ED_LDS_TABLE) return 0;
 	return p.out_width <= 1024 ? 2 : 3;
 }
 
@@ -4288,6 +4306,7 @@ struct WorkSet {
 	const int2 *d_ilv = nullptr;
 	const int *d_chunks = nullptr;
 	int *d_counters = nullptr;
+	std::vector<uint8_t> pack;  // the lists' host image (ws_pack)
 };
 
 // The chosen-form kernel variant of a plan's tiles (FAST_*), decided by the
@@ -4393,13 +4412,12 @@ void ws_layout(WorkSet &W)
 	W.bytes = (L.off + 255) & ~(size_t)255;
 }
 
-// Queue the copies of the work lists to base (W must live until the stream
-// is synchronised).
-bool ws_upload(WorkSet &W, char *base, hipStream_t st)
+// The work lists' places at base, and their host image (W.pack).
+void ws_pack(WorkSet &W, char *base)
 {
-	bool ok = true;
+	W.pack.assign(W.bytes, 0);
 	auto up = [&](size_t off, const void *src, size_t bytes) {
-		if (bytes) ok &= hipMemcpyAsync(base + off, src, bytes, hipMemcpyHostToDevice, st) == hipSuccess;
+		if (bytes) memcpy(W.pack.data() + off, src, bytes);
 	};
 	W.d_plans = (const DevPlan *)(base + W.o_plans);
 	up(W.o_plans, W.plans.data(), W.plans.size() * sizeof(DevPlan));
@@ -4425,7 +4443,14 @@ bool ws_upload(WorkSet &W, char *base, hipStream_t st)
 	W.d_chunks = (const int *)(base + W.o_chunks);
 	up(W.o_chunks, W.fast_chunks, sizeof(W.fast_chunks));
 	W.d_done = (int *)(base + W.o_done);
-	return ok;
+}
+
+// Queue the copy of the work lists to base (W must live until the stream is
+// synchronised).
+bool ws_upload(WorkSet &W, char *base, hipStream_t st)
+{
+	ws_pack(W, base);
+	return hipMemcpyAsync(base, W.pack.data(), W.pack.size(), hipMemcpyHostToDevice, st) == hipSuccess;
 }
 
 int device_cu_count()
@@ -4520,12 +4545,12 @@ void ws_enqueue_errdiff(const WorkSet &W, hipStream_t st, bool interleave = true
 // horizontally for every output sample, per channel.
 double resample_flops(const iwamd_plan &p, const Staged &S)
 {
-	if (S.skip_pixels || S.dv.empty() || S.dh.empty()) return 0.0;
+	if (S.skip_pixels || S.lists[0].empty() || S.lists[1].empty()) return 0.0;
 	double f = 0.0;
 	for (int c = 0; c < p.inter_nch; c++) {
 		double tv = 0.0, th = 0.0;
-		for (int j = 0; j < p.inter_height; j++) tv += S.dv[c].count[j];
-		for (int i = 0; i < p.out_width; i++) th += S.dh[c].count[i];
+		for (int j = 0; j < p.inter_height; j++) tv += S.dv(c).count[j];
+		for (int i = 0; i < p.out_width; i++) th += S.dh(c).count[i];
 		f += 2.0 * (tv * p.inter_width + th * p.out_height);
 	}
 	return f;
@@ -4599,8 +4624,8 @@ TuneKey tune_key(const iwamd_plan &p, const Staged &S, int form)
 	TuneKey k;
 	k.form = form;
 	k.nch = p.inter_nch;
-	k.tv = log2_bucket(mean_taps(S.dv[0], p.inter_height));
-	k.th = log2_bucket(mean_taps(S.dh[0], p.out_width));
+	k.tv = log2_bucket(mean_taps(S.dv(0), p.inter_height));
+	k.th = log2_bucket(mean_taps(S.dh(0), p.out_width));
 	k.wb = log2_bucket(p.out_width / 64.0);
 	return k;
 }
@@ -4610,7 +4635,7 @@ int tune_cands(const iwamd_plan &p, const Staged &S, int form, int *cand)
 	int n = 0;
 	if (form == 0) {
 		for (int R : {4, 2, 1})
-			if (band_fits(p, S.dv, R)) cand[n++] = R;
+			if (band_fits(p, S, R)) cand[n++] = R;
 	} else {
 		cand[n++] = 32;
 		cand[n++] = 16;
@@ -4718,7 +4743,7 @@ void tune_apply(const iwamd_plan &p, Staged &S, hipStream_t st, bool may_tune)
 	tune_set(p, S, form, fits ? shape : orig);
 }
 
-bool job_upload(iwamd_job *J)
+bool job_upload(iwamd_job *J, bool wait)
 {
 	iw_context *ctx = J->ctx;
 	const iwamd_plan &p = J->plan;
@@ -4749,23 +4774,91 @@ bool job_upload(iwamd_job *J)
 	char *base = (char *)J->block;
 	fill_dev_plan(S, p, base, J->D);
 	W->plans[0] = J->D;
-	bool ok = upload_job(S, p, base, J->stream);
-	ok &= ws_upload(*W, base + S.bytes, J->stream);
-	// Host tables are freed when S goes out of scope: wait for the copies.
-	ok &= hipStreamSynchronize(J->stream) == hipSuccess;
+	ws_pack(*W, base + S.bytes);
+	bool ok = upload_job(S, p, base, J->stream, &W->pack);
+	J->out_pixels = (double)p.out_width * p.out_height;
+	J->alg_bytes = (double)S.in_bytes + (double)S.out_bytes;
+	if (wait) {
+		J->flops = resample_flops(p, S);
+		ok &= hipStreamSynchronize(J->stream) == hipSuccess;
+	} else {
+		// The host tables live until the job's next wait.
+		J->host_tables.swap(S.pack);
+		J->host_input.swap(S.in_f64);
+	}
 	if (!ok) {
 		iw_set_error(ctx, "Host-to-device copy failed");
 		return false;
 	}
-	J->out_pixels = (double)p.out_width * p.out_height;
-	J->alg_bytes = (double)S.in_bytes + (double)S.out_bytes;
-	J->flops = resample_flops(p, S);
 	return true;
+}
+
+// Streams and events of finished jobs, kept for the next ones: making and
+// freeing them costs more than a small image's kernels.  At most
+// kJobStreams per device; a set belongs to one job at a time.
+struct JobStream {
+	hipStream_t stream = nullptr;
+	hipEvent_t ev[4] = {nullptr, nullptr, nullptr, nullptr};
+};
+
+constexpr size_t kJobStreams = 8;
+
+struct JobStreams {
+	std::mutex mu;
+	std::map<int, std::vector<JobStream>> free;  // by device
+};
+
+JobStreams &job_streams()
+{
+	static JobStreams s;
+	return s;
+}
+
+void job_stream_free(JobStream &js)
+{
+	for (auto &e : js.ev)
+		if (e) hipEventDestroy(e);
+	if (js.stream) hipStreamDestroy(js.stream);
+	js = JobStream();
+}
+
+bool job_stream_get(int dev, JobStream &js)
+{
+	{
+		std::lock_guard<std::mutex> lock(job_streams().mu);
+		std::vector<JobStream> &v = job_streams().free[dev];
+		if (!v.empty()) {
+			js = v.back();
+			v.pop_back();
+			return true;
+		}
+	}
+	bool ok = hipStreamCreateWithFlags(&js.stream, hipStreamNonBlocking) == hipSuccess;
+	for (auto &e : js.ev) ok = ok && hipEventCreate(&e) == hipSuccess;
+	if (!ok) job_stream_free(js);
+	return ok;
+}
+
+// The stream is idle.
+void job_stream_put(int dev, JobStream &js)
+{
+	if (!js.stream) return;
+	{
+		std::lock_guard<std::mutex> lock(job_streams().mu);
+		std::vector<JobStream> &v = job_streams().free[dev];
+		if (v.size() < kJobStreams) {
+			v.push_back(js);
+			js = JobStream();
+			return;
+		}
+	}
+	job_stream_free(js);
 }
 
 }  // namespace
 
-extern "C" struct iwamd_job *iwamd_job_create(struct iw_context *ctx)
+// wait: until the uploads are done, so that the context's input may change.
+static struct iwamd_job *job_create(struct iw_context *ctx, bool wait)
 {
 	iwamd_job *J = new iwamd_job();
 	J->ctx = ctx;
@@ -4774,17 +4867,25 @@ extern "C" struct iwamd_job *iwamd_job_create(struct iw_context *ctx)
 		delete J;
 		return nullptr;
 	}
-	if (hipStreamCreateWithFlags(&J->stream, hipStreamNonBlocking) != hipSuccess) {
+	JobStream js;
+	if (hipGetDevice(&J->device) != hipSuccess) J->device = 0;
+	if (!job_stream_get(J->device, js)) {
 		iw_set_error(ctx, "hipStreamCreate failed");
 		delete J;
 		return nullptr;
 	}
-	for (auto &e : J->ev) hipEventCreate(&e);
-	if (!job_upload(J)) {
+	J->stream = js.stream;
+	for (int k = 0; k < 4; k++) J->ev[k] = js.ev[k];
+	if (!job_upload(J, wait)) {
 		iwamd_job_destroy(J);
 		return nullptr;
 	}
 	return J;
+}
+
+extern "C" struct iwamd_job *iwamd_job_create(struct iw_context *ctx)
+{
+	return job_create(ctx, true);
 }
 
 namespace {
@@ -4940,9 +5041,10 @@ extern "C" void iwamd_job_destroy(struct iwamd_job *J)
 	if (J->stream) hipStreamSynchronize(J->stream);
 	dev_release(J->block, J->block_bytes);
 	delete (WorkSet *)J->ws;
-	for (auto &e : J->ev)
-		if (e) hipEventDestroy(e);
-	if (J->stream) hipStreamDestroy(J->stream);
+	JobStream js;
+	js.stream = J->stream;
+	for (int k = 0; k < 4; k++) js.ev[k] = J->ev[k];
+	job_stream_put(J->device, js);
 	delete J;
 }
 
@@ -5099,7 +5201,8 @@ extern "C" int iwamd_process_device_noalloc(struct iw_context *ctx, const void *
 		hipLaunchKernelGGL(zero_bytes_kernel, dim3(std::max(grid, 1)), dim3(256), 0, st, (uint8_t *)d_out, need_out);
 	} else {
 		W.plans[0] = D;
-		ok = upload_job(S, p, base, st) && ws_upload(W, base + S.bytes, st);
+		ws_pack(W, base + S.bytes);
+		ok = upload_job(S, p, base, st, &W.pack);
 		if (ok) enqueue_job(W, D, st, nullptr);
 		if (ok && ctx->req.negate_target) {
 			NegateArgs a;
@@ -5184,8 +5287,8 @@ extern "C" int iwamd_ed_decide_check(const struct iwamd_ochan *och, int tab, int
 	int *level)
 {
 	if (och->use_nc_table) return -1;
-	const iwx::QuantTable q = iwx::build_quant_table(*och, false);
-	const iwx::EdTables t = iwx::build_ed_tables(q);
+	const std::shared_ptr<const iwx::QuantTable> table = iwx::build_quant_table(*och, false, false, true);
+	const iwx::QuantTable &q = *table, &t = q;
 	const int P = q.P;
 	if (tab == 1 && P > ED_LDS_TABLE) return 0;
 	if (tab == 2 && P > ED_SMALL_P) return 0;
@@ -5217,7 +5320,8 @@ extern "C" int iwamd_ed_decide_check(const struct iwamd_ochan *och, int tab, int
 extern "C" int iwamd_quant_fold_check(const struct iwamd_ochan *och, int n, const double *s, double *code)
 {
 	if (och->use_nc_table) return -1;
-	const iwx::QuantTable q = iwx::build_quant_table(*och, false, true);
+	const std::shared_ptr<const iwx::QuantTable> table = iwx::build_quant_table(*och, false, true);
+	const iwx::QuantTable &q = *table;
 	if (q.ix.empty()) return 0;
 	const int NB = 1 << q.ix_log2;
 	for (int i = 0; i < n; i++) {
@@ -5862,7 +5966,7 @@ int iwx_gpu_device_count(void)
 // iw_process_image's pixel work: one job, run once.
 int iwx_gpu_process(iw_context *ctx)
 {
-	iwamd_job *J = iwamd_job_create(ctx);
+	iwamd_job *J = job_create(ctx, false);
 	if (!J) return 0;
 	int ok = iwamd_job_run(J) && iwamd_job_finish(J);
 	iwamd_job_destroy(J);

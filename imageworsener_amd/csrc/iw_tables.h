@@ -8,6 +8,7 @@
 #include "iwamd.h"
 
 #include <cstdint>
+#include <memory>
 #include <string>
 #include <vector>
 
@@ -70,6 +71,11 @@ struct QuantTable {
 	// D[k] = min(T[k], max(T[k-1], U[k], M[k])) -- each D[k] lies in
 	// [T[k-1], T[k]], so D is ascending and counts only its own level's step.
 	std::vector<double> D;       // when folded (P entries)
+	// Error diffusion, when asked for: a non-exact sample s at level k is
+	// rounded up iff (lin[k+1] - s) <= (s - lin[k]) in FP64
+	// (src/imagew-main.c:730-748); both differences are monotone in s, so that
+	// holds exactly for s >= M[k] (M[P] = 2: never).
+	std::vector<double> M;
 	bool code_is_level = false;  // code[k] == k for every k
 	// Bin index over the array the quantiser searches (nc when used, else T),
 	// 2^ix_log2 bins of [0, 1]: ix[b] = #{m : a[m] < b / 2^ix_log2} for
@@ -81,18 +87,10 @@ struct QuantTable {
 };
 
 // want_nc: nearest-colour midpoints.  fold_none (no dither, no nc): the
-// searched array is QuantTable::D below instead of T.
-QuantTable build_quant_table(const iwamd_ochan &oc, bool want_nc, bool fold_none = false);
-
-// Decision data for error diffusion over a QuantTable (src/imagew-main.c:
-// 730-748).  A non-exact sample s at level k is rounded up iff
-// (lin[k+1] - s) <= (s - lin[k]) in FP64; both differences are monotone in s,
-// so that holds exactly for s >= M[k] (M[P] = 2: never).
-struct EdTables {
-	std::vector<double> M;
-};
-
-EdTables build_ed_tables(const QuantTable &q);
+// searched array is QuantTable::D below instead of T.  ed: QuantTable::M.
+// One table per process for each set of options.
+std::shared_ptr<const QuantTable> build_quant_table(const iwamd_ochan &oc, bool want_nc, bool fold_none = false,
+	bool ed = false);
 
 // The smallest s in [0, 1] with (hi - s) <= (s - lo) in FP64 (2: none; the
 // predicate is monotone in s).
@@ -101,8 +99,9 @@ double round_up_point(double lo, double hi);
 // (T, U) for a transfer function and level count; cached per process.
 const std::pair<std::vector<double>, std::vector<double>> &thresholds(const struct iw_csdescr &cs, int P);
 
-// Linearising lookup for integer input samples: lut[v] = X(v / maxcc).
-std::vector<double> build_input_lut(int nvalues, double maxcc, const struct iw_csdescr &cs);
+// Linearising lookup for integer input samples: lut[v] = X(v / maxcc).  One
+// table per process for each set of options.
+std::shared_ptr<const std::vector<double>> build_input_lut(int nvalues, double maxcc, const struct iw_csdescr &cs);
 
 // Random dithering: the reference's lag-1 complementary multiply-with-carry
 // generator (src/imagew-util.c:199-243) viewed as Q_n = Q_1 * b^-(n-1) mod m,
