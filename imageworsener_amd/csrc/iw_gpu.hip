@@ -2515,6 +2515,8 @@ __global__ void __launch_bounds__(ED_THREADS) errdiff_kernel(const DevPlan *__re
 // stride held up the rows: 2500-wide RGB 12 us a row with them).
 
 #define EDR_MAX_W 4096   // 8 waves of 64 segments of 8 pixels
+#define EDR_W4 1024      // widest row in segments of 4 pixels
+#define EDR_THREADS 512
 
 // One wave's row as its neighbours see it: its first and last two errors (by
 // x: the end state of a walk downwards or upwards) and the start state its
@@ -2893,19 +2895,15 @@ __global__ void __launch_bounds__(256) edr_interleave_kernel(const DevPlan *__re
 	for (int t = threadIdx.x; t < q * rows; t += 256) edr_interleave4(P, it.y + t / q, (t % q) * 4);
 }
 
-// One workgroup per plane: planes[b] = (plan, output channel), rows of at
-// most 64 * NW * SEG pixels.
+// One plane on the workgroup's first NW waves: rows of at most 64 * NW * SEG
+// pixels.
 template <bool M1, int SEG, int NW>
-__global__ void __launch_bounds__(64 * NW) errdiff_rows_kernel(const DevPlan *__restrict__ plans,
-	const int2 *__restrict__ planes)
+__device__ __forceinline__ void edr_plane(const DevPlan &P, int o, EdrLds<NW> &S)
 {
 	static_assert(SEG == 4 || SEG == 8, "a lane's 8-bit codes are whole words");
-	__shared__ EdrLds<NW> S;
 	constexpr int NT = 64 * NW;
 	const int tid = threadIdx.x;
-	const int2 pl = planes[blockIdx.x];
-	const DevPlan &P = plans[pl.x];
-	const DevOChan &q = P.oc[pl.y];
+	const DevOChan &q = P.oc[o];
 	const int Pq = q.P;
 	g_cf64 *T = (g_cf64 *)q.T, *U = (g_cf64 *)q.U, *M = (g_cf64 *)q.M, *lin = (g_cf64 *)q.lin;
 
@@ -2962,6 +2960,27 @@ __global__ void __launch_bounds__(64 * NW) errdiff_rows_kernel(const DevPlan *__
 	}
 	__syncthreads();
 	ed_complete(P, tid, NT);
+}
+
+// One workgroup per plane: planes[b] = (plan, output channel).  The plane's
+// width picks the waves that work and their segments; the others end at once
+// (a barrier waits for the waves that are left).  All widths are one launch,
+// since launches of one stream would run one after another, and with the
+// registers of the widest shape a workgroup has a CU to itself: two on one
+// CU would share its SIMDs, which a plane's chain keeps busy.
+template <bool M1>
+__global__ void __launch_bounds__(EDR_THREADS) errdiff_rows_kernel(const DevPlan *__restrict__ plans,
+	const int2 *__restrict__ planes)
+{
+	__shared__ __align__(16) unsigned char lds[sizeof(EdrLds<8>)];
+	const int2 pl = planes[blockIdx.x];
+	const DevPlan &P = plans[pl.x];
+	const int W = P.out_w, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	if (wave >= (W <= 256 ? 1 : (W <= 2048 ? 4 : 8))) return;
+	if (W <= 256) edr_plane<M1, 4, 1>(P, pl.y, *(EdrLds<1> *)lds);
+	else if (W <= EDR_W4) edr_plane<M1, 4, 4>(P, pl.y, *(EdrLds<4> *)lds);
+	else if (W <= 2048) edr_plane<M1, 8, 4>(P, pl.y, *(EdrLds<4> *)lds);
+	else edr_plane<M1, 8, 8>(P, pl.y, *(EdrLds<8> *)lds);
 }
 
 // ---- device memory and stream -------------------------------------------
@@ -4232,21 +4251,14 @@ struct EdVariant {
 	void (*kernel)(const DevPlan *, const int2 *);
 	int threads;
 };
-// Row shapes of errdiff_rows_kernel: (pixels per segment, waves), by width.
-#define EDR_SHAPES(M1) \
-	{errdiff_rows_kernel<M1, 4, 1>, 64}, {errdiff_rows_kernel<M1, 4, 2>, 128}, {errdiff_rows_kernel<M1, 4, 4>, 256}, \
-	{errdiff_rows_kernel<M1, 8, 4>, 256}, {errdiff_rows_kernel<M1, 8, 8>, 512}
-constexpr int kEdrShapes = 5;
-constexpr int kEdrWidth[kEdrShapes] = {256, 512, 1024, 2048, EDR_MAX_W};
-constexpr int kEdRowsVariant = 8;  // the first variant of errdiff_rows_kernel
-constexpr int kEdVariants = kEdRowsVariant + 2 * kEdrShapes;
+constexpr int kEdRowsVariant = 8;  // errdiff_rows_kernel
+constexpr int kEdVariants = kEdRowsVariant + 2;
 const EdVariant kEdKernels[kEdVariants] = {
 	{errdiff_kernel<0, false, false>, ED_THREADS}, {errdiff_kernel<0, false, true>, ED_THREADS},
 	{errdiff_kernel<0, true, false>, ED_THREADS}, {errdiff_kernel<0, true, true>, ED_THREADS},
 	{errdiff_kernel<1, false, false>, ED_THREADS}, {errdiff_kernel<1, true, false>, ED_THREADS},
 	{errdiff_kernel<2, false, false>, ED_THREADS}, {errdiff_kernel<2, true, false>, ED_THREADS},
-	EDR_SHAPES(false), EDR_SHAPES(true)};
-#undef EDR_SHAPES
+	{errdiff_rows_kernel<false>, EDR_THREADS}, {errdiff_rows_kernel<true>, EDR_THREADS}};
 
 // Kernel variant of one error-diffusion plane.  rows: the job runs
 // errdiff_rows_kernel (ed_rows_shift).  Else errdiff_kernel: decision records
@@ -4258,11 +4270,7 @@ int ed_variant(const Staged &S, const iwamd_plan &p, int o, bool rows)
 	const int subtype = p.och[o].dithersubtype;
 	const int sub = (subtype >= 0 && subtype <= 7) ? subtype : 0;
 	const int m1 = sub != 0 && sub != 6;
-	if (rows) {
-		int shape = 0;
-		while (p.out_width > kEdrWidth[shape]) shape++;
-		return kEdRowsVariant + kEdrShapes * m1 + shape;
-	}
+	if (rows) return kEdRowsVariant + m1;
 	const int P = S.qt[o]->P;
 	const int tabm = P <= ED_SMALL_P ? 2 : (P <= ED_LDS_TABLE ? 1 : 0);
 	if (tabm) return 2 + 2 * tabm + m1;
@@ -4277,7 +4285,7 @@ int ed_rows_shift(const Staged &S, const iwamd_plan &p)
 	if (!S.n_ed || p.out_width > EDR_MAX_W) return 0;
 	for (int e = 0; e < S.n_ed; e++)
 		if (S.qt[S.ed_list[e]]->P > ED_LDS_TABLE) return 0;
-	return p.out_width <= 1024 ? 2 : 3;
+	return p.out_width <= EDR_W4 ? 2 : 3;
 }
 
 struct WorkSet {
