@@ -69,7 +69,10 @@ struct DevWeights {
 	const int *copy_src;
 	double edge;
 	int edge_transparent;  // outside positions read edge (else the nearest sample)
-	// The list by input position (iwx::DenseWeights).
+	// The list by input position (iwx::DenseWeights).  Vertical lists: output
+	// j's weights at dw[doff[j]]..; horizontal ones: weight k of output i at
+	// dw[k * num_out + i], so that neighbouring pixels read neighbouring
+	// weights.
 	const int *dfirst, *dcount, *doff;
 	const double *dw;
 	int dmax;
@@ -731,12 +734,104 @@ __device__ __forceinline__ void emit_pixel(const DevPlan &P, int i, int j, Gathe
 	emit_px(E, i, j, gather);
 }
 
+// The horizontal pass and per-pixel work of column i of RR output rows from
+// j0 on, n of which exist, for plans whose channels share the horizontal list
+// (DevPlan::h_shared).  A tap's weight and position are read once for all
+// rows and channels; positions the list does not hold between its first and
+// last weigh 0 (stored as -0.0), which leaves a sum's bits unchanged for
+// finite samples.  SKIP: samples may not be finite, so those are left out.
+// load(c, r, x): sample x of intermediate row r.  Then the rows' pixels one by
+// one.
+template <int RR, bool SKIP, class Emit, class Load>
+__device__ __forceinline__ void hrows(const DevPlan &P, const Emit &E, int i, int j0, int n, Load load)
+{
+	const int C = P.inter_nch, W = P.W, ow = P.out_w;
+	const DevWeights &h0 = P.ic[0].h;
+	const int f0 = ((const g_cint *)h0.dfirst)[i], cnt = ((const g_cint *)h0.dcount)[i];
+	const g_cf64 *hw = (const g_cf64 *)h0.dw + i;
+	double acc[RR][IWAMD_MAX_CH];
+#pragma unroll
+	for (int r = 0; r < RR; r++)
+#pragma unroll
+		for (int c = 0; c < IWAMD_MAX_CH; c++) acc[r][c] = 0.0;
+	for (int u = 0; u < cnt; u++) {
+		const double w = hw[(size_t)u * ow];
+		const int pos = f0 + u;
+		const bool outside = pos < 0 || pos >= W;
+		const int pc = pos < 0 ? 0 : (pos >= W ? W - 1 : pos);
+		if (SKIP && __double_as_longlong(w) == (long long)(1ull << 63)) continue;
+#pragma unroll
+		for (int c = 0; c < IWAMD_MAX_CH; c++) {
+			if (c >= C) break;
+			const DevWeights &h = P.ic[c].h;
+			const bool edge = outside && h.edge_transparent;
+#pragma unroll
+			for (int r = 0; r < RR; r++) {
+				const double v = edge ? h.edge : (double)load(c, r, pc);
+				acc[r][c] = acc[r][c] + v * w;
+			}
+		}
+	}
+#pragma unroll
+	for (int r = 0; r < RR; r++) {
+		if (r >= n) break;
+		asm volatile("" ::: "memory");  // one pixel's work at a time: fewer registers
+		if constexpr (std::is_same<Emit, EmitSimple>::value) {
+			const int pi[1] = {i}, pj[1] = {j0 + r};
+			const bool live[1] = {true};
+			emit_px_simple<1, true>(E, pi, pj, live, [&](int, double (&g)[IWAMD_MAX_CH]) {
+#pragma unroll
+				for (int c = 0; c < IWAMD_MAX_CH; c++) g[c] = acc[r][c];
+			});
+		} else {
+			emit_px(E, i, j0 + r, [&](int c) {
+				return c == 0 ? acc[r][0] : (c == 1 ? acc[r][1] : (c == 2 ? acc[r][2] : acc[r][3]));
+			});
+		}
+	}
+}
+
 __global__ void __launch_bounds__(256) hpass_kernel(DevPlan P)
 {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
 	const int j = blockIdx.y;
 	if (i >= P.out_w) return;
 	emit_pixel(P, i, j, [&](int c) { return hgather(P, c, j, i); });
+}
+
+// The two-pass form's horizontal pass where the channels share the list and
+// the per-pixel work is simple: HP_ROWS rows per thread.  Bound by the loads
+// of the intermediate samples (L2) and, per pixel, the dependent table
+// searches; with a pixel per thread and a list read per channel it was bound
+// by the lists.  4000 to 1000 columns, 750 rows, RGB, Lanczos3: 316 -> 119 us;
+// 4096 to 1000, 1000 rows, RGBA, Mitchell: 318 -> 167 us.
+#define HP_ROWS 4
+__global__ void __launch_bounds__(256) hpass_rows_kernel(DevPlan P)
+{
+	const int i = blockIdx.x * blockDim.x + threadIdx.x;
+	const int j0 = blockIdx.y * HP_ROWS;
+	if (i >= P.out_w) return;
+	EmitSimple E;
+	emit_simple_ctx(P, E);
+	typedef const __attribute__((address_space(1))) float g_cf32;
+	hrows<HP_ROWS, false>(P, E, i, j0, min(HP_ROWS, P.out_h - j0), [&](int c, int r, int x) {
+		return ((const g_cf32 *)P.inter)[((size_t)c * P.Hp + min(j0 + r, P.out_h - 1)) * P.W + x];
+	});
+}
+
+// Queue the two-pass form's horizontal pass.  (Floating-point samples may not
+// be finite, so those plans keep to the list's own entries; the generic
+// per-pixel work is too large to repeat for several rows: with both in one
+// kernel it kept 1936 bytes per thread in scratch memory, 202 us for the first
+// size above.)
+void enqueue_hpass(const DevPlan &D, hipStream_t st)
+{
+	EmitSimple E;
+	const int nx = (D.out_w + 255) / 256;
+	if (D.h_shared && !D.in_float && emit_simple_ctx(D, E))
+		hipLaunchKernelGGL(hpass_rows_kernel, dim3(nx, (D.out_h + HP_ROWS - 1) / HP_ROWS), dim3(256), 0, st, D);
+	else
+		hipLaunchKernelGGL(hpass_kernel, dim3(nx, D.out_h), dim3(256), 0, st, D);
 }
 
 // ---- fused band kernel ------------------------------------------------------
@@ -1072,50 +1167,56 @@ __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned cha
 		}
 		return acc;
 	};
+	// With a shared list a thread takes one column of several of the band's
+	// rows, so that a weight is read once for them: all the rows where the
+	// columns fill the threads, fewer where that leaves less to do per thread
+	// (per column its rows and about one row's worth of weights).  3072 to 3072
+	// columns of grey, ordered dither: 530 -> 421 us; 1000 to 300, RGB over a
+	// background: 126 -> 90 us; 1000 to 1900, RGBA: 115 -> 106 us.
+	// (The generic per-pixel work goes row by row: it is too large to repeat,
+	// and meets floating-point input, whose samples may not be finite.)
+	auto columns = [&](const auto &E) {
+		constexpr bool SIMPLE = std::is_same<typename std::decay<decltype(E)>::type, EmitSimple>::value;
+		auto cost = [&](int g) { return (P.out_w + 256 / g - 1) / (256 / g) * (R / g + 1); };
+		int groups = 1;
+		if (R >= 2 && cost(2) < cost(groups)) groups = 2;
+		if (R >= 4 && cost(4) < cost(groups)) groups = 4;
+		const int cols = 256 / groups, per = R / groups, r0 = tid / cols * per, n = min(per, rows - r0);
+		if (n <= 0) return;
+		auto load = [&](int c, int r, int x) { return inter[((size_t)c * R + r0 + min(r, n - 1)) * W + x]; };
+		for (int i = tid % cols; i < P.out_w; i += cols) {
+			if constexpr (SIMPLE) {
+				if (per == 1) hrows<1, false>(P, E, i, j0 + r0, n, load);
+				else if (per == 2) hrows<(R < 2 ? 1 : 2), false>(P, E, i, j0 + r0, n, load);
+				else hrows<R, false>(P, E, i, j0 + r0, n, load);
+			} else {
+				for (int q = 0; q < n; q++)
+					hrows<1, true>(P, E, i, j0 + r0 + q, 1, [&](int c, int, int x) { return load(c, q, x); });
+			}
+		}
+	};
 	EmitSimple ES;
 	if (emit_simple_ctx(P, ES)) {
-		// Every channel's horizontal sum of one pixel: through the shared dense
-		// list (one weight load per tap for all channels) when the channels
-		// share it, else channel by channel.  A dense position the list does
-		// not hold weighs 0, which leaves a sum's bits unchanged.
-		const DevWeights &h0 = P.ic[0].h;
-		const g_cint *hfirst = (const g_cint *)h0.dfirst, *hcount = (const g_cint *)h0.dcount;
-		const g_cint *hoff = (const g_cint *)h0.doff;
-		const g_cf64 *hdw = (const g_cf64 *)h0.dw;
-		auto hsum_all = [&](int r, int i, double (&g)[IWAMD_MAX_CH]) {
-			if (!P.h_shared) {
-#pragma unroll
-				for (int c = 0; c < IWAMD_MAX_CH; c++) g[c] = c < C ? hsum(c, r, i) : 0.0;
-				return;
-			}
-			double acc[IWAMD_MAX_CH] = {0.0, 0.0, 0.0, 0.0};
-			const int f0 = hfirst[i], n = hcount[i], o0 = hoff[i];
-			for (int u = 0; u < n; u++) {
-				const double w = hdw[o0 + u];
-				const int pos = f0 + u;
-				const bool outside = pos < 0 || pos >= W;
-				const int pc = pos < 0 ? 0 : (pos >= W ? W - 1 : pos);
-#pragma unroll
-				for (int c = 0; c < IWAMD_MAX_CH; c++) {
-					if (c >= C) break;
-					const DevWeights &h = P.ic[c].h;
-					const double v = (outside && h.edge_transparent) ? h.edge :
-						(double)inter[((size_t)c * R + r) * W + pc];
-					acc[c] = acc[c] + v * w;
-				}
-			}
-#pragma unroll
-			for (int c = 0; c < IWAMD_MAX_CH; c++) g[c] = acc[c];
-		};
+		if (P.h_shared) {
+			columns(ES);
+			return;
+		}
 		for (int t = tid; t < n_px; t += blockDim.x) {
 			const int r[1] = {t / P.out_w}, pi[1] = {t % P.out_w};
 			const int pj[1] = {j0 + r[0]};
 			const bool live[1] = {true};
-			emit_px_simple<1, true>(ES, pi, pj, live, [&](int n, double (&g)[IWAMD_MAX_CH]) { hsum_all(r[n], pi[n], g); });
+			emit_px_simple<1, true>(ES, pi, pj, live, [&](int n, double (&g)[IWAMD_MAX_CH]) {
+#pragma unroll
+				for (int c = 0; c < IWAMD_MAX_CH; c++) g[c] = c < C ? hsum(c, r[n], pi[n]) : 0.0;
+			});
 		}
 	} else {
 		EmitCtx E;
 		emit_ctx(P, E);
+		if (P.h_shared) {
+			columns(E);
+			return;
+		}
 		for (int t = tid; t < n_px; t += blockDim.x) {
 			const int r = t / P.out_w, i = t % P.out_w;
 			emit_px(E, i, j0 + r, [&](int c) { return hsum(c, r, i); });
@@ -3967,7 +4068,7 @@ bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path
 			o.dfirst = L.add<int>(l.d.first.size());
 			o.dcount = L.add<int>(l.d.count.size());
 			o.doff = L.add<int>(l.d.off.size());
-			o.dw = L.add<double>(l.d.w.size());
+			o.dw = L.add<double>(dim == IW_DIMENSION_H ? (size_t)l.d.max_count * l.d.first.size() : l.d.w.size());
 			S.o_list[dim].push_back(o);
 		}
 	}
@@ -4040,7 +4141,14 @@ bool upload_job(Staged &S, const iwamd_plan &p, char *base, hipStream_t st, cons
 			up(o.dfirst, d.first.data(), d.first.size() * 4);
 			up(o.dcount, d.count.data(), d.count.size() * 4);
 			up(o.doff, d.off.data(), d.off.size() * 4);
-			up(o.dw, d.w.data(), d.w.size() * 8);
+			if (dim == IW_DIMENSION_V) {
+				up(o.dw, d.w.data(), d.w.size() * 8);
+			} else {
+				double *t = (double *)(S.pack.data() + (o.dw - t0));
+				const size_t n = d.first.size();
+				for (size_t i = 0; i < n; i++)
+					for (int k = 0; k < d.count[i]; k++) t[k * n + i] = d.w[d.off[i] + k];
+			}
 		}
 	}
 	up(S.o_h4i, S.h4i.data(), S.h4i.size() * sizeof(int4));
@@ -4532,7 +4640,7 @@ void ws_enqueue_resample(const WorkSet &W, hipStream_t st, bool persistent)
 	for (int jx : W.twopass) {
 		const DevPlan &D = W.plans[jx];
 		enqueue_vpass(D, st);
-		hipLaunchKernelGGL(hpass_kernel, dim3((D.out_w + 255) / 256, D.out_h), dim3(256), 0, st, D);
+		enqueue_hpass(D, st);
 	}
 }
 
@@ -4911,7 +5019,7 @@ void enqueue_job(const WorkSet &W, const DevPlan &D, hipStream_t st, hipEvent_t 
 	} else {
 		enqueue_vpass(D, st);
 		if (ev) hipEventRecord(ev[1], st);
-		hipLaunchKernelGGL(hpass_kernel, dim3((D.out_w + 255) / 256, D.out_h), dim3(256), 0, st, D);
+		enqueue_hpass(D, st);
 	}
 	if (ev) hipEventRecord(ev[2], st);
 	ws_enqueue_errdiff(W, st);

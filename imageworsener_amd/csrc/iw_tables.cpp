@@ -457,7 +457,7 @@ DenseWeights dense_weights(const WeightList &wl)
 			const int p0 = wl.pos[a], p1 = wl.pos[b - 1];
 			d.first[o] = p0;
 			d.count[o] = p1 - p0 + 1;
-			d.w.resize(d.off[o] + d.count[o], 0.0);
+			d.w.resize(d.off[o] + d.count[o], -0.0);
 			for (int t = a; t < b; t++) d.w[d.off[o] + (wl.pos[t] - p0)] = wl.w[t];
 		}
 		d.max_count = std::max(d.max_count, d.count[o]);

@@ -33,7 +33,7 @@ struct WeightList {
 };
 
 // The same list by input position: output o reads positions
-// first[o] .. first[o]+count[o]-1 with weights w[off[o] + k], zero where the
+// first[o] .. first[o]+count[o]-1 with weights w[off[o] + k], -0.0 where the
 // list has no entry (a dropped zero weight: adding v*0 to an accumulator that
 // is never -0.0 leaves its bits unchanged).  A position outside 0..num_in-1
 // reads the edge value (TRANSPARENT) or the nearest sample (REPLICATE); the
