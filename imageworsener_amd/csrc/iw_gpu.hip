@@ -57,6 +57,7 @@ typedef __attribute__((address_space(1))) unsigned char g_u8;
 typedef const __attribute__((address_space(1))) double g_cf64;
 typedef const __attribute__((address_space(1))) unsigned short g_cu16;
 typedef const __attribute__((address_space(1))) int g_cint;
+typedef const __attribute__((address_space(1))) float g_cf32;
 typedef __attribute__((address_space(1), aligned(1))) unsigned int g_u32u;  // at any byte
 
 // ---- device-side plan ----------------------------------------------------
@@ -138,6 +139,7 @@ struct DevPlan {
 	size_t out_bytes;
 	int apply_bkgd, late, checker, check_size, ox, oy, bk_has_trans;
 	int v_shared;  // every channel has the same vertical weights (dense form) in WEIGHTS mode
+	int band_lds_max;  // fused form: LDS a workgroup may use
 	int vband_r;   // two-pass form: output rows per thread of vband_kernel (0: vpass_kernel)
 	int h_shared;  // the same for the horizontal weights
 	double bk1a, bk2a;
@@ -813,7 +815,6 @@ __global__ void __launch_bounds__(256) hpass_rows_kernel(DevPlan P)
 	if (i >= P.out_w) return;
 	EmitSimple E;
 	emit_simple_ctx(P, E);
-	typedef const __attribute__((address_space(1))) float g_cf32;
 	hrows<HP_ROWS, false>(P, E, i, j0, min(HP_ROWS, P.out_h - j0), [&](int c, int r, int x) {
 		return ((const g_cf32 *)P.inter)[((size_t)c * P.Hp + min(j0 + r, P.out_h - 1)) * P.W + x];
 	});
@@ -883,6 +884,7 @@ struct FastCin {
 	// the device divides exactly (the table holds the same quotients).
 	double lmax[IWAMD_MAX_CH], amax;
 	int lean;                // no channel in mode 2 and none with a transparent edge
+	int slot[IWAMD_MAX_CH], aslot;  // 8-bit tables in LDS (fast_cin_slots): each channel's, the alpha's
 };
 
 __host__ __device__ inline int fast_cin_depth(const DevPlan &P, FastCin &F)
@@ -933,12 +935,88 @@ __host__ __device__ inline int fast_cin_depth(const DevPlan &P, FastCin &F)
 	return P.bit_depth;
 }
 
-// The plain form's vertical passes keep the tables for linear channels too:
-// with its FP64 sums per band row, a division costs more there than a gather.
-__host__ __device__ inline void fast_cin_tables_only(FastCin &F)
+// The same for 32-bit floating-point samples ("depth" 33), whose value is the
+// sample itself.  (The fused form's bands only: they weigh positions outside
+// a row's list by 0, which for samples that are not finite differs from
+// leaving them out, as the other forms do.)
+__host__ __device__ inline int float_cin_depth(const DevPlan &P, FastCin &F)
 {
-	for (int c = 0; c < IWAMD_MAX_CH; c++) F.lmax[c] = 0.0;
+	if (!P.in_float || P.bit_depth != 32 || P.in_f64) return 0;
+	bool need_a = false;
+	F.lean = 1;
+	for (int c = 0; c < IWAMD_MAX_CH; c++) {
+		const DevIChan &ic = P.ic[c < P.inter_nch ? c : 0];
+		if (ic.cvt_gray || ic.input_channel >= P.nch_phys) return 0;
+		F.chb[c] = ic.input_channel * 4;
+		F.lut[c] = nullptr;
+		F.mode[c] = ic.need_unassoc ? 1 : (ic.early_bkgd ? 2 : 0);
+		F.bkgd[c] = ic.bkgd;
+		F.edge[c] = ic.v.edge;
+		F.et[c] = ic.v.edge_transparent;
+		F.lmax[c] = 0.0;
+		need_a |= F.mode[c] != 0;
+		if (F.mode[c] == 2 || F.et[c]) F.lean = 0;
+	}
+	F.ab = F.chb[0];
+	F.alut = nullptr;
 	F.amax = 0.0;
+	if (need_a) {
+		if (P.alpha_in_index >= P.nch_phys) return 0;
+		F.ab = P.alpha_in_index * 4;
+	}
+	int rx, ry;
+	long long o[3];
+	const int px[3] = {0, 1, 0}, py[3] = {0, 0, 1};
+	for (int k = 0; k < 3; k++) {
+		logical_to_physical(P, px[k], py[k], rx, ry);
+		o[k] = (long long)ry * (long long)P.in_bpr + (long long)rx * P.nch_phys * 4;
+	}
+	F.base = o[0];
+	F.dx = o[1] - o[0];
+	F.dy = o[2] - o[0];
+	return ((F.base | F.dx | F.dy) & 3) || ((uintptr_t)P.in & 3) ? 0 : 33;
+}
+
+// 8-bit input: up to two different tables go to LDS, where a gather does not
+// cost a cache line per lane.  Fills lds and F.slot; false: more tables.
+#define CIN_LDS (2 * 256 * sizeof(double))
+__device__ __forceinline__ bool fast_cin_slots(FastCin &F, double *lds)
+{
+	const double *t[2] = {F.lut[0], nullptr};
+	bool ok = true;
+	auto slot = [&](const double *p) {
+		if (p == t[0]) return 0;
+		if (!t[1]) t[1] = p;
+		if (p == t[1]) return 1;
+		ok = false;
+		return 0;
+	};
+	for (int c = 0; c < IWAMD_MAX_CH; c++) F.slot[c] = slot(F.lut[c]);
+	F.aslot = slot(F.alut);
+	if (!ok) return false;
+	for (int k = threadIdx.x; k < 512; k += blockDim.x)
+		if (t[k >> 8]) lds[k] = ((const g_cf64 *)t[k >> 8])[k & 255];
+	return true;
+}
+
+// Which of the plain form's vertical passes a direct colour-in takes: the
+// channel count for whole pixels without background or transparent edges (one
+// or three channels as read, or four with the alpha last), else 0.
+__device__ __forceinline__ int fast_cin_channels(const FastCin &F, int C)
+{
+	const bool as_read = !F.mode[0] && !F.mode[1] && !F.mode[2] && !F.mode[3];
+	if (!F.lean) return 0;
+	if (C == 1 || C == 3) return as_read ? C : 0;
+	if (C != 4 || F.mode[3]) return 0;
+	return as_read || (F.ab == F.chb[3] && F.alut == F.lut[3]) ? 4 : 0;
+}
+
+// v / 65535, correctly rounded, for whole v in 0..65535: the quotient by the
+// reciprocal and one residual step.
+__host__ __device__ inline double div65535(unsigned int v)
+{
+	const double r = 1.0 / 65535.0, x = (double)v, q = x * r;
+	return __builtin_fma(__builtin_fma(-q, 65535.0, x), r, q);
 }
 
 template <int DEPTH>
@@ -953,9 +1031,10 @@ __device__ __forceinline__ unsigned int fast_raw(const g_u8 *in, long long off)
 // (channels from C on are left unspecified).  LEAN: no early background and
 // no transparent edge (FastCin::lean), so a channel is its table value times
 // alpha or times 1 (which leaves it unchanged).
-template <int DEPTH, bool LEAN, class T = float>
+// lds: 8-bit tables as fast_cin_slots placed them, or null.
+template <int DEPTH, bool LEAN, class T = float, bool LDS = false>
 __device__ __forceinline__ void fast_fetch(const DevPlan &P, const FastCin &F, long long cb, int p,
-	T v[IWAMD_MAX_CH])
+	T v[IWAMD_MAX_CH], const double *lds = nullptr)
 {
 	const int C = P.inter_nch;
 	if (DEPTH == 0) {
@@ -968,6 +1047,17 @@ __device__ __forceinline__ void fast_fetch(const DevPlan &P, const FastCin &F, l
 	const int pin = p < 0 ? 0 : (p >= P.ih ? P.ih - 1 : p);
 	const long long off = cb + (long long)pin * F.dy;
 	const g_u8 *in = (const g_u8 *)P.in;
+	if (DEPTH == 33) {
+		const double a = (double)*(g_cf32 *)(in + off + F.ab);
+#pragma unroll
+		for (int c = 0; c < IWAMD_MAX_CH; c++) {
+			const double x = (double)*(g_cf32 *)(in + off + F.chb[c]);
+			double y = F.mode[c] == 1 ? x * a : (F.mode[c] == 2 ? a * x + (1.0 - a) * F.bkgd[c] : x);
+			if (p != pin && F.et[c]) y = F.edge[c];
+			v[c] = (T)y;
+		}
+		return;
+	}
 	unsigned int raw[IWAMD_MAX_CH], araw;
 	if (DEPTH == 32) {
 		const unsigned int word = *(const __attribute__((address_space(1))) unsigned int *)(in + off);
@@ -991,14 +1081,17 @@ __device__ __forceinline__ void fast_fetch(const DevPlan &P, const FastCin &F, l
 	}
 	// 16-bit tables are 512 KiB, so a gather costs a cache line per lane; a
 	// linear channel divides instead.
-	auto value = [&](unsigned int v, const double *lut, double lmax) {
-		if ((DEPTH == 16 || DEPTH == 64) && lmax > 0.0) return (double)v / lmax;
+	// (Not for the plain form, T double, whose calls with linear channels are
+	// band_fetch's.)
+	auto value = [&](unsigned int v, const double *lut, double lmax, int slot) {
+		if (std::is_same<T, float>::value && (DEPTH == 16 || DEPTH == 64) && lmax > 0.0) return (double)v / lmax;
+		if constexpr (LDS) return lds[slot * 256 + v];
 		return ((const g_cf64 *)lut)[v];
 	};
-	const double a = value(araw, F.alut, F.amax);
+	const double a = value(araw, F.alut, F.amax, F.aslot);
 #pragma unroll
 	for (int c = 0; c < IWAMD_MAX_CH; c++) {
-		const double x = value(raw[c], F.lut[c], F.lmax[c]);
+		const double x = value(raw[c], F.lut[c], F.lmax[c], F.slot[c]);
 		if (LEAN) {
 			v[c] = (T)(x * (F.mode[c] ? a : 1.0));
 			continue;
@@ -1011,19 +1104,64 @@ __device__ __forceinline__ void fast_fetch(const DevPlan &P, const FastCin &F, l
 	}
 }
 
+// fast_fetch for the NC channels of fast_cin_channels: 1 or 3 as read, or 4
+// with the alpha last.  LIN: 16-bit channels that are all linear and
+// full-range, which divide instead of reading the tables.
+template <int DEPTH, int NC, bool LIN>
+__device__ __forceinline__ void band_fetch(const DevPlan &P, const FastCin &F, long long cb, int p, double v[NC],
+	const double *lds)
+{
+	const int pin = p < 0 ? 0 : (p >= P.ih ? P.ih - 1 : p);
+	const g_u8 *in = (const g_u8 *)P.in + (cb + (long long)pin * F.dy);
+	unsigned int raw[NC];
+	if (DEPTH == 32) {
+		const unsigned int word = *(const __attribute__((address_space(1))) unsigned int *)in;
+#pragma unroll
+		for (int c = 0; c < NC; c++) raw[c] = (word >> (8 * F.chb[c])) & 0xffu;
+	} else if (DEPTH == 64) {
+		const unsigned long long word = *(const __attribute__((address_space(1))) unsigned long long *)in;
+#pragma unroll
+		for (int c = 0; c < NC; c++) {
+			const unsigned int h = (unsigned int)(word >> (8 * F.chb[c])) & 0xffffu;
+			raw[c] = ((h & 0xffu) << 8) | (h >> 8);
+		}
+	} else if (DEPTH != 33) {
+#pragma unroll
+		for (int c = 0; c < NC; c++) raw[c] = fast_raw<DEPTH>(in, F.chb[c]);
+	}
+#pragma unroll
+	for (int c = 0; c < NC; c++) {
+		if (DEPTH == 33) v[c] = (double)*(g_cf32 *)(in + F.chb[c]);
+		else if (DEPTH == 8 || DEPTH == 32) v[c] = lds[F.slot[c] * 256 + raw[c]];
+		else if (LIN) v[c] = div65535(raw[c]);
+		else v[c] = ((const g_cf64 *)F.lut[c])[raw[c]];
+	}
+	if (NC == 4) {
+#pragma unroll
+		for (int c = 0; c < NC - 1; c++) v[c] = v[c] * (F.mode[c] ? v[NC - 1] : 1.0);
+	}
+}
+
 // The band's vertical pass when every channel shares one weight list
 // (DevPlan::v_shared) and the input takes the direct colour-in: each column's
 // pixels are read once for all channels, four input rows at a time with every
 // load issued before the first is used.  Each accumulator still gets its terms
 // in list order, with the same FP64 operations as colour_in and the generic
-// pass.
+// pass.  NC: fast_cin_channels (0: any plan, through fast_fetch).
+// Bound by the table gathers, then the FP64 sums: with the tables in LDS and
+// only the plan's own channels looked up (five gathers per pixel before,
+// whatever the channels), 4000x3000 RGB to 750 rows: 159 -> 88 us; 16-bit
+// (tables in L2), 1500 to 375 rows: 180 -> 138 us; the fused kernel for 3072
+// squared of grey 475 -> 390 us, 1023x767 floats (through colour_in before)
+// 135 -> 55 us, 640x480 RGB to 320x240 65 -> 52 us.
 // Columns x0, x0 + xstep, ... below W; row r of channel c of column x goes to
 // out[c * cstride + r * W + x].
-template <int R, int DEPTH, bool LEAN>
-__device__ __forceinline__ void band_vertical_direct(const DevPlan &P, const FastCin &F, int j0, int rows,
-	const double *wd, float *out, size_t cstride, int x0, int xstep)
+template <int R, int DEPTH, int NC, bool LIN, bool LDS>
+__device__ __forceinline__ void band_vertical(const DevPlan &P, const FastCin &F, int j0, int rows,
+	const double *wd, float *out, size_t cstride, int x0, int xstep, const double *lds)
 {
-	const int W = P.W, C = P.inter_nch;
+	constexpr int NV = NC ? NC : IWAMD_MAX_CH;
+	const int W = P.W, C = NC ? NC : P.inter_nch;
 	const DevWeights &dv = P.ic[0].v;
 	int p_lo = 0x7fffffff, p_hi = -0x7fffffff;
 	for (int r = 0; r < rows; r++) {
@@ -1035,20 +1173,24 @@ __device__ __forceinline__ void band_vertical_direct(const DevPlan &P, const Fas
 	const int K = (p_hi >= p_lo) ? p_hi - p_lo + 1 : 0;
 	for (int x = x0; x < W; x += xstep) {
 		const long long cb = F.base + (long long)x * F.dx;
-		double acc[IWAMD_MAX_CH][R];
+		double acc[NV][R];
 #pragma unroll
-		for (int c = 0; c < IWAMD_MAX_CH; c++)
+		for (int c = 0; c < NV; c++)
 #pragma unroll
 			for (int r = 0; r < R; r++) acc[c][r] = 0.0;
 		for (int k = 0; k < K; k += 4) {
-			double v[4][IWAMD_MAX_CH];
+			double v[4][NV];
 #pragma unroll
-			for (int t = 0; t < 4; t++) fast_fetch<DEPTH, LEAN, double>(P, F, cb, p_lo + min(k + t, K - 1), v[t]);
+			for (int t = 0; t < 4; t++) {
+				const int p = p_lo + min(k + t, K - 1);
+				if constexpr (NC) band_fetch<DEPTH, NC, LIN>(P, F, cb, p, v[t], lds);
+				else fast_fetch<DEPTH, false, double, LDS>(P, F, cb, p, v[t], lds);
+			}
 #pragma unroll
 			for (int t = 0; t < 4; t++) {
 				if (k + t >= K) break;
 #pragma unroll
-				for (int c = 0; c < IWAMD_MAX_CH; c++) {
+				for (int c = 0; c < NV; c++) {
 					if (c >= C) break;
 #pragma unroll
 					for (int r = 0; r < R; r++) acc[c][r] = acc[c][r] + v[t][c] * wd[r * BAND_MAX_K + k + t];
@@ -1056,7 +1198,7 @@ __device__ __forceinline__ void band_vertical_direct(const DevPlan &P, const Fas
 			}
 		}
 #pragma unroll
-		for (int c = 0; c < IWAMD_MAX_CH; c++) {
+		for (int c = 0; c < NV; c++) {
 			if (c >= C) break;
 #pragma unroll
 			for (int r = 0; r < R; r++) {
@@ -1069,19 +1211,76 @@ __device__ __forceinline__ void band_vertical_direct(const DevPlan &P, const Fas
 	}
 }
 
+// band_vertical of a direct colour-in (depth != 0).  tab: room for the 8-bit
+// tables (CIN_LDS bytes, written here; ends with a barrier), or null.
+template <int R, bool FLOAT>
+__device__ __forceinline__ void band_vertical_direct(int depth, FastCin &F, const DevPlan &P, int j0, int rows,
+	const double *wd, float *out, size_t cs, int x0, int xs, double *tab)
+{
+	const bool lds = (depth == 8 || depth == 32) && tab && fast_cin_slots(F, tab);
+	__syncthreads();
+	int nc = fast_cin_channels(F, P.inter_nch);
+	if (depth == 8 || depth == 32) {
+		if (!lds) {
+			if (depth == 32) band_vertical<R, 32, 0, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+			else band_vertical<R, 8, 0, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+		} else if (depth == 32) {
+			if (nc == 4) band_vertical<R, 32, 4, false, true>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+			else band_vertical<R, 32, 0, false, true>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+		} else {
+			if (nc == 3) band_vertical<R, 8, 3, false, true>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+			else if (nc == 1) band_vertical<R, 8, 1, false, true>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+			else band_vertical<R, 8, 0, false, true>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+		}
+		return;
+	}
+	if (FLOAT && depth == 33) {
+		if (nc == 4) band_vertical<R, 33, 4, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+		else if (nc == 3) band_vertical<R, 33, 3, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+		else band_vertical<R, 33, 0, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+		return;
+	}
+	const bool lin = F.lmax[0] == 65535.0 && F.lmax[1] == 65535.0 && F.lmax[2] == 65535.0 && F.lmax[3] == 65535.0;
+	if (depth == 64 && nc == 4) {
+		if (lin) band_vertical<R, 64, 4, true, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+		else band_vertical<R, 64, 4, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+	} else if (depth == 16 && nc == 3) {
+		if (lin) band_vertical<R, 16, 3, true, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+		else band_vertical<R, 16, 3, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+	} else if (depth == 16 && nc == 1) {
+		if (lin) band_vertical<R, 16, 1, true, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+		else band_vertical<R, 16, 1, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+	} else {
+		band_vertical<R, 16, 0, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+	}
+}
+
+// LDS of a band of R rows: its weights, its samples and, for 8-bit input with
+// room for them, the tables of the direct colour-in.
+__host__ __device__ inline size_t band_lds_rows(int R, int C, int W)
+{
+	return sizeof(double) * (size_t)R * BAND_MAX_K + sizeof(float) * (size_t)C * R * W;
+}
+
+__host__ __device__ inline bool band_has_tab(bool in8, int R, int C, int W, size_t lds_max)
+{
+	return in8 && band_lds_rows(R, C, W) + CIN_LDS <= lds_max;
+}
+
 template <int R>
 __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned char *band_lds)
 {
 	double *wd = (double *)band_lds;                       // [R][BAND_MAX_K]
-	float *inter = (float *)(band_lds + sizeof(double) * R * BAND_MAX_K);  // [C][R][W]
+	double *tab = band_has_tab(P.bit_depth == 8 && !P.in_float, R, P.inter_nch, P.W, P.band_lds_max) ? wd + R * BAND_MAX_K : nullptr;  // [2][256]
+	float *inter = (float *)(wd + R * BAND_MAX_K + (tab ? CIN_LDS / sizeof(double) : 0));  // [C][R][W]
 	const int tid = threadIdx.x;
 	const int rows = min(R, P.Hp - j0);
 	const int W = P.W, C = P.inter_nch;
 	const int num_in = P.ih;
 
 	FastCin F;
-	const int depth = P.v_shared ? fast_cin_depth(P, F) : 0;
-	fast_cin_tables_only(F);
+	int depth = P.v_shared ? fast_cin_depth(P, F) : 0;
+	if (!depth && P.v_shared) depth = float_cin_depth(P, F);
 	for (int c = 0; c < (depth ? 1 : C); c++) {
 		const DevIChan &ic = P.ic[c];
 		const DevWeights &dv = ic.v;
@@ -1104,25 +1303,12 @@ __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned cha
 			}
 			wd[t] = w;
 		}
-		__syncthreads();
 		if (depth) {
 			// Channel 0's weights are every channel's.
-			const size_t cs = (size_t)R * W;
-			const int x0 = threadIdx.x, xs = blockDim.x;
-			if (depth == 32) {
-				if (F.lean) band_vertical_direct<R, 32, true>(P, F, j0, rows, wd, inter, cs, x0, xs);
-				else band_vertical_direct<R, 32, false>(P, F, j0, rows, wd, inter, cs, x0, xs);
-			} else if (depth == 8) {
-				if (F.lean) band_vertical_direct<R, 8, true>(P, F, j0, rows, wd, inter, cs, x0, xs);
-				else band_vertical_direct<R, 8, false>(P, F, j0, rows, wd, inter, cs, x0, xs);
-			} else if (depth == 64) {
-				band_vertical_direct<R, 64, true>(P, F, j0, rows, wd, inter, cs, x0, xs);
-			} else {
-				if (F.lean) band_vertical_direct<R, 16, true>(P, F, j0, rows, wd, inter, cs, x0, xs);
-				else band_vertical_direct<R, 16, false>(P, F, j0, rows, wd, inter, cs, x0, xs);
-			}
+			band_vertical_direct<R, true>(depth, F, P, j0, rows, wd, inter, (size_t)R * W, tid, blockDim.x, tab);
 			continue;
 		}
+		__syncthreads();
 		for (int x = tid; x < W; x += blockDim.x) {
 			double acc[R];
 #pragma unroll
@@ -1259,6 +1445,7 @@ template <int R>
 __global__ void __launch_bounds__(256) vband_kernel(DevPlan P)
 {
 	__shared__ double wd[R * BAND_MAX_K];
+	__shared__ double tab[CIN_LDS / sizeof(double)];
 	const int j0 = blockIdx.y * R;
 	const int rows = min(R, P.Hp - j0);
 	const DevWeights &dv = P.ic[0].v;
@@ -1279,25 +1466,10 @@ __global__ void __launch_bounds__(256) vband_kernel(DevPlan P)
 		}
 		wd[t] = w;
 	}
-	__syncthreads();
 	FastCin F;
 	const int depth = fast_cin_depth(P, F);
-	fast_cin_tables_only(F);
-	const int x0 = blockIdx.x * blockDim.x + threadIdx.x, xs = gridDim.x * blockDim.x;
-	float *out = P.inter + (size_t)j0 * P.W;
-	const size_t cs = (size_t)P.Hp * P.W;
-	if (depth == 32) {
-		if (F.lean) band_vertical_direct<R, 32, true>(P, F, j0, rows, wd, out, cs, x0, xs);
-		else band_vertical_direct<R, 32, false>(P, F, j0, rows, wd, out, cs, x0, xs);
-	} else if (depth == 8) {
-		if (F.lean) band_vertical_direct<R, 8, true>(P, F, j0, rows, wd, out, cs, x0, xs);
-		else band_vertical_direct<R, 8, false>(P, F, j0, rows, wd, out, cs, x0, xs);
-	} else if (depth == 64) {
-		band_vertical_direct<R, 64, true>(P, F, j0, rows, wd, out, cs, x0, xs);
-	} else {
-		if (F.lean) band_vertical_direct<R, 16, true>(P, F, j0, rows, wd, out, cs, x0, xs);
-		else band_vertical_direct<R, 16, false>(P, F, j0, rows, wd, out, cs, x0, xs);
-	}
+	band_vertical_direct<R, false>(depth, F, P, j0, rows, wd, P.inter + (size_t)j0 * P.W, (size_t)P.Hp * P.W,
+		blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, tab);
 }
 
 // Queue the two-pass form's vertical pass of a plan: vband_kernel<vband_r>
@@ -3730,16 +3902,11 @@ struct Staged {
 	std::vector<uint8_t> pack;  // their host image, sent in one copy (lives until the stream syncs)
 };
 
-size_t band_lds_bytes(int R, int C, int W)
-{
-	return sizeof(double) * (size_t)R * BAND_MAX_K + sizeof(float) * (size_t)C * R * W;
-}
-
 // Whether bands of R output rows fit the band kernel: LDS for the rows and
 // input spans of at most BAND_MAX_K positions.
 bool band_fits(const iwamd_plan &p, const Staged &S, int R)
 {
-	if (band_lds_bytes(R, p.inter_nch, p.inter_width) > rt().band_lds_max) return false;
+	if (band_lds_rows(R, p.inter_nch, p.inter_width) > rt().band_lds_max) return false;
 	for (const Staged::List &l : S.lists[IW_DIMENSION_V]) {
 		const iwx::DenseWeights &d = l.d;
 		for (int j0 = 0; j0 < p.inter_height; j0 += R) {
@@ -4237,6 +4404,7 @@ void fill_dev_plan(const Staged &S, const iwamd_plan &p, char *base, DevPlan &D)
 	}
 	D.W = p.inter_width;
 	D.Hp = p.inter_height;
+	D.band_lds_max = (int)rt().band_lds_max;
 	D.v_shared = p.inter_nch > 0 && one_list(S, IW_DIMENSION_V) && S.wv(0).mode == iwx::WeightList::WEIGHTS;
 	D.h_shared = p.inter_nch > 0 && one_list(S, IW_DIMENSION_H) && S.wh(0).mode == iwx::WeightList::WEIGHTS;
 	for (int c = 0; c < p.inter_nch; c++) {
@@ -4466,7 +4634,9 @@ int ws_add(WorkSet &W, const Staged &S, const iwamd_plan &p)
 		}
 	} else if (S.band_rows) {
 		const int ri = S.band_rows == 4 ? 2 : (S.band_rows == 2 ? 1 : 0);
-		const size_t lds = band_lds_bytes(S.band_rows, p.inter_nch, p.inter_width);
+		const bool tab = band_has_tab(S.in_int && p.in_bit_depth == 8, S.band_rows, p.inter_nch, p.inter_width,
+			rt().band_lds_max);
+		const size_t lds = band_lds_rows(S.band_rows, p.inter_nch, p.inter_width) + (tab ? CIN_LDS : 0);
 		const int q = lds_class(lds);
 		for (int j0 = 0; j0 < p.inter_height; j0 += S.band_rows) W.bands[ri][q].push_back(make_int2(jx, j0));
 		W.band_lds[ri][q] = std::max(W.band_lds[ri][q], lds);
