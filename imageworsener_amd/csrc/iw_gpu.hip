@@ -140,6 +140,7 @@ struct DevPlan {
 	int apply_bkgd, late, checker, check_size, ox, oy, bk_has_trans;
 	int v_shared;  // every channel has the same vertical weights (dense form) in WEIGHTS mode
 	int band_lds_max;  // fused form: LDS a workgroup may use
+	int band_group;    // fused form: a row's sum visits the positions of its group of so many rows
 	int vband_r;   // two-pass form: output rows per thread of vband_kernel (0: vpass_kernel)
 	int h_shared;  // the same for the horizontal weights
 	double bk1a, bk2a;
@@ -1142,6 +1143,20 @@ __device__ __forceinline__ void band_fetch(const DevPlan &P, const FastCin &F, l
 	}
 }
 
+// The input positions [p_lo, p_lo + K) that rows [a, b) list.
+__device__ __forceinline__ void band_span(const DevWeights &dv, int a, int b, int &p_lo, int &K)
+{
+	int lo = 0x7fffffff, hi = -0x7fffffff;
+	for (int r = a; r < b; r++) {
+		const int n = dv.dcount[r];
+		if (n == 0) continue;
+		lo = min(lo, dv.dfirst[r]);
+		hi = max(hi, dv.dfirst[r] + n - 1);
+	}
+	p_lo = lo;
+	K = hi >= lo ? hi - lo + 1 : 0;
+}
+
 // The band's vertical pass when every channel shares one weight list
 // (DevPlan::v_shared) and the input takes the direct colour-in: each column's
 // pixels are read once for all channels, four input rows at a time with every
@@ -1157,20 +1172,11 @@ __device__ __forceinline__ void band_fetch(const DevPlan &P, const FastCin &F, l
 // Columns x0, x0 + xstep, ... below W; row r of channel c of column x goes to
 // out[c * cstride + r * W + x].
 template <int R, int DEPTH, int NC, bool LIN, bool LDS>
-__device__ __forceinline__ void band_vertical(const DevPlan &P, const FastCin &F, int j0, int rows,
+__device__ __forceinline__ void band_vertical(const DevPlan &P, const FastCin &F, int p_lo, int K, int rows,
 	const double *wd, float *out, size_t cstride, int x0, int xstep, const double *lds)
 {
 	constexpr int NV = NC ? NC : IWAMD_MAX_CH;
 	const int W = P.W, C = NC ? NC : P.inter_nch;
-	const DevWeights &dv = P.ic[0].v;
-	int p_lo = 0x7fffffff, p_hi = -0x7fffffff;
-	for (int r = 0; r < rows; r++) {
-		const int n = dv.dcount[j0 + r];
-		if (n == 0) continue;
-		p_lo = min(p_lo, dv.dfirst[j0 + r]);
-		p_hi = max(p_hi, dv.dfirst[j0 + r] + n - 1);
-	}
-	const int K = (p_hi >= p_lo) ? p_hi - p_lo + 1 : 0;
 	for (int x = x0; x < W; x += xstep) {
 		const long long cb = F.base + (long long)x * F.dx;
 		double acc[NV][R];
@@ -1214,7 +1220,7 @@ __device__ __forceinline__ void band_vertical(const DevPlan &P, const FastCin &F
 // band_vertical of a direct colour-in (depth != 0).  tab: room for the 8-bit
 // tables (CIN_LDS bytes, written here; ends with a barrier), or null.
 template <int R, bool FLOAT>
-__device__ __forceinline__ void band_vertical_direct(int depth, FastCin &F, const DevPlan &P, int j0, int rows,
+__device__ __forceinline__ void band_vertical_direct(int depth, FastCin &F, const DevPlan &P, int p_lo, int K, int rows,
 	const double *wd, float *out, size_t cs, int x0, int xs, double *tab)
 {
 	const bool lds = (depth == 8 || depth == 32) && tab && fast_cin_slots(F, tab);
@@ -1222,36 +1228,36 @@ __device__ __forceinline__ void band_vertical_direct(int depth, FastCin &F, cons
 	int nc = fast_cin_channels(F, P.inter_nch);
 	if (depth == 8 || depth == 32) {
 		if (!lds) {
-			if (depth == 32) band_vertical<R, 32, 0, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
-			else band_vertical<R, 8, 0, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+			if (depth == 32) band_vertical<R, 32, 0, false, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
+			else band_vertical<R, 8, 0, false, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
 		} else if (depth == 32) {
-			if (nc == 4) band_vertical<R, 32, 4, false, true>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
-			else band_vertical<R, 32, 0, false, true>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+			if (nc == 4) band_vertical<R, 32, 4, false, true>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
+			else band_vertical<R, 32, 0, false, true>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
 		} else {
-			if (nc == 3) band_vertical<R, 8, 3, false, true>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
-			else if (nc == 1) band_vertical<R, 8, 1, false, true>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
-			else band_vertical<R, 8, 0, false, true>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+			if (nc == 3) band_vertical<R, 8, 3, false, true>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
+			else if (nc == 1) band_vertical<R, 8, 1, false, true>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
+			else band_vertical<R, 8, 0, false, true>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
 		}
 		return;
 	}
 	if (FLOAT && depth == 33) {
-		if (nc == 4) band_vertical<R, 33, 4, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
-		else if (nc == 3) band_vertical<R, 33, 3, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
-		else band_vertical<R, 33, 0, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+		if (nc == 4) band_vertical<R, 33, 4, false, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
+		else if (nc == 3) band_vertical<R, 33, 3, false, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
+		else band_vertical<R, 33, 0, false, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
 		return;
 	}
 	const bool lin = F.lmax[0] == 65535.0 && F.lmax[1] == 65535.0 && F.lmax[2] == 65535.0 && F.lmax[3] == 65535.0;
 	if (depth == 64 && nc == 4) {
-		if (lin) band_vertical<R, 64, 4, true, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
-		else band_vertical<R, 64, 4, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+		if (lin) band_vertical<R, 64, 4, true, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
+		else band_vertical<R, 64, 4, false, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
 	} else if (depth == 16 && nc == 3) {
-		if (lin) band_vertical<R, 16, 3, true, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
-		else band_vertical<R, 16, 3, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+		if (lin) band_vertical<R, 16, 3, true, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
+		else band_vertical<R, 16, 3, false, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
 	} else if (depth == 16 && nc == 1) {
-		if (lin) band_vertical<R, 16, 1, true, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
-		else band_vertical<R, 16, 1, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+		if (lin) band_vertical<R, 16, 1, true, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
+		else band_vertical<R, 16, 1, false, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
 	} else {
-		band_vertical<R, 16, 0, false, false>(P, F, j0, rows, wd, out, cs, x0, xs, tab);
+		band_vertical<R, 16, 0, false, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, tab);
 	}
 }
 
@@ -1284,15 +1290,10 @@ __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned cha
 	for (int c = 0; c < (depth ? 1 : C); c++) {
 		const DevIChan &ic = P.ic[c];
 		const DevWeights &dv = ic.v;
-		// The band's input positions.
-		int p_lo = 0x7fffffff, p_hi = -0x7fffffff;
-		for (int r = 0; r < rows; r++) {
-			const int n = dv.dcount[j0 + r];
-			if (n == 0) continue;
-			p_lo = min(p_lo, dv.dfirst[j0 + r]);
-			p_hi = max(p_hi, dv.dfirst[j0 + r] + n - 1);
-		}
-		const int K = (p_hi >= p_lo) ? p_hi - p_lo + 1 : 0;
+		// The group's input positions.
+		const int g0 = j0 - j0 % P.band_group, g1 = min(g0 + P.band_group, P.Hp);
+		int p_lo, K;
+		band_span(dv, g0, g1, p_lo, K);
 		__syncthreads();  // previous channel's weights no longer read
 		for (int t = tid; t < R * BAND_MAX_K; t += blockDim.x) {
 			const int r = t / BAND_MAX_K, k = t % BAND_MAX_K;
@@ -1305,7 +1306,7 @@ __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned cha
 		}
 		if (depth) {
 			// Channel 0's weights are every channel's.
-			band_vertical_direct<R, true>(depth, F, P, j0, rows, wd, inter, (size_t)R * W, tid, blockDim.x, tab);
+			band_vertical_direct<R, true>(depth, F, P, p_lo, K, rows, wd, inter, (size_t)R * W, tid, blockDim.x, tab);
 			continue;
 		}
 		__syncthreads();
@@ -1449,14 +1450,8 @@ __global__ void __launch_bounds__(256) vband_kernel(DevPlan P)
 	const int j0 = blockIdx.y * R;
 	const int rows = min(R, P.Hp - j0);
 	const DevWeights &dv = P.ic[0].v;
-	int p_lo = 0x7fffffff, p_hi = -0x7fffffff;
-	for (int r = 0; r < rows; r++) {
-		const int n = dv.dcount[j0 + r];
-		if (n == 0) continue;
-		p_lo = min(p_lo, dv.dfirst[j0 + r]);
-		p_hi = max(p_hi, dv.dfirst[j0 + r] + n - 1);
-	}
-	const int K = (p_hi >= p_lo) ? p_hi - p_lo + 1 : 0;
+	int p_lo, K;
+	band_span(dv, j0, j0 + rows, p_lo, K);
 	for (int t = threadIdx.x; t < R * BAND_MAX_K; t += blockDim.x) {
 		const int r = t / BAND_MAX_K, k = t % BAND_MAX_K;
 		double w = 0.0;
@@ -1468,7 +1463,7 @@ __global__ void __launch_bounds__(256) vband_kernel(DevPlan P)
 	}
 	FastCin F;
 	const int depth = fast_cin_depth(P, F);
-	band_vertical_direct<R, false>(depth, F, P, j0, rows, wd, P.inter + (size_t)j0 * P.W, (size_t)P.Hp * P.W,
+	band_vertical_direct<R, false>(depth, F, P, p_lo, K, rows, wd, P.inter + (size_t)j0 * P.W, (size_t)P.Hp * P.W,
 		blockIdx.x * blockDim.x + threadIdx.x, gridDim.x * blockDim.x, tab);
 }
 
@@ -3887,6 +3882,7 @@ struct Staged {
 	size_t in_f64_bpr = 0;
 	bool skip_pixels = false;  // unknown filter: the reference reports and outputs zeros
 	int band_rows = 0;         // rows per band of the fused kernel; 0: two-pass kernels
+	int band_group = 0;        // band_rows before band_rows_alone (0: the same)
 	int fast_ti = 0;           // output columns per chosen-precision tile
 	std::vector<int4> h4i;     // chosen form: the horizontal list by 4-column blocks (DevPlan::h4i)
 	std::vector<float> h4w;
@@ -4234,7 +4230,7 @@ bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path
 			o.copy = L.add<int>(l.wl.copy_src.size());
 			o.dfirst = L.add<int>(l.d.first.size());
 			o.dcount = L.add<int>(l.d.count.size());
-			o.doff = L.add<int>(l.d.off.size());
+			o.doff = L.add<int>(dim == IW_DIMENSION_V ? l.d.off.size() : 0);
 			o.dw = L.add<double>(dim == IW_DIMENSION_H ? (size_t)l.d.max_count * l.d.first.size() : l.d.w.size());
 			S.o_list[dim].push_back(o);
 		}
@@ -4307,8 +4303,8 @@ bool upload_job(Staged &S, const iwamd_plan &p, char *base, hipStream_t st, cons
 			up(o.copy, wl.copy_src.data(), wl.copy_src.size() * 4);
 			up(o.dfirst, d.first.data(), d.first.size() * 4);
 			up(o.dcount, d.count.data(), d.count.size() * 4);
-			up(o.doff, d.off.data(), d.off.size() * 4);
 			if (dim == IW_DIMENSION_V) {
+				up(o.doff, d.off.data(), d.off.size() * 4);
 				up(o.dw, d.w.data(), d.w.size() * 8);
 			} else {
 				double *t = (double *)(S.pack.data() + (o.dw - t0));
@@ -4405,6 +4401,7 @@ void fill_dev_plan(const Staged &S, const iwamd_plan &p, char *base, DevPlan &D)
 	D.W = p.inter_width;
 	D.Hp = p.inter_height;
 	D.band_lds_max = (int)rt().band_lds_max;
+	D.band_group = S.in_int || !S.band_group ? std::max(1, S.band_rows) : S.band_group;
 	D.v_shared = p.inter_nch > 0 && one_list(S, IW_DIMENSION_V) && S.wv(0).mode == iwx::WeightList::WEIGHTS;
 	D.h_shared = p.inter_nch > 0 && one_list(S, IW_DIMENSION_H) && S.wh(0).mode == iwx::WeightList::WEIGHTS;
 	for (int c = 0; c < p.inter_nch; c++) {
@@ -4992,6 +4989,23 @@ bool tune_enabled()
 	return !(v && v[0] == '0');
 }
 
+// A job that runs alone has only its own bands to fill the device: bands of
+// fewer rows, down to one, until there are two for each of the 256 CUs.  A
+// workgroup's chain of loads and sums gets shorter, for more input read twice.
+// 240 rows (640x480 to 320x240, RGB): 52.4 us in bands of 4, 28.9 of 1; 600
+// (RGB floats): 51.6, 25.4; at 1300 and 1536 rows bands of 2 are the best
+// (rgba 100.8 / 99.6 / 109 for 4 / 2 / 1, grey with diffusion 76 / 59 / 73).
+// The positions a row's sum visits stay those of the taller band: where
+// floating-point samples are not finite, a position of weight 0 counts.
+#define BANDS_ALONE 512
+
+void band_rows_alone(const iwamd_plan &p, Staged &S)
+{
+	if (S.shape_forced || !S.band_rows || !S.fast.empty()) return;
+	S.band_group = S.band_rows;
+	while (S.band_rows > 1 && (p.inter_height + S.band_rows - 1) / S.band_rows < BANDS_ALONE) S.band_rows /= 2;
+}
+
 // Gives the plan its class's tuned shape; a class without one is measured on
 // this job first when may_tune.  A shape that does not fit this job (or a
 // failed measurement) keeps the default choice.
@@ -5039,6 +5053,7 @@ bool job_upload(iwamd_job *J, bool wait)
 		const char *t = iw_get_option(ctx, "amd:tune");
 		tune_apply(p, S, J->stream, t && atoi(t) == 1);
 	}
+	band_rows_alone(p, S);
 	J->skip_pixels = S.skip_pixels;
 	J->n_ed = S.n_ed;
 	for (int e = 0; e < 4; e++) J->ed_list[e] = S.ed_list[e];
@@ -5454,9 +5469,18 @@ extern "C" int iwamd_process_device_noalloc(struct iw_context *ctx, const void *
 	Staged S;
 	if (!stage_job(ctx, p, S, iw_get_option(ctx, "amd:resample"), true, true)) return 0;
 	tune_apply(p, S, st, false);  // look the shape up; never tunes (tuning allocates)
+	const int tall = S.band_rows;
+	band_rows_alone(p, S);
 	WorkSet W;
 	ws_add(W, S, p);
 	ws_layout(W);
+	if (S.bytes + W.bytes > IWAMD_NOALLOC_SCRATCH && S.band_rows != tall) {
+		// The shorter bands' work list does not fit: the taller ones'.
+		S.band_rows = tall;
+		W = WorkSet();
+		ws_add(W, S, p);
+		ws_layout(W);
+	}
 	const size_t need = S.bytes + W.bytes;
 	if (need > IWAMD_NOALLOC_SCRATCH) {
 		iw_set_errorf(ctx, "This job needs %zu bytes of device scratch; iwamd_process_device_noalloc has %zu",
