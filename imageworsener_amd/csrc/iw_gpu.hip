@@ -744,7 +744,24 @@ __device__ __forceinline__ void emit_pixel(const DevPlan &P, int i, int j, Gathe
 // last weigh 0 (stored as -0.0), which leaves a sum's bits unchanged for
 // finite samples.  SKIP: samples may not be finite, so those are left out.
 // load(c, r, x): sample x of intermediate row r.  Then the rows' pixels one by
-// one.
+// one.  InterRows: columns whose list lies inside the row read four samples at
+// a time, so that a cache line is asked for once per four taps.
+struct InterRows {
+	const float *p;
+	size_t cstride, rstride;
+	int last;  // the last row
+	typedef float v4 __attribute__((ext_vector_type(4), aligned(4)));
+	__device__ __forceinline__ const g_cf32 *at(int c, int r, int x) const
+	{
+		return (const g_cf32 *)p + c * cstride + min(r, last) * rstride + x;
+	}
+	__device__ __forceinline__ float operator()(int c, int r, int x) const { return *at(c, r, x); }
+	__device__ __forceinline__ v4 four(int c, int r, int x) const
+	{
+		return *(const __attribute__((address_space(1))) v4 *)at(c, r, x);
+	}
+};
+
 template <int RR, bool SKIP, class Emit, class Load>
 __device__ __forceinline__ void hrows(const DevPlan &P, const Emit &E, int i, int j0, int n, Load load)
 {
@@ -757,7 +774,28 @@ __device__ __forceinline__ void hrows(const DevPlan &P, const Emit &E, int i, in
 	for (int r = 0; r < RR; r++)
 #pragma unroll
 		for (int c = 0; c < IWAMD_MAX_CH; c++) acc[r][c] = 0.0;
-	for (int u = 0; u < cnt; u++) {
+	int u = 0;
+	if constexpr (std::is_same<Load, InterRows>::value) {
+		if (f0 >= 0 && f0 + cnt <= W) {
+			for (; u + 4 <= cnt; u += 4) {
+				double w[4];
+#pragma unroll
+				for (int t = 0; t < 4; t++) w[t] = hw[(size_t)(u + t) * ow];
+#pragma unroll
+				for (int c = 0; c < IWAMD_MAX_CH; c++) {
+					if (c >= C) break;
+					InterRows::v4 v[RR];
+#pragma unroll
+					for (int r = 0; r < RR; r++) v[r] = load.four(c, r, f0 + u);
+#pragma unroll
+					for (int t = 0; t < 4; t++)
+#pragma unroll
+						for (int r = 0; r < RR; r++) acc[r][c] = acc[r][c] + (double)v[r][t] * w[t];
+				}
+			}
+		}
+	}
+	for (; u < cnt; u++) {
 		const double w = hw[(size_t)u * ow];
 		const int pos = f0 + u;
 		const bool outside = pos < 0 || pos >= W;
@@ -803,11 +841,13 @@ __global__ void __launch_bounds__(256) hpass_kernel(DevPlan P)
 }
 
 // The two-pass form's horizontal pass where the channels share the list and
-// the per-pixel work is simple: HP_ROWS rows per thread.  Bound by the loads
-// of the intermediate samples (L2) and, per pixel, the dependent table
-// searches; with a pixel per thread and a list read per channel it was bound
-// by the lists.  4000 to 1000 columns, 750 rows, RGB, Lanczos3: 316 -> 119 us;
-// 4096 to 1000, 1000 rows, RGBA, Mitchell: 318 -> 167 us.
+// the per-pixel work is simple: HP_ROWS rows per thread, four taps per load.
+// Bound by the requests for intermediate samples to L2 (with one tap per load
+// each line was asked for by every tap: 119 and 167 us for the sizes below)
+// and, per pixel, the dependent table searches; with a pixel per thread and a
+// list read per channel it was bound by the lists.  4000 to 1000 columns, 750
+// rows, RGB, Lanczos3: 316 -> 35 us; 4096 to 1000, 1000 rows, RGBA, Mitchell:
+// 318 -> 54 us.
 #define HP_ROWS 4
 __global__ void __launch_bounds__(256) hpass_rows_kernel(DevPlan P)
 {
@@ -816,9 +856,8 @@ __global__ void __launch_bounds__(256) hpass_rows_kernel(DevPlan P)
 	if (i >= P.out_w) return;
 	EmitSimple E;
 	emit_simple_ctx(P, E);
-	hrows<HP_ROWS, false>(P, E, i, j0, min(HP_ROWS, P.out_h - j0), [&](int c, int r, int x) {
-		return ((const g_cf32 *)P.inter)[((size_t)c * P.Hp + min(j0 + r, P.out_h - 1)) * P.W + x];
-	});
+	const InterRows rows = {P.inter + (size_t)j0 * P.W, (size_t)P.Hp * P.W, (size_t)P.W, P.out_h - 1 - j0};
+	hrows<HP_ROWS, false>(P, E, i, j0, min(HP_ROWS, P.out_h - j0), rows);
 }
 
 // Queue the two-pass form's horizontal pass.  (Floating-point samples may not
