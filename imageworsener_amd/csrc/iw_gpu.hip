@@ -737,15 +737,7 @@ __device__ __forceinline__ void emit_pixel(const DevPlan &P, int i, int j, Gathe
 	emit_px(E, i, j, gather);
 }
 
-// The horizontal pass and per-pixel work of column i of RR output rows from
-// j0 on, n of which exist, for plans whose channels share the horizontal list
-// (DevPlan::h_shared).  A tap's weight and position are read once for all
-// rows and channels; positions the list does not hold between its first and
-// last weigh 0 (stored as -0.0), which leaves a sum's bits unchanged for
-// finite samples.  SKIP: samples may not be finite, so those are left out.
-// load(c, r, x): sample x of intermediate row r.  Then the rows' pixels one by
-// one.  InterRows: columns whose list lies inside the row read four samples at
-// a time, so that a cache line is asked for once per four taps.
+// Rows of the intermediate image.
 struct InterRows {
 	const float *p;
 	size_t cstride, rstride;
@@ -762,6 +754,32 @@ struct InterRows {
 	}
 };
 
+// The same for a band's rows in LDS.
+struct BandRows {
+	const float *p;
+	int cstride, rstride, last;
+	typedef InterRows::v4 v4;
+	__device__ __forceinline__ float operator()(int c, int r, int x) const
+	{
+		return p[c * cstride + min(r, last) * rstride + x];
+	}
+	__device__ __forceinline__ v4 four(int c, int r, int x) const
+	{
+		return *(const v4 *)(p + (c * cstride + min(r, last) * rstride + x));
+	}
+};
+
+// The horizontal pass and per-pixel work of column i of RR output rows from
+// j0 on, n of which exist, for plans whose channels share the horizontal list
+// (DevPlan::h_shared).  A tap's weight and position are read once for all
+// rows and channels; positions the list does not hold between its first and
+// last weigh 0 (stored as -0.0), which leaves a sum's bits unchanged for
+// finite samples.  SKIP: samples may not be finite, so those are left out (and
+// the taps summed one by one: the sign of a sum of two NaNs depends on the
+// order of the operands in the machine code).
+// load(c, r, x): sample x of intermediate row r.  Columns whose list lies
+// inside the row read four samples at a time (load.four), so that a cache line
+// is asked for once per four taps.  Then the rows' pixels one by one.
 template <int RR, bool SKIP, class Emit, class Load>
 __device__ __forceinline__ void hrows(const DevPlan &P, const Emit &E, int i, int j0, int n, Load load)
 {
@@ -775,22 +793,21 @@ __device__ __forceinline__ void hrows(const DevPlan &P, const Emit &E, int i, in
 #pragma unroll
 		for (int c = 0; c < IWAMD_MAX_CH; c++) acc[r][c] = 0.0;
 	int u = 0;
-	if constexpr (std::is_same<Load, InterRows>::value) {
-		if (f0 >= 0 && f0 + cnt <= W) {
-			for (; u + 4 <= cnt; u += 4) {
-				double w[4];
+	if (!SKIP && f0 >= 0 && f0 + cnt <= W) {
+		for (; u + 4 <= cnt; u += 4) {
+			double w[4];
 #pragma unroll
-				for (int t = 0; t < 4; t++) w[t] = hw[(size_t)(u + t) * ow];
+			for (int t = 0; t < 4; t++) w[t] = hw[(size_t)(u + t) * ow];
 #pragma unroll
-				for (int c = 0; c < IWAMD_MAX_CH; c++) {
-					if (c >= C) break;
-					InterRows::v4 v[RR];
+			for (int c = 0; c < IWAMD_MAX_CH; c++) {
+				if (c >= C) break;
+				typename Load::v4 v[RR];
 #pragma unroll
-					for (int r = 0; r < RR; r++) v[r] = load.four(c, r, f0 + u);
+				for (int r = 0; r < RR; r++) v[r] = load.four(c, r, f0 + u);
 #pragma unroll
-					for (int t = 0; t < 4; t++)
+				for (int t = 0; t < 4; t++) {
 #pragma unroll
-						for (int r = 0; r < RR; r++) acc[r][c] = acc[r][c] + (double)v[r][t] * w[t];
+					for (int r = 0; r < RR; r++) acc[r][c] = acc[r][c] + (double)v[r][t] * w[t];
 				}
 			}
 		}
@@ -1396,9 +1413,11 @@ __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned cha
 	// With a shared list a thread takes one column of several of the band's
 	// rows, so that a weight is read once for them: all the rows where the
 	// columns fill the threads, fewer where that leaves less to do per thread
-	// (per column its rows and about one row's worth of weights).  3072 to 3072
-	// columns of grey, ordered dither: 530 -> 421 us; 1000 to 300, RGB over a
-	// background: 126 -> 90 us; 1000 to 1900, RGBA: 115 -> 106 us.
+	// (per column its rows and about one row's worth of weights), and
+	// four taps per LDS read.  2048 to 3072 columns of grey, ordered dither: the
+	// columns 530 -> 421 us, the reads 334 -> 295 us; 1000 to 300, RGB over a
+	// background: 126 -> 90 and 51 -> 41 us; 1000 to 1900, RGBA: 115 -> 106 and
+	// 100 -> 90 us.
 	// (The generic per-pixel work goes row by row: it is too large to repeat,
 	// and meets floating-point input, whose samples may not be finite.)
 	auto columns = [&](const auto &E) {
@@ -1409,15 +1428,18 @@ __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned cha
 		if (R >= 4 && cost(4) < cost(groups)) groups = 4;
 		const int cols = 256 / groups, per = R / groups, r0 = tid / cols * per, n = min(per, rows - r0);
 		if (n <= 0) return;
-		auto load = [&](int c, int r, int x) { return inter[((size_t)c * R + r0 + min(r, n - 1)) * W + x]; };
+		const BandRows load = {inter + r0 * W, R * W, W, n - 1};  // the thread's rows
 		for (int i = tid % cols; i < P.out_w; i += cols) {
 			if constexpr (SIMPLE) {
 				if (per == 1) hrows<1, false>(P, E, i, j0 + r0, n, load);
 				else if (per == 2) hrows<(R < 2 ? 1 : 2), false>(P, E, i, j0 + r0, n, load);
 				else hrows<R, false>(P, E, i, j0 + r0, n, load);
 			} else {
-				for (int q = 0; q < n; q++)
-					hrows<1, true>(P, E, i, j0 + r0 + q, 1, [&](int c, int, int x) { return load(c, q, x); });
+				for (int q = 0; q < n; q++) {
+					const BandRows row = {load.p + q * W, load.cstride, W, 0};
+					if (P.in_float) hrows<1, true>(P, E, i, j0 + r0 + q, 1, row);
+					else hrows<1, false>(P, E, i, j0 + r0 + q, 1, row);
+				}
 			}
 		}
 	};
