@@ -11,8 +11,8 @@
 //                   and hand their linear samples on.
 //   vpass/hpass  -- the same work as two kernels with the intermediate in HBM,
 //                   for rows too wide for a band in LDS.
-//   fast_kernel  -- the chosen-precision form: both resamples as FP16 MFMA
-//                   band products with FP32 sums, the per-pixel work in FP64.
+//   fast_kernel  -- the chosen-precision form: both resamples as FP32 MFMA
+//                   band products, the per-pixel work in FP64.
 //   errdiff      -- one workgroup per error-diffused plane walking the
 //                   reference's serpentine order (src/imagew-main.c:497-567,
 //                   1072-1136): errdiff_rows_kernel with the rows in registers
@@ -1218,7 +1218,8 @@ __device__ __forceinline__ void band_span(const DevWeights &dv, int a, int b, in
 // pixels are read once for all channels, four input rows at a time with every
 // load issued before the first is used.  Each accumulator still gets its terms
 // in list order, with the same FP64 operations as colour_in and the generic
-// pass.  NC: fast_cin_channels (0: any plan, through fast_fetch).
+// pass.  NC: fast_cin_channels (0: any plan, through fast_fetch; LIN is its LEAN
+// then).
 // Bound by the table gathers, then the FP64 sums: with the tables in LDS and
 // only the plan's own channels looked up (five gathers per pixel before,
 // whatever the channels), 4000x3000 RGB to 750 rows: 159 -> 88 us; 16-bit
@@ -1246,7 +1247,7 @@ __device__ __forceinline__ void band_vertical(const DevPlan &P, const FastCin &F
 			for (int t = 0; t < 4; t++) {
 				const int p = p_lo + min(k + t, K - 1);
 				if constexpr (NC) band_fetch<DEPTH, NC, LIN>(P, F, cb, p, v[t], lds);
-				else fast_fetch<DEPTH, false, double, LDS>(P, F, cb, p, v[t], lds);
+				else fast_fetch<DEPTH, LIN, double, LDS>(P, F, cb, p, v[t], lds);
 			}
 #pragma unroll
 			for (int t = 0; t < 4; t++) {
@@ -1329,11 +1330,33 @@ __host__ __device__ inline bool band_has_tab(bool in8, int R, int C, int W, size
 	return in8 && band_lds_rows(R, C, W) + CIN_LDS <= lds_max;
 }
 
+// The same for bands of a batch, which fill the chip: the tables stay in
+// memory.  In LDS they cost more than the gathers, which the other waves hide
+// (4096 small RGBA images: 45.1 -> 42.7 ms without them).
 template <int R>
+__device__ __forceinline__ void band_vertical_batch(int depth, const FastCin &F, const DevPlan &P, int p_lo, int K,
+	int rows, const double *wd, float *out, size_t cs, int x0, int xs)
+{
+	if (depth == 32) {
+		if (F.lean) band_vertical<R, 32, 0, true, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, nullptr);
+		else band_vertical<R, 32, 0, false, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, nullptr);
+	} else if (depth == 8) {
+		if (F.lean) band_vertical<R, 8, 0, true, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, nullptr);
+		else band_vertical<R, 8, 0, false, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, nullptr);
+	} else if (depth == 64) {
+		band_vertical<R, 64, 0, true, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, nullptr);
+	} else {
+		if (F.lean) band_vertical<R, 16, 0, true, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, nullptr);
+		else band_vertical<R, 16, 0, false, false>(P, F, p_lo, K, rows, wd, out, cs, x0, xs, nullptr);
+	}
+}
+
+// ALONE: the band of a job that runs by itself, else of a batch or a flight.
+template <int R, bool ALONE>
 __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned char *band_lds)
 {
 	double *wd = (double *)band_lds;                       // [R][BAND_MAX_K]
-	double *tab = band_has_tab(P.bit_depth == 8 && !P.in_float, R, P.inter_nch, P.W, P.band_lds_max) ? wd + R * BAND_MAX_K : nullptr;  // [2][256]
+	double *tab = ALONE && band_has_tab(P.bit_depth == 8 && !P.in_float, R, P.inter_nch, P.W, P.band_lds_max) ? wd + R * BAND_MAX_K : nullptr;  // [2][256]
 	float *inter = (float *)(wd + R * BAND_MAX_K + (tab ? CIN_LDS / sizeof(double) : 0));  // [C][R][W]
 	const int tid = threadIdx.x;
 	const int rows = min(R, P.Hp - j0);
@@ -1342,7 +1365,7 @@ __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned cha
 
 	FastCin F;
 	int depth = P.v_shared ? fast_cin_depth(P, F) : 0;
-	if (!depth && P.v_shared) depth = float_cin_depth(P, F);
+	if (ALONE && !depth && P.v_shared) depth = float_cin_depth(P, F);
 	for (int c = 0; c < (depth ? 1 : C); c++) {
 		const DevIChan &ic = P.ic[c];
 		const DevWeights &dv = ic.v;
@@ -1362,7 +1385,12 @@ __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned cha
 		}
 		if (depth) {
 			// Channel 0's weights are every channel's.
-			band_vertical_direct<R, true>(depth, F, P, p_lo, K, rows, wd, inter, (size_t)R * W, tid, blockDim.x, tab);
+			if constexpr (ALONE) {
+				band_vertical_direct<R, true>(depth, F, P, p_lo, K, rows, wd, inter, (size_t)R * W, tid, blockDim.x, tab);
+			} else {
+				__syncthreads();
+				band_vertical_batch<R>(depth, F, P, p_lo, K, rows, wd, inter, (size_t)R * W, tid, blockDim.x);
+			}
 			continue;
 		}
 		__syncthreads();
@@ -1446,7 +1474,17 @@ __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned cha
 	EmitSimple ES;
 	if (emit_simple_ctx(P, ES)) {
 		if (P.h_shared) {
-			columns(ES);
+			if constexpr (ALONE) {
+				columns(ES);
+			} else {
+				// Every thread the same number of pixels (44.4 against 45.1 ms by
+				// columns for the batch above).
+				for (int t = tid; t < n_px; t += blockDim.x) {
+					const int r = t / P.out_w, i = t % P.out_w;
+					const BandRows row = {inter + r * W, R * W, W, 0};
+					hrows<1, false>(P, ES, i, j0 + r, 1, row);
+				}
+			}
 			return;
 		}
 		for (int t = tid; t < n_px; t += blockDim.x) {
@@ -1477,7 +1515,7 @@ __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned cha
 // gridDim.x + atomicAdd(counter, 1) until none is left -- a persistent
 // kernel over a whole batch.  (The band lists keep this one queue: with the
 // chosen form's per-XCD chunks the C3 batch's plain form ran 41.1 -> 45.3 ms.)
-template <int R>
+template <int R, bool ALONE>
 __global__ void __launch_bounds__(256) band_kernel(const DevPlan *__restrict__ plans,
 	const int2 *__restrict__ items, int n_items, int *counter)
 {
@@ -1486,7 +1524,7 @@ __global__ void __launch_bounds__(256) band_kernel(const DevPlan *__restrict__ p
 	int it = blockIdx.x;
 	while (it < n_items) {
 		const int2 w = items[it];
-		band_body<R>(plans[w.x], w.y, band_lds);
+		band_body<R, ALONE>(plans[w.x], w.y, band_lds);
 		if (!counter) break;
 		__syncthreads();  // LDS of this item is no longer read
 		if (threadIdx.x == 0) next_item = (int)gridDim.x + atomicAdd(counter, 1);
@@ -3355,7 +3393,9 @@ bool runtime_init(iw_context *ctx)
 	}
 	// The band kernels size their LDS per launch, up to the workgroup limit
 	// (160 KB on gfx950); where the runtime refuses, they keep 64 KB.
-	const void *bk[3] = {(const void *)band_kernel<1>, (const void *)band_kernel<2>, (const void *)band_kernel<4>};
+	const void *bk[6] = {(const void *)band_kernel<1, false>, (const void *)band_kernel<2, false>,
+		(const void *)band_kernel<4, false>, (const void *)band_kernel<1, true>, (const void *)band_kernel<2, true>,
+		(const void *)band_kernel<4, true>};
 	R.band_lds_max = 160 * 1024;
 	for (const void *f : bk) {
 		if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)R.band_lds_max) != hipSuccess) {
@@ -4631,6 +4671,7 @@ struct WorkSet {
 	std::vector<DevPlan> plans;       // host copies; the two-pass kernels take them by value
 	std::vector<int2> bands[3][kLdsClasses];  // (plan, first row), by band height kBandR and LDS class
 	size_t band_lds[3][kLdsClasses] = {};      // largest LDS of a band in each list
+	size_t band_lds_alone[3][kLdsClasses] = {};  // the same with the tables of a job that runs alone
 	std::vector<int2> planes[kEdVariants];  // (plan, output channel), by ed_variant
 	std::vector<int2> ilv;            // (plan, first row) of the outputs edr_interleave_kernel forms
 	std::vector<int> twopass;         // plans resampled by vpass + hpass
@@ -4699,10 +4740,11 @@ int ws_add(WorkSet &W, const Staged &S, const iwamd_plan &p)
 		const int ri = S.band_rows == 4 ? 2 : (S.band_rows == 2 ? 1 : 0);
 		const bool tab = band_has_tab(S.in_int && p.in_bit_depth == 8, S.band_rows, p.inter_nch, p.inter_width,
 			rt().band_lds_max);
-		const size_t lds = band_lds_rows(S.band_rows, p.inter_nch, p.inter_width) + (tab ? CIN_LDS : 0);
+		const size_t lds = band_lds_rows(S.band_rows, p.inter_nch, p.inter_width);
 		const int q = lds_class(lds);
 		for (int j0 = 0; j0 < p.inter_height; j0 += S.band_rows) W.bands[ri][q].push_back(make_int2(jx, j0));
 		W.band_lds[ri][q] = std::max(W.band_lds[ri][q], lds);
+		W.band_lds_alone[ri][q] = std::max(W.band_lds_alone[ri][q], lds + (tab ? CIN_LDS : 0));
 	} else {
 		W.twopass.push_back(jx);
 	}
@@ -4864,10 +4906,16 @@ void ws_enqueue_resample(const WorkSet &W, hipStream_t st, bool persistent)
 				grid = std::min(n, device_cu_count() * per_cu);
 			}
 			int *ctr = persistent ? W.d_counters + r * kLdsClasses + q : nullptr;
+			auto launch = [&](auto alone, auto batch) {
+				if (persistent)
+					hipLaunchKernelGGL(batch, dim3(grid), dim3(256), lds, st, W.d_plans, items, n, ctr);
+				else
+					hipLaunchKernelGGL(alone, dim3(grid), dim3(256), W.band_lds_alone[r][q], st, W.d_plans, items, n, ctr);
+			};
 			switch (kBandR[r]) {
-			case 1: hipLaunchKernelGGL(band_kernel<1>, dim3(grid), dim3(256), lds, st, W.d_plans, items, n, ctr); break;
-			case 2: hipLaunchKernelGGL(band_kernel<2>, dim3(grid), dim3(256), lds, st, W.d_plans, items, n, ctr); break;
-			default: hipLaunchKernelGGL(band_kernel<4>, dim3(grid), dim3(256), lds, st, W.d_plans, items, n, ctr); break;
+			case 1: launch(band_kernel<1, true>, band_kernel<1, false>); break;
+			case 2: launch(band_kernel<2, true>, band_kernel<2, false>); break;
+			default: launch(band_kernel<4, true>, band_kernel<4, false>); break;
 			}
 		}
 	for (int jx : W.twopass) {
