@@ -2848,11 +2848,14 @@ __global__ void __launch_bounds__(ED_THREADS) errdiff_kernel(const DevPlan *__re
 // has settled when none of its start states changed, bit for bit.  The row's
 // first segment starts from zero in the reference too, so at the fixed point
 // every segment is the true chain, by induction, and each round makes at
-// least one more segment true; two walks' states meet within a few dozen
-// pixels, so the rounds are few.  Waves read their predecessor's end state as
-// it stands when a round begins, without waiting for it.  One barrier ends
-// the row: after it every wave compares all waves' start states with their
-// predecessors' end states, and all of them go on if any differs.
+// least one more segment true (a row walked downwards starts past its end, in
+// pixels whose samples are -1: clamped to 0 and on level 0 from the first
+// lookup on, they hand an error of 0 to the row's last pixel); two walks'
+// states meet within a few dozen pixels, so the rounds are few.  Waves read
+// their predecessor's end state as it stands when a round begins, without
+// waiting for it.  One barrier ends the row: after it every wave compares all
+// waves' start states with their predecessors' end states, and all of them go
+// on if any differs.
 //
 // Decision (as ed_decide): the level is #{D <= s} with the folded boundaries
 // D[k] = min(T[k], max(T[k-1], U[k], M[k])) (QuantTable::D), the error
@@ -2898,7 +2901,7 @@ struct EdrLds {
 	double D[ED_LDS_TABLE + 4];
 	double lin[ED_LDS_TABLE + 2];
 	double lo[ED_LDS_TABLE + 1], hi[ED_LDS_TABLE + 1];  // level k's exact samples: [lo[k], hi[k])
-	unsigned short Q[ED_NB];                 // first guess of b by s * ED_NB
+	unsigned short Q[1 + ED_NB];             // first guess of b: 0 below 0, then by s * ED_NB
 	unsigned short code[ED_LDS_TABLE + 1];   // output code per level
 	unsigned long long eps;                  // bits of the widest distance of an exact sample from its level
 	EdrEdge edge[2][NW];
@@ -2937,12 +2940,12 @@ __device__ __forceinline__ void edr_put(double *p, double v)
 	__hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 }
 
-// Pixel i's boundary for sample s: the index's guess; SETTLE: stepped until
-// s lies in its range.
+// Pixel i's boundary for sample s (before the clamp, or after it): the
+// index's guess; SETTLE: stepped until s lies in its range.
 template <bool SETTLE, bool M1, int SEG, class Lds>
 __device__ __forceinline__ void edr_lookup(EdrRow<M1, SEG> &r, const Lds &S, int i, double s)
 {
-	int b = S.Q[min((int)(s * ED_NB), ED_NB - 1)];
+	int b = S.Q[1 + max(min((int)(s * ED_NB), ED_NB - 1), -1)];
 	if (SETTLE) {
 		while (s < S.D[b]) b--;
 		while (s >= S.D[b + 2]) b++;
@@ -3053,7 +3056,7 @@ struct EdrCtx {
 	int par;                  // LDS slot of the current row (alternates at each barrier)
 };
 
-// The lane's samples of row j, 0.0 past the row's end.
+// The lane's samples of row j, -1.0 past the row's end.
 template <int SEG>
 __device__ __forceinline__ void edr_load(const EdrCtx &c, int j, double (&v)[SEG])
 {
@@ -3061,7 +3064,7 @@ __device__ __forceinline__ void edr_load(const EdrCtx &c, int j, double (&v)[SEG
 #pragma unroll
 	for (int i = 0; i < SEG; i++) {
 		const double s = row[ed_sample_at(min(c.x0 + i, c.W - 1), c.W, SEG == 8 ? 3 : 2)];
-		v[i] = i < c.n ? s : 0.0;
+		v[i] = i < c.n ? s : -1.0;
 	}
 }
 
@@ -3110,7 +3113,7 @@ __device__ __forceinline__ void edr_row(EdrCtx &c, EdrRow<M1, SEG> &r, double (&
 		}
 	}
 #pragma unroll
-	for (int i = 0; i < SEG; i++) edr_lookup<false>(r, S, i, fmin(fmax(r.X[i] + r.Y[i], 0.0), 1.0));
+	for (int i = 0; i < SEG; i++) edr_lookup<false>(r, S, i, fmax(r.X[i] + r.Y[i], -1.0));
 	r.ex = 0;
 
 	// (u1, u2): the state the last walk started from; pend: the predecessor
@@ -3307,8 +3310,9 @@ __device__ __forceinline__ void edr_plane(const DevPlan &P, int o, EdrLds<NW> &S
 		S.D[k] = d;
 	}
 	// The level below the bin's middle: its upper boundary is the nearest.
+	if (tid == 0) S.Q[0] = 0;
 	for (int k = tid; k < ED_NB; k += NT)
-		S.Q[k] = (unsigned short)(level_in(q.lin, 1, Pq, (k + 0.5) / (double)ED_NB) - 1);
+		S.Q[1 + k] = (unsigned short)(level_in(q.lin, 1, Pq, (k + 0.5) / (double)ED_NB) - 1);
 	__syncthreads();
 	c.eps_hi = (unsigned int)(S.eps >> 32) + 1u;
 
