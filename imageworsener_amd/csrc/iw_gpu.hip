@@ -70,10 +70,9 @@ struct DevWeights {
 	const int *copy_src;
 	double edge;
 	int edge_transparent;  // outside positions read edge (else the nearest sample)
-	// The list by input position (iwx::DenseWeights).  Vertical lists: output
-	// j's weights at dw[doff[j]]..; horizontal ones: weight k of output i at
-	// dw[k * num_out + i], so that neighbouring pixels read neighbouring
-	// weights.
+	// The list by input position (iwx::DenseWeights): output j's weights at
+	// dw[doff[j]].., or, in a horizontal list laid out by tap
+	// (DevPlan::h_by_tap), weight k of output i at dw[k * num_out + i].
 	const int *dfirst, *dcount, *doff;
 	const double *dw;
 	int dmax;
@@ -140,9 +139,10 @@ struct DevPlan {
 	int apply_bkgd, late, checker, check_size, ox, oy, bk_has_trans;
 	int v_shared;  // every channel has the same vertical weights (dense form) in WEIGHTS mode
 	int band_lds_max;  // fused form: LDS a workgroup may use
-	int band_group;    // fused form: a row's sum visits the positions of its group of so many rows
+	int band_group;    // bands of a job alone: a row's sum visits the positions of its group of so many rows
 	int vband_r;   // two-pass form: output rows per thread of vband_kernel (0: vpass_kernel)
 	int h_shared;  // the same for the horizontal weights
+	int h_by_tap;  // layout of the horizontal weights (DevWeights::dw)
 	double bk1a, bk2a;
 	// Chosen-precision form: the shared horizontal list by 4-column blocks.
 	// Output column i: (first block, block count, offset) in h4i[i]; block b
@@ -780,13 +780,14 @@ struct BandRows {
 // load(c, r, x): sample x of intermediate row r.  Columns whose list lies
 // inside the row read four samples at a time (load.four), so that a cache line
 // is asked for once per four taps.  Then the rows' pixels one by one.
-template <int RR, bool SKIP, class Emit, class Load>
+template <int RR, bool SKIP, bool BY_OUT, class Emit, class Load>
 __device__ __forceinline__ void hrows(const DevPlan &P, const Emit &E, int i, int j0, int n, Load load)
 {
 	const int C = P.inter_nch, W = P.W, ow = P.out_w;
 	const DevWeights &h0 = P.ic[0].h;
 	const int f0 = ((const g_cint *)h0.dfirst)[i], cnt = ((const g_cint *)h0.dcount)[i];
-	const g_cf64 *hw = (const g_cf64 *)h0.dw + i;
+	const g_cf64 *hw = (const g_cf64 *)h0.dw + (!BY_OUT && P.h_by_tap ? i : ((const g_cint *)h0.doff)[i]);
+	const int hstep = !BY_OUT && P.h_by_tap ? ow : 1;
 	double acc[RR][IWAMD_MAX_CH];
 #pragma unroll
 	for (int r = 0; r < RR; r++)
@@ -797,7 +798,7 @@ __device__ __forceinline__ void hrows(const DevPlan &P, const Emit &E, int i, in
 		for (; u + 4 <= cnt; u += 4) {
 			double w[4];
 #pragma unroll
-			for (int t = 0; t < 4; t++) w[t] = hw[(size_t)(u + t) * ow];
+			for (int t = 0; t < 4; t++) w[t] = hw[(size_t)(u + t) * hstep];
 #pragma unroll
 			for (int c = 0; c < IWAMD_MAX_CH; c++) {
 				if (c >= C) break;
@@ -813,7 +814,7 @@ __device__ __forceinline__ void hrows(const DevPlan &P, const Emit &E, int i, in
 		}
 	}
 	for (; u < cnt; u++) {
-		const double w = hw[(size_t)u * ow];
+		const double w = hw[(size_t)u * hstep];
 		const int pos = f0 + u;
 		const bool outside = pos < 0 || pos >= W;
 		const int pc = pos < 0 ? 0 : (pos >= W ? W - 1 : pos);
@@ -874,7 +875,7 @@ __global__ void __launch_bounds__(256) hpass_rows_kernel(DevPlan P)
 	EmitSimple E;
 	emit_simple_ctx(P, E);
 	const InterRows rows = {P.inter + (size_t)j0 * P.W, (size_t)P.Hp * P.W, (size_t)P.W, P.out_h - 1 - j0};
-	hrows<HP_ROWS, false>(P, E, i, j0, min(HP_ROWS, P.out_h - j0), rows);
+	hrows<HP_ROWS, false, false>(P, E, i, j0, min(HP_ROWS, P.out_h - j0), rows);
 }
 
 // Queue the two-pass form's horizontal pass.  (Floating-point samples may not
@@ -1351,10 +1352,18 @@ __device__ __forceinline__ void band_vertical_batch(int depth, const FastCin &F,
 	}
 }
 
-// ALONE: the band of a job that runs by itself, else of a batch or a flight.
-template <int R, bool ALONE>
+// What a band belongs to: a job that runs by itself, or a batch or flight,
+// whose plans with simple per-pixel work (EmitSimple) have kernels of their
+// own.  In one kernel with the generic per-pixel work (several columns' sums
+// at a time) the simple bands' code had 138 to 154 registers instead of 98 to
+// 115, and so a SIMD one wave less: 4096 small RGBA images 42.2 -> 39.2 ms, of
+// which 0.5 ms is the list by output (DevPlan::h_by_tap).
+enum BandKind { BAND_ALONE, BAND_BATCH, BAND_BATCH_ANY };
+
+template <int R, BandKind KIND>
 __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned char *band_lds)
 {
+	constexpr bool ALONE = KIND == BAND_ALONE;
 	double *wd = (double *)band_lds;                       // [R][BAND_MAX_K]
 	double *tab = ALONE && band_has_tab(P.bit_depth == 8 && !P.in_float, R, P.inter_nch, P.W, P.band_lds_max) ? wd + R * BAND_MAX_K : nullptr;  // [2][256]
 	float *inter = (float *)(wd + R * BAND_MAX_K + (tab ? CIN_LDS / sizeof(double) : 0));  // [C][R][W]
@@ -1369,8 +1378,8 @@ __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned cha
 	for (int c = 0; c < (depth ? 1 : C); c++) {
 		const DevIChan &ic = P.ic[c];
 		const DevWeights &dv = ic.v;
-		// The group's input positions.
-		const int g0 = j0 - j0 % P.band_group, g1 = min(g0 + P.band_group, P.Hp);
+		// The input positions of the band, or of the group that it is of.
+		const int g0 = ALONE ? j0 - j0 % P.band_group : j0, g1 = ALONE ? min(g0 + P.band_group, P.Hp) : j0 + rows;
 		int p_lo, K;
 		band_span(dv, g0, g1, p_lo, K);
 		__syncthreads();  // previous channel's weights no longer read
@@ -1459,20 +1468,20 @@ __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned cha
 		const BandRows load = {inter + r0 * W, R * W, W, n - 1};  // the thread's rows
 		for (int i = tid % cols; i < P.out_w; i += cols) {
 			if constexpr (SIMPLE) {
-				if (per == 1) hrows<1, false>(P, E, i, j0 + r0, n, load);
-				else if (per == 2) hrows<(R < 2 ? 1 : 2), false>(P, E, i, j0 + r0, n, load);
-				else hrows<R, false>(P, E, i, j0 + r0, n, load);
+				if (per == 1) hrows<1, false, !ALONE>(P, E, i, j0 + r0, n, load);
+				else if (per == 2) hrows<(R < 2 ? 1 : 2), false, !ALONE>(P, E, i, j0 + r0, n, load);
+				else hrows<R, false, !ALONE>(P, E, i, j0 + r0, n, load);
 			} else {
 				for (int q = 0; q < n; q++) {
 					const BandRows row = {load.p + q * W, load.cstride, W, 0};
-					if (P.in_float) hrows<1, true>(P, E, i, j0 + r0 + q, 1, row);
-					else hrows<1, false>(P, E, i, j0 + r0 + q, 1, row);
+					if (P.in_float) hrows<1, true, !ALONE>(P, E, i, j0 + r0 + q, 1, row);
+					else hrows<1, false, !ALONE>(P, E, i, j0 + r0 + q, 1, row);
 				}
 			}
 		}
 	};
 	EmitSimple ES;
-	if (emit_simple_ctx(P, ES)) {
+	if (KIND != BAND_BATCH_ANY && emit_simple_ctx(P, ES)) {
 		if (P.h_shared) {
 			if constexpr (ALONE) {
 				columns(ES);
@@ -1482,7 +1491,7 @@ __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned cha
 				for (int t = tid; t < n_px; t += blockDim.x) {
 					const int r = t / P.out_w, i = t % P.out_w;
 					const BandRows row = {inter + r * W, R * W, W, 0};
-					hrows<1, false>(P, ES, i, j0 + r, 1, row);
+					hrows<1, false, true>(P, ES, i, j0 + r, 1, row);
 				}
 			}
 			return;
@@ -1496,7 +1505,7 @@ __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned cha
 				for (int c = 0; c < IWAMD_MAX_CH; c++) g[c] = c < C ? hsum(c, r[n], pi[n]) : 0.0;
 			});
 		}
-	} else {
+	} else if constexpr (KIND != BAND_BATCH) {
 		EmitCtx E;
 		emit_ctx(P, E);
 		if (P.h_shared) {
@@ -1515,7 +1524,7 @@ __device__ __forceinline__ void band_body(const DevPlan &P, int j0, unsigned cha
 // gridDim.x + atomicAdd(counter, 1) until none is left -- a persistent
 // kernel over a whole batch.  (The band lists keep this one queue: with the
 // chosen form's per-XCD chunks the C3 batch's plain form ran 41.1 -> 45.3 ms.)
-template <int R, bool ALONE>
+template <int R, BandKind KIND>
 __global__ void __launch_bounds__(256) band_kernel(const DevPlan *__restrict__ plans,
 	const int2 *__restrict__ items, int n_items, int *counter)
 {
@@ -1524,7 +1533,7 @@ __global__ void __launch_bounds__(256) band_kernel(const DevPlan *__restrict__ p
 	int it = blockIdx.x;
 	while (it < n_items) {
 		const int2 w = items[it];
-		band_body<R, ALONE>(plans[w.x], w.y, band_lds);
+		band_body<R, KIND>(plans[w.x], w.y, band_lds);
 		if (!counter) break;
 		__syncthreads();  // LDS of this item is no longer read
 		if (threadIdx.x == 0) next_item = (int)gridDim.x + atomicAdd(counter, 1);
@@ -3397,9 +3406,11 @@ bool runtime_init(iw_context *ctx)
 	}
 	// The band kernels size their LDS per launch, up to the workgroup limit
 	// (160 KB on gfx950); where the runtime refuses, they keep 64 KB.
-	const void *bk[6] = {(const void *)band_kernel<1, false>, (const void *)band_kernel<2, false>,
-		(const void *)band_kernel<4, false>, (const void *)band_kernel<1, true>, (const void *)band_kernel<2, true>,
-		(const void *)band_kernel<4, true>};
+	const void *bk[9] = {(const void *)band_kernel<1, BAND_ALONE>, (const void *)band_kernel<2, BAND_ALONE>,
+		(const void *)band_kernel<4, BAND_ALONE>, (const void *)band_kernel<1, BAND_BATCH>,
+		(const void *)band_kernel<2, BAND_BATCH>, (const void *)band_kernel<4, BAND_BATCH>,
+		(const void *)band_kernel<1, BAND_BATCH_ANY>, (const void *)band_kernel<2, BAND_BATCH_ANY>,
+		(const void *)band_kernel<4, BAND_BATCH_ANY>};
 	R.band_lds_max = 160 * 1024;
 	for (const void *f : bk) {
 		if (hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)R.band_lds_max) != hipSuccess) {
@@ -3971,6 +3982,8 @@ struct Staged {
 	};
 	std::vector<List> lists[2];  // by IW_DIMENSION_*
 	int list_of[2][IWAMD_MAX_CH] = {};
+	bool batch = false;          // of a batch or a flight (set before stage_job)
+	bool h_by_tap = false;       // DevPlan::h_by_tap
 	const iwx::WeightList &wv(int c) const { return lists[IW_DIMENSION_V][list_of[IW_DIMENSION_V][c]].wl; }
 	const iwx::WeightList &wh(int c) const { return lists[IW_DIMENSION_H][list_of[IW_DIMENSION_H][c]].wl; }
 	const iwx::DenseWeights &dv(int c) const { return lists[IW_DIMENSION_V][list_of[IW_DIMENSION_V][c]].d; }
@@ -4322,6 +4335,9 @@ bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path
 	Layout L;
 	S.in_bytes = S.in_f64.empty() ? p.in_bpr * (size_t)phys_rows : S.in_f64.size() * sizeof(double);
 	S.in_elsewhere = in_elsewhere;
+	// A batch's bands read a list by output, four taps of one pixel at a time;
+	// the others by tap, so that neighbouring pixels read neighbouring weights.
+	S.h_by_tap = !S.batch || (!S.band_rows && S.fast.empty());
 	S.o_in = L.add<uint8_t>(in_elsewhere ? 0 : S.in_bytes);
 	S.o_inter = L.add<float>(S.band_rows ? 0 : (size_t)p.inter_nch * p.inter_height * p.inter_width);
 	S.out_bytes = p.out_bpr * (size_t)p.out_height;
@@ -4340,8 +4356,9 @@ bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path
 			o.copy = L.add<int>(l.wl.copy_src.size());
 			o.dfirst = L.add<int>(l.d.first.size());
 			o.dcount = L.add<int>(l.d.count.size());
-			o.doff = L.add<int>(dim == IW_DIMENSION_V ? l.d.off.size() : 0);
-			o.dw = L.add<double>(dim == IW_DIMENSION_H ? (size_t)l.d.max_count * l.d.first.size() : l.d.w.size());
+			const bool by_tap = dim == IW_DIMENSION_H && S.h_by_tap;
+			o.doff = L.add<int>(by_tap ? 0 : l.d.off.size());
+			o.dw = L.add<double>(by_tap ? (size_t)l.d.max_count * l.d.first.size() : l.d.w.size());
 			S.o_list[dim].push_back(o);
 		}
 	}
@@ -4413,7 +4430,7 @@ bool upload_job(Staged &S, const iwamd_plan &p, char *base, hipStream_t st, cons
 			up(o.copy, wl.copy_src.data(), wl.copy_src.size() * 4);
 			up(o.dfirst, d.first.data(), d.first.size() * 4);
 			up(o.dcount, d.count.data(), d.count.size() * 4);
-			if (dim == IW_DIMENSION_V) {
+			if (dim == IW_DIMENSION_V || !S.h_by_tap) {
 				up(o.doff, d.off.data(), d.off.size() * 4);
 				up(o.dw, d.w.data(), d.w.size() * 8);
 			} else {
@@ -4513,6 +4530,7 @@ void fill_dev_plan(const Staged &S, const iwamd_plan &p, char *base, DevPlan &D)
 	D.band_lds_max = (int)rt().band_lds_max;
 	D.band_group = S.in_int || !S.band_group ? std::max(1, S.band_rows) : S.band_group;
 	D.v_shared = p.inter_nch > 0 && one_list(S, IW_DIMENSION_V) && S.wv(0).mode == iwx::WeightList::WEIGHTS;
+	D.h_by_tap = S.h_by_tap;
 	D.h_shared = p.inter_nch > 0 && one_list(S, IW_DIMENSION_H) && S.wh(0).mode == iwx::WeightList::WEIGHTS;
 	for (int c = 0; c < p.inter_nch; c++) {
 		const iwamd_ichan &s = p.ich[c];
@@ -4615,13 +4633,14 @@ void fill_dev_plan(const Staged &S, const iwamd_plan &p, char *base, DevPlan &D)
 // two-pass kernels.
 
 constexpr int kBandR[3] = {1, 2, 4};
+constexpr int kBandLists = 6;  // by band height, the plans of BAND_BATCH_ANY after the others
 // Bands are also grouped by the LDS they need (<= 16, 32, 64, 128 KiB, more),
 // one persistent launch per group, so a batch's widest rows do not lower the
 // occupancy of its narrow ones.
 constexpr int kLdsClasses = 5;
 // Persistent work counters: one per band list (band height r, LDS class q)
 // at r * kLdsClasses + q, then XCD_COUNT per chosen-form variant.
-constexpr int kCounters = 3 * kLdsClasses + XCD_COUNT * FAST_NVAR;
+constexpr int kCounters = kBandLists * kLdsClasses + XCD_COUNT * FAST_NVAR;
 
 int lds_class(size_t bytes)
 {
@@ -4673,9 +4692,10 @@ int ed_rows_shift(const Staged &S, const iwamd_plan &p)
 
 struct WorkSet {
 	std::vector<DevPlan> plans;       // host copies; the two-pass kernels take them by value
-	std::vector<int2> bands[3][kLdsClasses];  // (plan, first row), by band height kBandR and LDS class
-	size_t band_lds[3][kLdsClasses] = {};      // largest LDS of a band in each list
-	size_t band_lds_alone[3][kLdsClasses] = {};  // the same with the tables of a job that runs alone
+	bool batch = false;               // the plans' Staged::batch: their bands run a batch's kernels
+	std::vector<int2> bands[kBandLists][kLdsClasses];  // (plan, first row), by kBandLists and LDS class
+	size_t band_lds[kBandLists][kLdsClasses] = {};  // largest LDS of a band in each list
+	size_t band_lds_alone[kBandLists][kLdsClasses] = {};  // the same with the tables of a job that runs alone
 	std::vector<int2> planes[kEdVariants];  // (plan, output channel), by ed_variant
 	std::vector<int2> ilv;            // (plan, first row) of the outputs edr_interleave_kernel forms
 	std::vector<int> twopass;         // plans resampled by vpass + hpass
@@ -4685,7 +4705,7 @@ struct WorkSet {
 	std::vector<int4> fast_runs;      // (first, count, variant, -) per band, before splitting
 	std::vector<int2> fast[FAST_NVAR];
 	int fast_chunks[FAST_NVAR][XCD_COUNT + 1] = {};  // each chosen-form list's chunks, one per XCD
-	size_t o_plans = 0, o_bands[3][kLdsClasses] = {}, o_planes[kEdVariants] = {0}, o_counters = 0, o_fast[FAST_NVAR] = {},
+	size_t o_plans = 0, o_bands[kBandLists][kLdsClasses] = {}, o_planes[kEdVariants] = {0}, o_counters = 0, o_fast[FAST_NVAR] = {},
 		o_chunks = 0, o_done = 0, o_ilv = 0;
 	size_t bytes = 0;
 	const FastItem *d_fast_tiles = nullptr;
@@ -4693,7 +4713,7 @@ struct WorkSet {
 	size_t o_fast_tiles = 0;
 	int *d_done = nullptr;  // one error-diffusion completion counter per plan
 	const DevPlan *d_plans = nullptr;
-	const int2 *d_bands[3][kLdsClasses] = {};
+	const int2 *d_bands[kBandLists][kLdsClasses] = {};
 	const int2 *d_planes[kEdVariants] = {nullptr};
 	const int2 *d_ilv = nullptr;
 	const int *d_chunks = nullptr;
@@ -4719,12 +4739,23 @@ int fast_variant(const Staged &S, const iwamd_plan &p)
 	return fast_rgba8_ok(D, ES, F) ? FAST_RGBA8 : FAST_LEAN8;
 }
 
+// The band kernel of a plan's bands, decided as fast_variant decides.
+BandKind band_kind(const Staged &S, const iwamd_plan &p)
+{
+	if (!S.batch) return BAND_ALONE;
+	DevPlan D;
+	fill_dev_plan(S, p, (char *)(uintptr_t)0x100000000ull, D);
+	EmitSimple ES;
+	return emit_simple_ctx(D, ES) ? BAND_BATCH : BAND_BATCH_ANY;
+}
+
 // Adds a job's work; its kernel arguments are set later (W.plans[index]),
 // once its device data has a place.  Returns the job's index.
 int ws_add(WorkSet &W, const Staged &S, const iwamd_plan &p)
 {
 	const int jx = (int)W.plans.size();
 	W.plans.push_back(DevPlan());
+	W.batch = S.batch;
 	if (S.skip_pixels) return jx;
 	if (!S.fast.empty()) {
 		const int var = fast_variant(S, p);
@@ -4741,7 +4772,7 @@ int ws_add(WorkSet &W, const Staged &S, const iwamd_plan &p)
 			k = e;
 		}
 	} else if (S.band_rows) {
-		const int ri = S.band_rows == 4 ? 2 : (S.band_rows == 2 ? 1 : 0);
+		const int ri = (S.band_rows == 4 ? 2 : (S.band_rows == 2 ? 1 : 0)) + (band_kind(S, p) == BAND_BATCH_ANY ? 3 : 0);
 		const bool tab = band_has_tab(S.in_int && p.in_bit_depth == 8, S.band_rows, p.inter_nch, p.inter_width,
 			rt().band_lds_max);
 		const size_t lds = band_lds_rows(S.band_rows, p.inter_nch, p.inter_width);
@@ -4795,7 +4826,7 @@ void ws_layout(WorkSet &W)
 	}
 	Layout L;
 	W.o_plans = L.add<DevPlan>(W.plans.size());
-	for (int r = 0; r < 3; r++)
+	for (int r = 0; r < kBandLists; r++)
 		for (int q = 0; q < kLdsClasses; q++) W.o_bands[r][q] = L.add<int2>(W.bands[r][q].size());
 	for (int v = 0; v < kEdVariants; v++) W.o_planes[v] = L.add<int2>(W.planes[v].size());
 	W.o_ilv = L.add<int2>(W.ilv.size());
@@ -4816,7 +4847,7 @@ void ws_pack(WorkSet &W, char *base)
 	};
 	W.d_plans = (const DevPlan *)(base + W.o_plans);
 	up(W.o_plans, W.plans.data(), W.plans.size() * sizeof(DevPlan));
-	for (int r = 0; r < 3; r++) {
+	for (int r = 0; r < kBandLists; r++) {
 		for (int q = 0; q < kLdsClasses; q++) {
 			W.d_bands[r][q] = (const int2 *)(base + W.o_bands[r][q]);
 			up(W.o_bands[r][q], W.bands[r][q].data(), W.bands[r][q].size() * sizeof(int2));
@@ -4877,7 +4908,7 @@ void ws_enqueue_resample(const WorkSet &W, hipStream_t st, bool persistent)
 		const int n = (int)W.fast[v].size();
 		if (!n) continue;
 		const int grid = persistent ? std::min(n, device_cu_count() * (v == FAST_GENERIC ? 1 : FAST_WG_PER_CU)) : n;
-		int *ctr = persistent ? W.d_counters + 3 * kLdsClasses + XCD_COUNT * v : nullptr;
+		int *ctr = persistent ? W.d_counters + kBandLists * kLdsClasses + XCD_COUNT * v : nullptr;
 		const int *ch = W.d_chunks + v * (XCD_COUNT + 1);
 		switch (v) {
 		case FAST_RGBA8:
@@ -4898,11 +4929,11 @@ void ws_enqueue_resample(const WorkSet &W, hipStream_t st, bool persistent)
 			break;
 		}
 	}
-	for (int r = 0; r < 3; r++)
+	for (int r = 0; r < kBandLists; r++)
 		for (int q = 0; q < kLdsClasses; q++) {
 			const int n = (int)W.bands[r][q].size();
 			if (!n) continue;
-			const size_t lds = W.band_lds[r][q];
+			const size_t lds = W.batch ? W.band_lds[r][q] : W.band_lds_alone[r][q];
 			const int2 *items = W.d_bands[r][q];
 			int grid = n;
 			if (persistent) {
@@ -4910,16 +4941,14 @@ void ws_enqueue_resample(const WorkSet &W, hipStream_t st, bool persistent)
 				grid = std::min(n, device_cu_count() * per_cu);
 			}
 			int *ctr = persistent ? W.d_counters + r * kLdsClasses + q : nullptr;
-			auto launch = [&](auto alone, auto batch) {
-				if (persistent)
-					hipLaunchKernelGGL(batch, dim3(grid), dim3(256), lds, st, W.d_plans, items, n, ctr);
-				else
-					hipLaunchKernelGGL(alone, dim3(grid), dim3(256), W.band_lds_alone[r][q], st, W.d_plans, items, n, ctr);
+			auto launch = [&](auto alone, auto batch, auto any) {
+				hipLaunchKernelGGL(!W.batch ? alone : (r < 3 ? batch : any), dim3(grid), dim3(256), lds, st, W.d_plans,
+					items, n, ctr);
 			};
-			switch (kBandR[r]) {
-			case 1: launch(band_kernel<1, true>, band_kernel<1, false>); break;
-			case 2: launch(band_kernel<2, true>, band_kernel<2, false>); break;
-			default: launch(band_kernel<4, true>, band_kernel<4, false>); break;
+			switch (kBandR[r % 3]) {
+			case 1: launch(band_kernel<1, BAND_ALONE>, band_kernel<1, BAND_BATCH>, band_kernel<1, BAND_BATCH_ANY>); break;
+			case 2: launch(band_kernel<2, BAND_ALONE>, band_kernel<2, BAND_BATCH>, band_kernel<2, BAND_BATCH_ANY>); break;
+			default: launch(band_kernel<4, BAND_ALONE>, band_kernel<4, BAND_BATCH>, band_kernel<4, BAND_BATCH_ANY>); break;
 			}
 		}
 	for (int jx : W.twopass) {
@@ -4967,7 +4996,8 @@ double resample_flops(const iwamd_plan &p, const Staged &S)
 // 16-column chunks they sum over do not depend on the tile width.  So the
 // shape for a class of jobs -- form, channels, vertical and horizontal taps
 // per output (filter radius x scale factor) and output width, each as
-// ceil(log2) -- is chosen by timing: the first job of a class that may be
+// ceil(log2), and the band kernel -- is chosen by timing: the first job of a
+// class that may be
 // tuned runs its resampling once per candidate shape on its own device copy,
 // its work repeated to fill the device (a warm run, then the best of three;
 // time per copy: a batch's throughput, not one job's latency), the fastest
@@ -4977,9 +5007,10 @@ double resample_flops(const iwamd_plan &p, const Staged &S)
 
 struct TuneKey {
 	int form, nch, tv, th, wb;
+	int kind;  // BandKind (bands)
 	bool operator<(const TuneKey &o) const
 	{
-		return std::tie(form, nch, tv, th, wb) < std::tie(o.form, o.nch, o.tv, o.th, o.wb);
+		return std::tie(form, nch, tv, th, wb, kind) < std::tie(o.form, o.nch, o.tv, o.th, o.wb, o.kind);
 	}
 };
 
@@ -5028,6 +5059,7 @@ TuneKey tune_key(const iwamd_plan &p, const Staged &S, int form)
 	k.tv = log2_bucket(mean_taps(S.dv(0), p.inter_height));
 	k.th = log2_bucket(mean_taps(S.dh(0), p.out_width));
 	k.wb = log2_bucket(p.out_width / 64.0);
+	k.kind = form == 0 ? band_kind(S, p) : BAND_ALONE;
 	return k;
 }
 
@@ -5843,6 +5875,7 @@ extern "C" int iwamd_batch_add(struct iwamd_batch *B, struct iw_context *ctx)
 	}
 	iwamd_batch::Job *J = new iwamd_batch::Job();
 	J->ctx = ctx;
+	J->S.batch = true;
 	if (!iwamd_prepare(ctx, &J->plan) || !runtime_init(ctx) ||
 		!stage_job(ctx, J->plan, J->S, iw_get_option(ctx, "amd:resample"), true)) {
 		delete J;
@@ -6315,6 +6348,7 @@ extern "C" int iwamd_server_submit(struct iwamd_server *V, struct iw_context *ct
 {
 	ServerExec::Loop::Req *R = new ServerExec::Loop::Req();
 	R->data.ctx = ctx;
+	R->data.S.batch = true;
 	if (!iwamd_prepare(ctx, &R->data.plan) || !runtime_init(ctx) ||
 		!stage_job(ctx, R->data.plan, R->data.S, iw_get_option(ctx, "amd:resample"), true)) {
 		delete R;

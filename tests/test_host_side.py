@@ -1,0 +1,100 @@
+"""The library's host side without a GPU: decisions, work lists, pools and error
+paths, on a HIP runtime of host memory whose kernels do nothing
+(tests/hip_mock.c).  Each test runs in a process of its own, since the mock
+takes the place of the HIP runtime in it."""
+import ctypes
+import os
+import subprocess
+import sys
+
+import numpy as np
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+
+@pytest.fixture(scope="session")
+def mock_so(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("mock") / "libhip_mock.so")
+    subprocess.run(["gcc", "-O1", "-Wall", "-shared", "-fPIC", os.path.join(HERE, "hip_mock.c"), "-o", so, "-lpthread"],
+                   check=True)
+    return so
+
+
+@pytest.fixture
+def scenario(mock_so):
+    def run(name, *args):
+        r = subprocess.run([sys.executable, os.path.abspath(__file__), mock_so, name] + [str(a) for a in args],
+                           stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=300)
+        assert r.returncode == 0, r.stdout[-4000:]
+    return run
+
+
+# ---- scenarios (run in the child) -----------------------------------------------
+
+class Mock:
+    """The mock runtime, loaded for the whole process, and the library on it."""
+
+    def __init__(self, so):
+        self.m = ctypes.CDLL(so, mode=ctypes.RTLD_GLOBAL)
+        self.m.mock_launch.restype = ctypes.c_char_p
+        self.m.mock_launch_items.restype = ctypes.c_void_p
+        self.m.mock_fail_malloc.argtypes = [ctypes.c_size_t, ctypes.c_size_t]
+        sys.path[:0] = [os.path.dirname(HERE), HERE]
+        from imageworsener_amd import api
+        self.lib = api.Library()
+
+    def launches(self, part=""):
+        """(index, name, grid) of the launches so far whose kernel has part in its name."""
+        out = []
+        g = (ctypes.c_uint * 3)()
+        for i in range(self.m.mock_launches()):
+            name = self.m.mock_launch(i, g).decode()
+            if part in name:
+                out.append((i, name, tuple(g)))
+        return out
+
+
+def s_batch_bands(M):
+    """A batch of plans with simple and with generic per-pixel work, more of
+    each than one band height and LDS class takes: every band kernel gets a
+    work list of its own, of rows that its plans have, and every row of every
+    fused plan is in one list."""
+    import cases
+    from imageworsener_amd import api, synth
+    jobs = [dict(j, options=[("amd:band_rows", str(r))]) for _, j in cases.sweep_jobs() for r in (1, 2, 4)]
+    big = synth.c3_image(900, 60, 3)
+    for w in (20, 200, 900):
+        for bkgd in (False, True):
+            j = api.image_job(np.ascontiguousarray(big[:, :w]), w, 60, cases.RGBA, 8, canvas=(w, 77),
+                              resize=api.resize_both("catrom"), options=[("amd:band_rows", "4")])
+            jobs.append(dict(j, bkgd=(0.2, 0.5, 0.9, 0.5)) if bkgd else j)
+    os.environ["IWAMD_TUNE"] = "0"
+    M.m.mock_clear_log()
+    b = M.lib.batch(jobs)
+    seen, kinds = {}, set()
+    for i, name, grid in M.launches("11band_kernel"):
+        rows = int(name.split("band_kernelILi")[1][0])
+        kinds.add((rows, name.split("BandKindE")[1][0]))
+        n, p = M.m.mock_launch_count(i), M.m.mock_launch_items(i)
+        assert p and n >= grid[0] > 0, (name, n, p)
+        items = np.ctypeslib.as_array((ctypes.c_int * (2 * n)).from_address(p)).reshape(n, 2)
+        for plan, row in items:
+            assert 0 <= plan < len(jobs) and row % rows == 0, (name, plan, row)
+            assert (plan, row) not in seen
+            seen[plan, row] = rows
+    assert kinds == {(r, k) for r in (1, 2, 4) for k in "12"}, kinds
+    for k, j in enumerate(jobs):
+        got = sorted(r for p, r in seen if p == k)
+        if got:
+            assert got == list(range(0, j["canvas"][1], seen[k, 0])), (k, got)
+    assert len({p for p, _ in seen}) > len(jobs) // 2
+    b.close()
+
+
+def test_batch_bands(scenario):
+    scenario("s_batch_bands")
+
+
+if __name__ == "__main__":
+    globals()[sys.argv[2]](Mock(sys.argv[1]), *sys.argv[3:])
