@@ -4005,7 +4005,7 @@ struct Staged {
 	size_t in_f64_bpr = 0;
 	bool skip_pixels = false;  // unknown filter: the reference reports and outputs zeros
 	int band_rows = 0;         // rows per band of the fused kernel; 0: two-pass kernels
-	int band_group = 0;        // band_rows before band_rows_alone (0: the same)
+	int band_group = 0;        // band_rows as staged, before tuning and band_rows_alone
 	int fast_ti = 0;           // output columns per chosen-precision tile
 	std::vector<int4> h4i;     // chosen form: the horizontal list by 4-column blocks (DevPlan::h4i)
 	std::vector<float> h4w;
@@ -4330,6 +4330,7 @@ bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path
 			S.band_rows = want_rows;
 			S.shape_forced = true;
 		}
+		S.band_group = S.band_rows;
 	}
 
 	Layout L;
@@ -4528,7 +4529,7 @@ void fill_dev_plan(const Staged &S, const iwamd_plan &p, char *base, DevPlan &D)
 	D.W = p.inter_width;
 	D.Hp = p.inter_height;
 	D.band_lds_max = (int)rt().band_lds_max;
-	D.band_group = S.in_int || !S.band_group ? std::max(1, S.band_rows) : S.band_group;
+	D.band_group = std::max(1, S.in_int ? S.band_rows : S.band_group);
 	D.v_shared = p.inter_nch > 0 && one_list(S, IW_DIMENSION_V) && S.wv(0).mode == iwx::WeightList::WEIGHTS;
 	D.h_by_tap = S.h_by_tap;
 	D.h_shared = p.inter_nch > 0 && one_list(S, IW_DIMENSION_H) && S.wh(0).mode == iwx::WeightList::WEIGHTS;
@@ -5001,9 +5002,11 @@ double resample_flops(const iwamd_plan &p, const Staged &S)
 // tuned runs its resampling once per candidate shape on its own device copy,
 // its work repeated to fill the device (a warm run, then the best of three;
 // time per copy: a batch's throughput, not one job's latency), the fastest
-// shape is kept for the class, and later jobs of the class take it.  Batches tune; single jobs
-// and the request loop only look the class up (amd:tune=1 lets a single job
-// tune; IWAMD_TUNE=0 in the environment turns tuning off).
+// shape is kept for the class, and later jobs of the class take it.  A single
+// job's bands have a kernel and so classes of their own, timed as one job.
+// Batches tune; single jobs and the request loop only look the class up
+// (amd:tune=1 lets a single job tune; IWAMD_TUNE=0 in the environment turns
+// tuning off).
 
 struct TuneKey {
 	int form, nch, tv, th, wb;
@@ -5085,20 +5088,22 @@ void tune_set(const iwamd_plan &p, Staged &S, int form, int shape)
 // One job's resampling cost with each candidate shape, on its own device
 // copy, as a batch would see it: the job's work items are repeated until the
 // list holds about four workgroups per CU (the copies write the same bytes to
-// the same output), and the time is divided by the number of copies.
+// the same output), and the time is divided by the number of copies.  The
+// bands of a job alone are timed as they will run: once, one workgroup each.
 bool tune_measure(const iwamd_plan &p, Staged &S, int form, const int *cand, int n, double *ms, hipStream_t st)
 {
 	const size_t out_al = (S.out_bytes + 255) & ~(size_t)255;
 	void *blk = dev_alloc(S.bytes + out_al);
 	if (!blk) return false;
 	char *base = (char *)blk;
+	const bool alone = form == 0 && !S.batch;
 	bool ok = upload_job(S, p, base, st);
 	hipEvent_t e0 = nullptr, e1 = nullptr;
 	ok = ok && hipEventCreate(&e0) == hipSuccess && hipEventCreate(&e1) == hipSuccess;
 	for (int k = 0; k < n && ok; k++) {
 		tune_set(p, S, form, cand[k]);
 		const int items = form == 0 ? (p.inter_height + S.band_rows - 1) / S.band_rows : (int)S.fast.size();
-		const int copies = std::max(1, std::min(256, 4 * device_cu_count() / std::max(1, items)));
+		const int copies = alone ? 1 : std::max(1, std::min(256, 4 * device_cu_count() / std::max(1, items)));
 		WorkSet W;
 		DevPlan D;
 		fill_dev_plan(S, p, base, D);
@@ -5117,7 +5122,7 @@ bool tune_measure(const iwamd_plan &p, Staged &S, int form, const int *cand, int
 		double best = 1e30;
 		for (int r = 0; r < 4 && ok; r++) {
 			ok = hipEventRecord(e0, st) == hipSuccess;
-			ws_enqueue_resample(W, st, true);
+			ws_enqueue_resample(W, st, !alone);
 			ok = ok && hipEventRecord(e1, st) == hipSuccess && hipEventSynchronize(e1) == hipSuccess;
 			float t = 0.0f;
 			if (ok && hipEventElapsedTime(&t, e0, e1) == hipSuccess && r > 0) best = std::min(best, (double)t);
@@ -5149,23 +5154,23 @@ bool tune_enabled()
 // floating-point samples are not finite, a position of weight 0 counts.
 #define BANDS_ALONE 512
 
-void band_rows_alone(const iwamd_plan &p, Staged &S)
+// Where the job's class has been tuned its shape stands.
+void band_rows_alone(const iwamd_plan &p, Staged &S, bool tuned)
 {
-	if (S.shape_forced || !S.band_rows || !S.fast.empty()) return;
-	S.band_group = S.band_rows;
+	if (tuned || S.shape_forced || !S.band_rows || !S.fast.empty()) return;
 	while (S.band_rows > 1 && (p.inter_height + S.band_rows - 1) / S.band_rows < BANDS_ALONE) S.band_rows /= 2;
 }
 
 // Gives the plan its class's tuned shape; a class without one is measured on
 // this job first when may_tune.  A shape that does not fit this job (or a
-// failed measurement) keeps the default choice.
-void tune_apply(const iwamd_plan &p, Staged &S, hipStream_t st, bool may_tune)
+// failed measurement) keeps the default choice (false).
+bool tune_apply(const iwamd_plan &p, Staged &S, hipStream_t st, bool may_tune)
 {
 	const int form = tune_form(S);
-	if (form < 0 || S.shape_forced) return;
+	if (form < 0 || S.shape_forced) return false;
 	int cand[3];
 	const int n = tune_cands(p, S, form, cand);
-	if (n < 2) return;
+	if (n < 2) return false;
 	const int orig = form == 0 ? S.band_rows : S.fast_ti;
 	const TuneKey key = tune_key(p, S, form);
 	Tuner &T = tuner();
@@ -5191,6 +5196,7 @@ void tune_apply(const iwamd_plan &p, Staged &S, hipStream_t st, bool may_tune)
 	bool fits = false;
 	for (int k = 0; k < n; k++) fits |= shape && cand[k] == shape;
 	tune_set(p, S, form, fits ? shape : orig);
+	return fits;
 }
 
 bool job_upload(iwamd_job *J, bool wait)
@@ -5201,9 +5207,8 @@ bool job_upload(iwamd_job *J, bool wait)
 	if (!stage_job(ctx, p, S, iw_get_option(ctx, "amd:resample"))) return false;
 	{
 		const char *t = iw_get_option(ctx, "amd:tune");
-		tune_apply(p, S, J->stream, t && atoi(t) == 1);
+		band_rows_alone(p, S, tune_apply(p, S, J->stream, t && atoi(t) == 1));
 	}
-	band_rows_alone(p, S);
 	J->skip_pixels = S.skip_pixels;
 	J->n_ed = S.n_ed;
 	for (int e = 0; e < 4; e++) J->ed_list[e] = S.ed_list[e];
@@ -5618,9 +5623,9 @@ extern "C" int iwamd_process_device_noalloc(struct iw_context *ctx, const void *
 	hipStream_t st = (hipStream_t)stream;
 	Staged S;
 	if (!stage_job(ctx, p, S, iw_get_option(ctx, "amd:resample"), true, true)) return 0;
-	tune_apply(p, S, st, false);  // look the shape up; never tunes (tuning allocates)
-	const int tall = S.band_rows;
-	band_rows_alone(p, S);
+	// Look the shape up; never tune (tuning allocates).
+	band_rows_alone(p, S, tune_apply(p, S, st, false));
+	const int tall = S.band_group;
 	WorkSet W;
 	ws_add(W, S, p);
 	ws_layout(W);

@@ -152,10 +152,13 @@ IW_EXPORT(int) iwamd_ed_tables(const struct iwamd_ochan *och, double *lin, doubl
  * how the work is cut, not the bytes, so each class of jobs -- form,
  * channels, ceil(log2) of the mean vertical and horizontal taps per output
  * (filter radius x scale factor) and of the output width -- gets the shape
- * that ran fastest on its first tuned job.  Batches tune classes they meet;
- * single jobs (unless the option amd:tune is 1) and the request loop only
- * look them up; IWAMD_TUNE=0 in the environment turns tuning off; the
- * options amd:band_rows (1, 2, 4) and amd:tile (16, 32) fix a job's shape.
+ * that ran fastest on its first tuned job.  The band kernels of single jobs,
+ * of batched plans with simple per-pixel work (8/16-bit output without a late
+ * background, no dither or error diffusion) and of other batched plans have
+ * entries of their own.  Batches tune classes they meet; single jobs (unless
+ * the option amd:tune is 1) and the request loop only look them up;
+ * IWAMD_TUNE=0 in the environment turns tuning off; the options amd:band_rows
+ * (1, 2, 4) and amd:tile (16, 32) fix a job's shape.
  * iwamd_tune_entries() copies up to max entries and returns the count. */
 struct iwamd_tune_entry {
 	int form;          /* 0: band kernel (shape = output rows per band); 1: chosen-precision tiles (shape = output columns) */
@@ -163,7 +166,8 @@ struct iwamd_tune_entry {
 	int shape;         /* the chosen candidate */
 	int n;             /* candidates timed */
 	int cand[3];
-	double ms[3];      /* resampling time per copy of the tuned job, each candidate (copies fill the device) */
+	double ms[3];      /* resampling time per copy of the tuned job, each candidate (copies fill the
+	                      device; a single job's bands: the one job) */
 };
 IW_EXPORT(int) iwamd_tune_entries(struct iwamd_tune_entry *out, int max);
 

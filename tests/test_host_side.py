@@ -96,5 +96,50 @@ def test_batch_bands(scenario):
     scenario("s_batch_bands")
 
 
+def s_tune_alone(M):
+    """amd:tune = 1 times a single job's own band kernels, one launch each, and
+    the job runs the shape that was fastest; later single jobs of its class
+    take it too, batches do not."""
+    import cases
+    from imageworsener_amd import api
+    fastest = [4]
+
+    def ms(nlog):
+        _, name, _ = M.launches("11band_kernel")[-1]
+        return 1.0 if "band_kernelILi%d" % fastest[0] in name else 2.0
+    cb = ctypes.CFUNCTYPE(ctypes.c_double, ctypes.c_int)(ms)
+
+    def bands(job):
+        M.m.mock_clear_log()
+        j = M.lib.device_job(job)
+        timed = len(M.launches("11band_kernel"))
+        j.run()
+        j.sync()
+        last = M.launches("11band_kernel")
+        assert len(last) == timed + 1 and all("BandKindE0" in n for _, n, _ in last)
+        j.close()
+        return int(last[-1][1].split("band_kernelILi")[1][0]), last[-1][2][0], timed
+
+    job = cases.c0_job()
+    assert bands(job) == (1, 240, 0)  # the rule of band_rows_alone
+    M.m.mock_event_ms(cb)
+    tuned = dict(job, options=[("amd:tune", "1")])
+    for f in (4, 2):
+        fastest[0] = f
+        rows, grid, timed = bands(dict(tuned, resize=api.resize_both({4: "lanczos3", 2: "triangle"}[f])))
+        assert (rows, grid) == (f, 240 // f) and timed == 3 * 4, (f, rows, grid, timed)
+    assert bands(job) == (4, 60, 0)
+    M.m.mock_clear_log()
+    b = M.lib.batch([job])
+    assert len(M.launches("11band_kernel")) > 1 and all("BandKindE1" in n for _, n, _ in M.launches("11band_kernel"))
+    b.close()
+    e = [t for t in M.lib.tune_entries() if t["form"] == "band"]
+    assert len(e) == 3 and all(t["candidates"][t["shape"]] == min(t["candidates"].values()) for t in e)
+
+
+def test_tune_alone(scenario):
+    scenario("s_tune_alone")
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]](Mock(sys.argv[1]), *sys.argv[3:])
