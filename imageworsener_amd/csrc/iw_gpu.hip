@@ -3263,12 +3263,13 @@ __device__ __forceinline__ void edr_row(EdrCtx &c, EdrRow<M1, SEG> &r, double (&
 }
 
 // The codes of plans diffused by errdiff_rows_kernel into their outputs:
-// items[blockIdx.x] = (plan, first row), EDR_ILV_ROWS rows each.
+// items[blockIdx.x] = (plan, first row), EDR_ILV_ROWS rows each; without a
+// list plan 0's rows in order.
 #define EDR_ILV_ROWS 8
 __global__ void __launch_bounds__(256) edr_interleave_kernel(const DevPlan *__restrict__ plans,
 	const int2 *__restrict__ items)
 {
-	const int2 it = items[blockIdx.x];
+	const int2 it = items ? items[blockIdx.x] : make_int2(0, blockIdx.x * EDR_ILV_ROWS);
 	const DevPlan &P = plans[it.x];
 	const int q = (P.out_w + 3) >> 2, rows = min(EDR_ILV_ROWS, P.out_h - it.y);
 	for (int t = threadIdx.x; t < q * rows; t += 256) edr_interleave4(P, it.y + t / q, (t % q) * 4);
@@ -3983,6 +3984,7 @@ struct Staged {
 	std::vector<List> lists[2];  // by IW_DIMENSION_*
 	int list_of[2][IWAMD_MAX_CH] = {};
 	bool batch = false;          // of a batch or a flight (set before stage_job)
+	bool least_bytes = false;    // no padding of the horizontal lists (set before stage_job)
 	bool h_by_tap = false;       // DevPlan::h_by_tap
 	const iwx::WeightList &wv(int c) const { return lists[IW_DIMENSION_V][list_of[IW_DIMENSION_V][c]].wl; }
 	const iwx::WeightList &wh(int c) const { return lists[IW_DIMENSION_H][list_of[IW_DIMENSION_H][c]].wl; }
@@ -4336,9 +4338,11 @@ bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path
 	Layout L;
 	S.in_bytes = S.in_f64.empty() ? p.in_bpr * (size_t)phys_rows : S.in_f64.size() * sizeof(double);
 	S.in_elsewhere = in_elsewhere;
-	// A batch's bands read a list by output, four taps of one pixel at a time;
-	// the others by tap, so that neighbouring pixels read neighbouring weights.
-	S.h_by_tap = !S.batch || (!S.band_rows && S.fast.empty());
+	// A batch's bands read a horizontal list by output, four taps of one pixel
+	// at a time; the other kernels by tap, so that neighbouring pixels read
+	// neighbouring weights.
+	// (By tap every output has room for the most taps of any.)
+	S.h_by_tap = !S.least_bytes && (!S.batch || (!S.band_rows && S.fast.empty()));
 	S.o_in = L.add<uint8_t>(in_elsewhere ? 0 : S.in_bytes);
 	S.o_inter = L.add<float>(S.band_rows ? 0 : (size_t)p.inter_nch * p.inter_height * p.inter_width);
 	S.out_bytes = p.out_bpr * (size_t)p.out_height;
@@ -4698,7 +4702,8 @@ struct WorkSet {
 	size_t band_lds[kBandLists][kLdsClasses] = {};  // largest LDS of a band in each list
 	size_t band_lds_alone[kBandLists][kLdsClasses] = {};  // the same with the tables of a job that runs alone
 	std::vector<int2> planes[kEdVariants];  // (plan, output channel), by ed_variant
-	std::vector<int2> ilv;            // (plan, first row) of the outputs edr_interleave_kernel forms
+	std::vector<int2> ilv;            // (plan, first row) of the outputs edr_interleave_kernel forms (a batch's)
+	int ilv_alone = 0;                // the same for a job alone: workgroups, without a list
 	std::vector<int> twopass;         // plans resampled by vpass + hpass
 	// Chosen-precision tiles, and work items over them: runs of one band's
 	// tiles (first tile, count), by kernel variant.
@@ -4789,7 +4794,8 @@ int ws_add(WorkSet &W, const Staged &S, const iwamd_plan &p)
 		const int o = S.ed_list[e];
 		W.planes[ed_variant(S, p, o, rows)].push_back(make_int2(jx, o));
 	}
-	if (rows)
+	if (rows && !S.batch) W.ilv_alone = (p.out_height + EDR_ILV_ROWS - 1) / EDR_ILV_ROWS;
+	else if (rows)
 		for (int j0 = 0; j0 < p.out_height; j0 += EDR_ILV_ROWS) W.ilv.push_back(make_int2(jx, j0));
 	return jx;
 }
@@ -4967,8 +4973,10 @@ void ws_enqueue_errdiff(const WorkSet &W, hipStream_t st, bool interleave = true
 		const int n = (int)W.planes[v].size();
 		if (n) hipLaunchKernelGGL(kEdKernels[v].kernel, dim3(n), dim3(kEdKernels[v].threads), 0, st, W.d_plans, W.d_planes[v]);
 	}
-	if (interleave && !W.ilv.empty())
-		hipLaunchKernelGGL(edr_interleave_kernel, dim3((unsigned int)W.ilv.size()), dim3(256), 0, st, W.d_plans, W.d_ilv);
+	const unsigned int n_ilv = W.batch ? (unsigned int)W.ilv.size() : (unsigned int)W.ilv_alone;
+	if (interleave && n_ilv)
+		hipLaunchKernelGGL(edr_interleave_kernel, dim3(n_ilv), dim3(256), 0, st, W.d_plans,
+			W.batch ? W.d_ilv : (const int2 *)nullptr);
 }
 
 // Useful floating-point operations of a plan's resampling: a multiply and an
@@ -5625,16 +5633,24 @@ extern "C" int iwamd_process_device_noalloc(struct iw_context *ctx, const void *
 	if (!stage_job(ctx, p, S, iw_get_option(ctx, "amd:resample"), true, true)) return 0;
 	// Look the shape up; never tune (tuning allocates).
 	band_rows_alone(p, S, tune_apply(p, S, st, false));
-	const int tall = S.band_group;
 	WorkSet W;
-	ws_add(W, S, p);
-	ws_layout(W);
-	if (S.bytes + W.bytes > IWAMD_NOALLOC_SCRATCH && S.band_rows != tall) {
-		// The shorter bands' work list does not fit: the taller ones'.
-		S.band_rows = tall;
+	auto lay_out = [&]() {
 		W = WorkSet();
 		ws_add(W, S, p);
 		ws_layout(W);
+		return S.bytes + W.bytes <= IWAMD_NOALLOC_SCRATCH;
+	};
+	bool fits = lay_out();
+	if (!fits && S.band_rows != S.band_group) {
+		// Taller bands have a shorter work list.
+		S.band_rows = S.band_group;
+		fits = lay_out();
+	}
+	if (!fits && S.h_by_tap) {
+		S = Staged();
+		S.least_bytes = true;
+		if (!stage_job(ctx, p, S, iw_get_option(ctx, "amd:resample"), true, true)) return 0;
+		lay_out();
 	}
 	const size_t need = S.bytes + W.bytes;
 	if (need > IWAMD_NOALLOC_SCRATCH) {

@@ -141,5 +141,42 @@ def test_tune_alone(scenario):
     scenario("s_tune_alone")
 
 
+def _noalloc(M, job):
+    """(accepted, error) of iwamd_process_device_noalloc for a job."""
+    d = M.lib.dll
+    fn = d.iwamd_process_device_noalloc
+    fn.argtypes = [ctypes.c_void_p, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_size_t,
+                   ctypes.c_void_p, ctypes.c_void_p]
+    ctx = d.iw_create_context(None)
+    M.lib._setup(ctx, job)
+    size = job["image"]["bpr"] * job["image"]["height"] + job["canvas"][0] * job["canvas"][1] * 8
+    a, b = ctypes.create_string_buffer(size), ctypes.create_string_buffer(size)
+    ok = fn(ctx, a, size, b, size, None, None)
+    buf = ctypes.create_string_buffer(300)
+    err = d.iw_get_errormsg(ctx, buf, 300).decode()
+    d.iw_destroy_context(ctx)
+    return bool(ok), err
+
+
+def s_noalloc_lists(M):
+    """The fixed scratch array's limit.  Blurs so wide that outputs at the
+    image's sides have half the taps of those in its middle: the lists fit only
+    without room for the most taps in every output.  And narrow rows by the
+    thousand, diffused: they fit without a list of them."""
+    import cases
+    from imageworsener_amd import api
+    for w, h, ow, oh, fits in [(3000, 40, 999, 800, True), (1000, 1000, 2900, 480, True), (3000, 40, 1500, 800, False),
+                              (40, 2520, 1, 3686, True), (40, 2520, 1, 3690, False)]:
+        job = api.image_job(np.zeros((h, w, 3), np.uint8), w, h, cases.RGB, 8, canvas=(ow, oh),
+                            resize=api.resize_both("triangle", 500.0), values=[(cases.V_CVT_GRAY, 1)],
+                            dither=[(api.CH_ALL, 2, 0)])
+        ok, err = _noalloc(M, job)
+        assert ok == fits, (w, h, ow, oh, err)
+
+
+def test_noalloc_lists(scenario):
+    scenario("s_noalloc_lists")
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]](Mock(sys.argv[1]), *sys.argv[3:])
