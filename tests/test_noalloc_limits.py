@@ -10,6 +10,9 @@ from imageworsener_amd import api, synth
 
 pytestmark = pytest.mark.gpu
 
+pytest.importorskip("torch")  # before the library, so that both use torch's HIP runtime
+import test_zz_no_alloc as zz
+
 JOBS = {  # name: size, output size, horizontal blur, kind
     "fused": (2000, 24, 3700, 30, 500.0, None),
     "fused-late-bkgd": (2000, 24, 3700, 30, 500.0, "bkgd"),
@@ -34,7 +37,6 @@ def make(name):
 
 @pytest.mark.parametrize("name", sorted(JOBS))
 def test_lists_by_output(prod, oracle_exec, name):
-    zz = pytest.importorskip("test_zz_no_alloc")
     job = make(name)
     zz._check(prod, name, job)
     plain = dict(job, allow_opt=zz.NO_OPT)
