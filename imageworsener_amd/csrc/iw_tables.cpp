@@ -6,9 +6,9 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <exception>
 #include <map>
 #include <mutex>
-#include <system_error>
 #include <thread>
 #include <tuple>
 
@@ -219,17 +219,27 @@ WeightList build_weight_list(const iwamd_resize &rs, int channeltype, double edg
 		build(wl, 0, rs.num_out);
 	} else {
 		std::vector<WeightList> p(parts);
+		std::vector<std::exception_ptr> failed(parts);
+		auto run = [&](int k) {
+			try {
+				build(p[k], (int)((long long)rs.num_out * k / parts), (int)((long long)rs.num_out * (k + 1) / parts));
+			} catch (...) {
+				failed[k] = std::current_exception();
+			}
+		};
 		std::vector<std::thread> th;
-		auto at = [&](int k) { return (int)((long long)rs.num_out * k / parts); };
+		th.reserve(parts);
 		for (int k = 1; k < parts; k++) {
 			try {
-				th.emplace_back([&, k] { build(p[k], at(k), at(k + 1)); });
-			} catch (const std::system_error &) {
-				build(p[k], at(k), at(k + 1));  // no thread to be had
+				th.emplace_back(run, k);
+			} catch (...) {
+				run(k);  // no thread to be had
 			}
 		}
-		build(p[0], 0, at(1));
+		run(0);
 		for (auto &t : th) t.join();
+		for (const std::exception_ptr &e : failed)
+			if (e) std::rethrow_exception(e);  // as from a list built by the caller alone
 		for (const WeightList &q : p) {
 			const int base = (int)wl.src.size();
 			for (int v : q.start) wl.start.push_back(base + v);

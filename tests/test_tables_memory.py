@@ -1,0 +1,29 @@
+"""Weight lists when memory runs out (tests/tables_oom.cpp): an exception in one
+of the threads that build a long list reaches the caller, as it does from a
+list built by the caller alone, and does not end the process."""
+import os
+import subprocess
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+ROOT = os.path.dirname(HERE)
+CSRC = os.path.join(ROOT, "imageworsener_amd", "csrc")
+
+
+@pytest.fixture(scope="module")
+def exe(tmp_path_factory):
+    out = str(tmp_path_factory.mktemp("tables") / "tables_oom")
+    subprocess.run(["g++", "-std=c++17", "-O1", "-g", "-ffp-contract=off", "-w", "-I" + CSRC,
+                    "-I" + os.path.join(ROOT, "include"), os.path.join(HERE, "tables_oom.cpp"),
+                    os.path.join(CSRC, "iw_tables.cpp"), "-o", out, "-lpthread"], check=True)
+    return out
+
+
+def _run(exe, name):
+    r = subprocess.run([exe, name], stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True, timeout=120)
+    assert r.returncode == 0, (r.returncode, r.stdout[-2000:])
+
+
+def test_threads(exe):
+    _run(exe, "threads")
