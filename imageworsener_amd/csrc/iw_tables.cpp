@@ -169,7 +169,9 @@ WeightList build_weight_list(const iwamd_resize &rs, int channeltype, double edg
 	// Outputs [o0, o1) of the list into part (start from 0).
 	auto build = [&](WeightList &part, int o0, int o1) {
 	part.start.resize(o1 - o0);
-	const size_t guess = (size_t)((o1 - o0) * (2.0 * f.radius * reduction + 2.0));
+	double taps = 2.0 * f.radius * reduction + 2.0;
+	if (rs.edge_policy == IW_EDGE_POLICY_STANDARD) taps = std::min(taps, (double)rs.num_in);  // all inside
+	const size_t guess = (size_t)((o1 - o0) * taps);
 	if (guess < ((size_t)1 << 26)) {
 		part.src.reserve(guess);
 		part.pos.reserve(guess);

@@ -75,8 +75,25 @@ static int threads()
 	return failed >= n ? 0 : 2;
 }
 
+// Blurs up to the widest: what is asked for at once is no more than the list
+// itself could come to (its entries lie inside the image).
+static int reserve()
+{
+	for (double blur : {1.0, 30.0, 1000.0, 10000.0})
+		for (int out : {1, 40, 1000}) {
+			const iwamd_resize r = resize(IW_RESIZETYPE_LANCZOS, blur, 1000, out);
+			g_largest = 0;
+			const iwx::WeightList l = iwx::build_weight_list(r, 0, 0.0);
+			const size_t most = sizeof(double) * (size_t)out * (1000 + 2);
+			printf("blur %g, %d outputs: %zu entries, largest request %zu\n", blur, out, l.w.size(), g_largest.load());
+			if (g_largest > most) return 1;
+		}
+	return 0;
+}
+
 int main(int argc, char **argv)
 {
 	if (argc == 2 && !strcmp(argv[1], "threads")) return threads();
+	if (argc == 2 && !strcmp(argv[1], "reserve")) return reserve();
 	return 3;
 }

@@ -1,6 +1,7 @@
 """Weight lists when memory runs out (tests/tables_oom.cpp): an exception in one
 of the threads that build a long list reaches the caller, as it does from a
-list built by the caller alone, and does not end the process."""
+list built by the caller alone, and does not end the process.  And the memory
+asked for ahead is bounded by the list's own size."""
 import os
 import subprocess
 
@@ -27,3 +28,7 @@ def _run(exe, name):
 
 def test_threads(exe):
     _run(exe, "threads")
+
+
+def test_reserve(exe):
+    _run(exe, "reserve")
