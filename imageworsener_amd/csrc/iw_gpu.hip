@@ -5502,13 +5502,14 @@ extern "C" int iwamd_job_finish(struct iwamd_job *J)
 extern "C" void iwamd_job_destroy(struct iwamd_job *J)
 {
 	if (!J) return;
-	if (J->stream) hipStreamSynchronize(J->stream);
+	const bool idle = !J->stream || hipStreamSynchronize(J->stream) == hipSuccess;
 	dev_release(J->block, J->block_bytes);
 	delete (WorkSet *)J->ws;
 	JobStream js;
 	js.stream = J->stream;
 	for (int k = 0; k < 4; k++) js.ev[k] = J->ev[k];
-	job_stream_put(J->device, js);
+	if (idle) job_stream_put(J->device, js);
+	else job_stream_free(js);  // not for another job to find its error
 	delete J;
 }
 

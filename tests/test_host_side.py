@@ -178,5 +178,30 @@ def test_noalloc_lists(scenario):
     scenario("s_noalloc_lists")
 
 
+def s_failed_stream(M):
+    """A job's stream and events go to the next job, but not those of a job
+    whose last wait failed."""
+    import cases
+    job = cases.c0_job()
+
+    def one(errors):
+        j = M.lib.device_job(job)
+        j.run()
+        M.m.mock_sync_errors(errors)
+        j.close()
+        M.m.mock_sync_errors(0)
+        return M.m.mock_streams_made(), M.m.mock_streams_freed()
+
+    assert one(0) == (1, 0)
+    assert one(0) == (1, 0)
+    assert one(1) == (1, 1)
+    assert one(0) == (2, 1)
+    assert one(0) == (2, 1)
+
+
+def test_failed_stream(scenario):
+    scenario("s_failed_stream")
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]](Mock(sys.argv[1]), *sys.argv[3:])
