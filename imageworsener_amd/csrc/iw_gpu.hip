@@ -3855,16 +3855,18 @@ __global__ void __launch_bounds__(256) conv_kernel(ConvArgs A)
 	conv_pixels<NC, B16>(A, tab, idx);
 }
 
-// Forms the optimised image of the finished one at src on st.
-bool conv_enqueue(const iwx_out_conv &conv, const iw_context *ctx, const void *src, void *dst, hipStream_t st)
+// Forms pixels [first, first + n) of the optimised image of the finished one
+// at src on st, to dst.
+bool conv_enqueue(const iwx_out_conv &conv, const iw_context *ctx, const void *src, size_t first, size_t n, void *dst,
+	hipStream_t st)
 {
+	const int nc = iw_imgtype_num_channels(ctx->img2.imgtype), b16 = ctx->img2.bit_depth == 16;
 	ConvArgs A;
-	A.src = (const unsigned char *)src;
+	A.src = (const unsigned char *)src + first * nc * (b16 ? 2 : 1);
 	A.dst = (unsigned char *)dst;
-	A.npx = (unsigned long long)ctx->img2.width * ctx->img2.height;
+	A.npx = n;
 	A.c = conv;
 	const unsigned int grid = (unsigned int)((A.npx + 256 * CONV_PPT - 1) / (256 * CONV_PPT));
-	const int nc = iw_imgtype_num_channels(ctx->img2.imgtype), b16 = ctx->img2.bit_depth == 16;
 	typedef void (*Kernel)(ConvArgs);
 	static const Kernel k[8] = {conv_kernel<1, 0>, conv_kernel<1, 1>, conv_kernel<2, 0>, conv_kernel<2, 1>,
 		conv_kernel<3, 0>, conv_kernel<3, 1>, conv_kernel<4, 0>, conv_kernel<4, 1>};
@@ -5464,9 +5466,17 @@ extern "C" int iwamd_job_finish(struct iwamd_job *J)
 			if (!dst) {
 				done = 0;
 			} else if (conv.any) {
+				// In one piece where there is memory for it, else in smaller ones,
+				// down to the scan's own block.
 				cbytes = bytes;
-				cblk = dev_alloc(cbytes);
-				ok = cblk && conv_enqueue(conv, ctx, out, cblk, J->stream) && back(dst, cblk, bytes);
+				while (!(cblk = dev_alloc(cbytes)) && cbytes > 2 * sbytes) cbytes /= 2;
+				void *const buf = cblk ? cblk : sblk;
+				const size_t npx = (size_t)ctx->img2.width * ctx->img2.height, ob = bytes / npx;
+				const size_t room = (cblk ? cbytes : sbytes) / ob, step = room < npx ? room & ~(size_t)255 : npx;
+				for (size_t k = 0; k < npx && ok; k += step) {
+					const size_t n = std::min(step, npx - k);
+					ok = conv_enqueue(conv, ctx, out, k, n, buf, J->stream) && back(dst + k * ob, buf, n * ob);
+				}
 			} else {
 				ok = back(dst, out, bytes);
 			}

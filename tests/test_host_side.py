@@ -203,5 +203,29 @@ def test_failed_stream(scenario):
     scenario("s_failed_stream")
 
 
+def s_finish_memory(M, limit):
+    """An output whose optimised form finds no device memory is formed in
+    pieces, down to the size of the scan's block, and comes back whole.  (The
+    mock's scan sees no colour: RGB becomes grey, 320 x 240 bytes.)"""
+    import cases
+    limit = int(limit)
+    j = M.lib.device_job(cases.c0_job())
+    j.run()
+    M.m.mock_fail_malloc(limit, 1 << 40)
+    r = j.finish()
+    assert r["ok"], r["error"]
+    assert (r["width"], r["height"], r["bpr"], r["imgtype"]) == (320, 240, 320, cases.GRAY)
+    grids = [g[0] for _, _, g in M.launches("conv_kernel")]  # 1024 pixels a workgroup
+    if limit > 76800:
+        assert grids == [75]
+    else:
+        assert len(grids) > 1 and sum(grids) >= 75 and max(grids) * 1024 <= max(limit, 8192) + 1023, grids
+
+
+@pytest.mark.parametrize("limit", [76801, 76800, 20000, 4700])
+def test_finish_memory(scenario, limit):
+    scenario("s_finish_memory", limit)
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]](Mock(sys.argv[1]), *sys.argv[3:])
