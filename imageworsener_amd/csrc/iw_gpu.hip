@@ -4688,12 +4688,15 @@ int ed_variant(const Staged &S, const iwamd_plan &p, int o, bool rows)
 
 // The sample layout of a job whose planes run errdiff_rows_kernel (log2 of
 // its pixels per segment), or 0: rows of up to EDR_MAX_W pixels and at most
-// 257 levels in every error-diffused channel.
+// 257 levels in every error-diffused channel, whose curve ascends from 0 (a
+// colour space given by hand can have a gamma of 0, below 0 or not a number:
+// with such levels a row's rounds need not settle, nor need the pixels past a
+// row's end give an error of 0).
 int ed_rows_shift(const Staged &S, const iwamd_plan &p)
 {
 	if (!S.n_ed || p.out_width > EDR_MAX_W) return 0;
 	for (int e = 0; e < S.n_ed; e++)
-		if (S.qt[S.ed_list[e]]->P > ED_LDS_TABLE) return 0;
+		if (S.qt[S.ed_list[e]]->P > ED_LDS_TABLE || !S.qt[S.ed_list[e]]->ascending) return 0;
 	return p.out_width <= EDR_W4 ? 2 : 3;
 }
 

@@ -379,6 +379,7 @@ std::shared_ptr<const QuantTable> build_quant_table(const iwamd_ochan &oc, bool 
 	if (ed) {
 		q->M.assign(q->P + 1, 2.0);
 		for (int k = 0; k < q->P; k++) q->M[k] = round_up_point(q->lin[k], q->lin[k + 1]);
+		q->ascending = q->lin[0] == 0.0 && q->lin[q->P] <= 1.0 && std::is_sorted(q->lin.begin(), q->lin.end());
 	}
 	std::lock_guard<std::mutex> lock(g_quant_mutex);
 	return g_quant_cache.emplace(key, std::move(q)).first->second;

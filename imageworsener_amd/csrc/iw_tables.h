@@ -76,6 +76,7 @@ struct QuantTable {
 	// (src/imagew-main.c:730-748); both differences are monotone in s, so that
 	// holds exactly for s >= M[k] (M[P] = 2: never).
 	std::vector<double> M;
+	bool ascending = false;      // with M: lin[0] == 0, and lin ascends to at most 1
 	bool code_is_level = false;  // code[k] == k for every k
 	// Bin index over the array the quantiser searches (nc when used, else T),
 	// 2^ix_log2 bins of [0, 1]: ix[b] = #{m : a[m] < b / 2^ix_log2} for

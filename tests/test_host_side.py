@@ -227,5 +227,27 @@ def test_finish_memory(scenario, limit):
     scenario("s_finish_memory", limit)
 
 
+def s_odd_curves(M, gamma, rows):
+    """Output curves given by hand (iw_make_gamma_csdescr keeps its gammas to
+    0.1..10): rows go to errdiff_rows_kernel only where level 0 is at 0 and the
+    levels ascend to 1."""
+    import cases
+    from imageworsener_amd import api
+    job = api.image_job(np.zeros((20, 30, 3), np.uint8), 30, 20, cases.RGB, 8, canvas=(40, 30),
+                        resize=api.resize_both("catrom"), dither=[(api.CH_ALL, 2, 0)],
+                        output_cs=(api.CS["gamma"], float(gamma)))
+    j = M.lib.device_job(job)
+    j.run()
+    got = {n for _, n, _ in M.launches("errdiff")}
+    assert len(got) == 1 and ("errdiff_rows" in got.pop()) == (rows == "1")
+    j.close()
+
+
+@pytest.mark.parametrize("gamma,rows", [(2.2, 1), (0.1, 1), (10.0, 1), (0.01, 1), (0.0, 0), (-1.0, 0), ("inf", 1),
+                                        ("nan", 0)])
+def test_odd_curves(scenario, gamma, rows):
+    scenario("s_odd_curves", gamma, rows)
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]](Mock(sys.argv[1]), *sys.argv[3:])
