@@ -3986,6 +3986,7 @@ struct Staged {
 	std::vector<List> lists[2];  // by IW_DIMENSION_*
 	int list_of[2][IWAMD_MAX_CH] = {};
 	bool batch = false;          // of a batch or a flight (set before stage_job)
+	bool batch_bands = false;    // a job alone whose bands run a batch's kernel (band_rows_alone)
 	bool least_bytes = false;    // no padding of the horizontal lists (set before stage_job)
 	bool h_by_tap = false;       // DevPlan::h_by_tap
 	const iwx::WeightList &wv(int c) const { return lists[IW_DIMENSION_V][list_of[IW_DIMENSION_V][c]].wl; }
@@ -4010,6 +4011,8 @@ struct Staged {
 	bool skip_pixels = false;  // unknown filter: the reference reports and outputs zeros
 	int band_rows = 0;         // rows per band of the fused kernel; 0: two-pass kernels
 	int band_group = 0;        // band_rows as staged, before tuning and band_rows_alone
+	int alone_rows = 0;        // shape_alone's choice: band_rows, and whether a batch's kernel
+	bool alone_batch = false;
 	int fast_ti = 0;           // output columns per chosen-precision tile
 	std::vector<int4> h4i;     // chosen form: the horizontal list by 4-column blocks (DevPlan::h4i)
 	std::vector<float> h4w;
@@ -4188,6 +4191,53 @@ bool build_f64_input(iw_context *ctx, const iwamd_plan &p, Staged &S, bool in_el
 }
 
 int ed_rows_shift(const Staged &S, const iwamd_plan &p);
+int device_cu_count();
+
+// How the bands of a job that runs alone are cut: it has only its own to fill
+// the device.  Bands run in rounds of as many workgroups as the CUs hold -- by
+// registers two a CU in bands of 4 rows, three of 2, four of 1, or as many as
+// its LDS has room for -- and a round of R rows takes about 3 + R (the fixed
+// part is the chain from the plan's fields to the first sums; 4 + R for
+// floating point, whose bands visit the taller group's positions), so the
+// least rounds x (3 + R) is taken, the taller bands where equal.  Narrow images
+// (no more than two columns per thread) do not fill the threads that share a
+// column's weights between rows, and may take a batch's kernel, of 4 rows and
+// four a CU; up to a column per thread also where that is equal.  (Floating
+// point keeps to its own direct colour-in.)
+// Measured, us for R = 4 / 2 / 1 / a batch's 4: RGB 640x480 to 320x240 44.5 /
+// 34.0 / 26.7 / -; 30x1700 to 30x1700 18.4 / 23.8 / 25.2 / 17.1; 30x2400 to
+// 150x2400 44.0 / 34.5 / 39.5 / 26.2; 1000x5000 to 1200x6000 254 / 235 / 256 /
+// 343.  Over 850 sizes and kinds 10 % less than with at least 512 bands,
+// always of this kernel, which made images of 1700 to 5000 narrow rows up to
+// 1.75 times slower than a batch's kernel.
+#define CU_LDS ((size_t)160 << 10)
+
+void shape_alone(const iwamd_plan &p, Staged &S)
+{
+	const int C = p.inter_nch, W = p.inter_width, widest = std::max(W, p.out_width);
+	const bool in8 = S.in_int && p.in_bit_depth == 8;
+	auto cost = [&](int R, int per_cu, size_t lds) {
+		const int fit = std::max(1, std::min(per_cu, (int)(CU_LDS / lds)));
+		const int bands = (p.inter_height + R - 1) / R, slots = device_cu_count() * fit;
+		return (long long)((bands + slots - 1) / slots) * ((S.in_int ? 3 : 4) + R);
+	};
+	long long best = 0;
+	for (int R : {4, 2, 1}) {
+		if (R > S.band_rows) continue;
+		const bool tab = band_has_tab(in8, R, C, W, rt().band_lds_max);
+		const long long c = cost(R, R == 4 ? 2 : (R == 2 ? 3 : 4), band_lds_rows(R, C, W) + (tab ? CIN_LDS : 0));
+		if (!best || c < best) {
+			best = c;
+			S.alone_rows = R;
+		}
+	}
+	if (!S.in_int || S.band_group != 4 || widest > 512) return;
+	const long long c = cost(4, 4, band_lds_rows(4, C, W));
+	if (c < best || (c == best && widest <= 256)) {
+		S.alone_rows = 4;
+		S.alone_batch = true;
+	}
+}
 
 // Build the host tables of a plan, choose its path and lay out its device
 // data (offsets from the job's base).  path: "band", "twopass" or null.
@@ -4335,6 +4385,7 @@ bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path
 			S.shape_forced = true;
 		}
 		S.band_group = S.band_rows;
+		if (S.band_rows && !S.batch && !S.shape_forced) shape_alone(p, S);
 	}
 
 	Layout L;
@@ -4342,9 +4393,9 @@ bool stage_job(iw_context *ctx, const iwamd_plan &p, Staged &S, const char *path
 	S.in_elsewhere = in_elsewhere;
 	// A batch's bands read a horizontal list by output, four taps of one pixel
 	// at a time; the other kernels by tap, so that neighbouring pixels read
-	// neighbouring weights.
-	// (By tap every output has room for the most taps of any.)
-	S.h_by_tap = !S.least_bytes && (!S.batch || (!S.band_rows && S.fast.empty()));
+	// neighbouring weights.  (By tap every output has room for the most taps of
+	// any.)
+	S.h_by_tap = !S.least_bytes && !S.alone_batch && (!S.batch || (!S.band_rows && S.fast.empty()));
 	S.o_in = L.add<uint8_t>(in_elsewhere ? 0 : S.in_bytes);
 	S.o_inter = L.add<float>(S.band_rows ? 0 : (size_t)p.inter_nch * p.inter_height * p.inter_width);
 	S.out_bytes = p.out_bpr * (size_t)p.out_height;
@@ -4702,7 +4753,8 @@ int ed_rows_shift(const Staged &S, const iwamd_plan &p)
 
 struct WorkSet {
 	std::vector<DevPlan> plans;       // host copies; the two-pass kernels take them by value
-	bool batch = false;               // the plans' Staged::batch: their bands run a batch's kernels
+	bool batch = false;               // of a batch or a flight
+	bool batch_bands = false;         // bands run a batch's kernels
 	std::vector<int2> bands[kBandLists][kLdsClasses];  // (plan, first row), by kBandLists and LDS class
 	size_t band_lds[kBandLists][kLdsClasses] = {};  // largest LDS of a band in each list
 	size_t band_lds_alone[kBandLists][kLdsClasses] = {};  // the same with the tables of a job that runs alone
@@ -4753,7 +4805,7 @@ int fast_variant(const Staged &S, const iwamd_plan &p)
 // The band kernel of a plan's bands, decided as fast_variant decides.
 BandKind band_kind(const Staged &S, const iwamd_plan &p)
 {
-	if (!S.batch) return BAND_ALONE;
+	if (!S.batch && !S.batch_bands) return BAND_ALONE;
 	DevPlan D;
 	fill_dev_plan(S, p, (char *)(uintptr_t)0x100000000ull, D);
 	EmitSimple ES;
@@ -4767,6 +4819,7 @@ int ws_add(WorkSet &W, const Staged &S, const iwamd_plan &p)
 	const int jx = (int)W.plans.size();
 	W.plans.push_back(DevPlan());
 	W.batch = S.batch;
+	W.batch_bands = S.batch || S.batch_bands;
 	if (S.skip_pixels) return jx;
 	if (!S.fast.empty()) {
 		const int var = fast_variant(S, p);
@@ -4945,7 +4998,7 @@ void ws_enqueue_resample(const WorkSet &W, hipStream_t st, bool persistent)
 		for (int q = 0; q < kLdsClasses; q++) {
 			const int n = (int)W.bands[r][q].size();
 			if (!n) continue;
-			const size_t lds = W.batch ? W.band_lds[r][q] : W.band_lds_alone[r][q];
+			const size_t lds = W.batch_bands ? W.band_lds[r][q] : W.band_lds_alone[r][q];
 			const int2 *items = W.d_bands[r][q];
 			int grid = n;
 			if (persistent) {
@@ -4954,7 +5007,7 @@ void ws_enqueue_resample(const WorkSet &W, hipStream_t st, bool persistent)
 			}
 			int *ctr = persistent ? W.d_counters + r * kLdsClasses + q : nullptr;
 			auto launch = [&](auto alone, auto batch, auto any) {
-				hipLaunchKernelGGL(!W.batch ? alone : (r < 3 ? batch : any), dim3(grid), dim3(256), lds, st, W.d_plans,
+				hipLaunchKernelGGL(!W.batch_bands ? alone : (r < 3 ? batch : any), dim3(grid), dim3(256), lds, st, W.d_plans,
 					items, n, ctr);
 			};
 			switch (kBandR[r % 3]) {
@@ -5157,21 +5210,14 @@ bool tune_enabled()
 	return !(v && v[0] == '0');
 }
 
-// A job that runs alone has only its own bands to fill the device: bands of
-// fewer rows, down to one, until there are two for each of the 256 CUs.  A
-// workgroup's chain of loads and sums gets shorter, for more input read twice.
-// 240 rows (640x480 to 320x240, RGB): 52.4 us in bands of 4, 28.9 of 1; 600
-// (RGB floats): 51.6, 25.4; at 1300 and 1536 rows bands of 2 are the best
-// (rgba 100.8 / 99.6 / 109 for 4 / 2 / 1, grey with diffusion 76 / 59 / 73).
-// The positions a row's sum visits stay those of the taller band: where
+// A job that runs alone: shape_alone's bands, or its class's tuned ones.  The
+// positions a row's sum visits stay those of the staged (taller) band: where
 // floating-point samples are not finite, a position of weight 0 counts.
-#define BANDS_ALONE 512
-
-// Where the job's class has been tuned its shape stands.
-void band_rows_alone(const iwamd_plan &p, Staged &S, bool tuned)
+void band_rows_alone(Staged &S, bool tuned)
 {
-	if (tuned || S.shape_forced || !S.band_rows || !S.fast.empty()) return;
-	while (S.band_rows > 1 && (p.inter_height + S.band_rows - 1) / S.band_rows < BANDS_ALONE) S.band_rows /= 2;
+	if (tuned || !S.alone_rows) return;
+	S.band_rows = S.alone_rows;
+	S.batch_bands = S.alone_batch;
 }
 
 // Gives the plan its class's tuned shape; a class without one is measured on
@@ -5220,7 +5266,7 @@ bool job_upload(iwamd_job *J, bool wait)
 	if (!stage_job(ctx, p, S, iw_get_option(ctx, "amd:resample"))) return false;
 	{
 		const char *t = iw_get_option(ctx, "amd:tune");
-		band_rows_alone(p, S, tune_apply(p, S, J->stream, t && atoi(t) == 1));
+		band_rows_alone(S, tune_apply(p, S, J->stream, t && atoi(t) == 1));
 	}
 	J->skip_pixels = S.skip_pixels;
 	J->n_ed = S.n_ed;
@@ -5646,7 +5692,7 @@ extern "C" int iwamd_process_device_noalloc(struct iw_context *ctx, const void *
 	Staged S;
 	if (!stage_job(ctx, p, S, iw_get_option(ctx, "amd:resample"), true, true)) return 0;
 	// Look the shape up; never tune (tuning allocates).
-	band_rows_alone(p, S, tune_apply(p, S, st, false));
+	band_rows_alone(S, tune_apply(p, S, st, false));
 	WorkSet W;
 	auto lay_out = [&]() {
 		W = WorkSet();

@@ -249,5 +249,40 @@ def test_odd_curves(scenario, gamma, rows):
     scenario("s_odd_curves", gamma, rows)
 
 
+def s_alone_shapes(M):
+    """The bands of single jobs (shape_alone): rounds of what 256 CUs hold at
+    once, and a batch's kernel for narrow images with many rows."""
+    import cases
+    from imageworsener_amd import api
+    for w, ow, oh, kind, want in [
+            (40, 30, 24, None, (1, "0")), (40, 30, 1024, None, (1, "0")), (40, 30, 1025, None, (2, "0")),
+            (40, 30, 1536, None, (2, "0")), (40, 30, 1537, None, (4, "1")), (40, 30, 2048, None, (4, "1")),
+            (40, 30, 2049, None, (4, "1")), (40, 30, 2049, "o", (4, "2")), (40, 30, 2049, "float", (2, "0")),
+            (300, 400, 1700, None, (4, "0")), (300, 400, 2049, None, (4, "1")), (300, 600, 2049, None, (2, "0")),
+            (2000, 1500, 3000, None, (1, "0")), (2000, 1500, 1000, None, (1, "0"))]:
+        img = np.zeros(w * 20 * 3 * (4 if kind == "float" else 1), np.uint8)
+        job = api.image_job(img, w, 20, cases.RGB, 32 if kind == "float" else 8, canvas=(ow, oh),
+                            resize=api.resize_both("catrom"))
+        if kind == "float":
+            job["image"]["sampletype"] = 1
+            job["input_cs"] = (api.CS["linear"], 0.0)
+        if kind == "o":
+            job["dither"] = [(api.CH_ALL,) + api.DITHER["o"]]
+        M.m.mock_clear_log()
+        j = M.lib.device_job(job)
+        j.run()
+        (i, name, grid), = M.launches("11band_kernel")
+        got = int(name.split("band_kernelILi")[1][0]), name.split("BandKindE")[1][0]
+        assert got == want and grid[0] == -(-oh // got[0]), (w, ow, oh, kind, got, grid)
+        n, p = M.m.mock_launch_count(i), M.m.mock_launch_items(i)
+        items = np.ctypeslib.as_array((ctypes.c_int * (2 * n)).from_address(p)).reshape(n, 2)
+        assert n == grid[0] and items.tolist() == [[0, k * got[0]] for k in range(n)]
+        j.close()
+
+
+def test_alone_shapes(scenario):
+    scenario("s_alone_shapes")
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]](Mock(sys.argv[1]), *sys.argv[3:])
