@@ -859,38 +859,46 @@ __global__ void __launch_bounds__(256) hpass_kernel(DevPlan P)
 }
 
 // The two-pass form's horizontal pass where the channels share the list and
-// the per-pixel work is simple: HP_ROWS rows per thread, four taps per load.
+// the per-pixel work is simple: RR rows per thread, four taps per load.
 // Bound by the requests for intermediate samples to L2 (with one tap per load
 // each line was asked for by every tap: 119 and 167 us for the sizes below)
 // and, per pixel, the dependent table searches; with a pixel per thread and a
 // list read per channel it was bound by the lists.  4000 to 1000 columns, 750
-// rows, RGB, Lanczos3: 316 -> 35 us; 4096 to 1000, 1000 rows, RGBA, Mitchell:
-// 318 -> 54 us.
-#define HP_ROWS 4
+// rows, RGB, Lanczos3: 316 -> 31 us; 4096 to 1000, 1000 rows, RGBA, Mitchell:
+// 333 -> 40 us.
+template <int RR>
 __global__ void __launch_bounds__(256) hpass_rows_kernel(DevPlan P)
 {
 	const int i = blockIdx.x * blockDim.x + threadIdx.x;
-	const int j0 = blockIdx.y * HP_ROWS;
+	const int j0 = blockIdx.y * RR;
 	if (i >= P.out_w) return;
 	EmitSimple E;
 	emit_simple_ctx(P, E);
 	const InterRows rows = {P.inter + (size_t)j0 * P.W, (size_t)P.Hp * P.W, (size_t)P.W, P.out_h - 1 - j0};
-	hrows<HP_ROWS, false, false>(P, E, i, j0, min(HP_ROWS, P.out_h - j0), rows);
+	hrows<RR, false, false>(P, E, i, j0, min(RR, P.out_h - j0), rows);
 }
 
-// Queue the two-pass form's horizontal pass.  (Floating-point samples may not
-// be finite, so those plans keep to the list's own entries; the generic
-// per-pixel work is too large to repeat for several rows: with both in one
-// kernel it kept 1936 bytes per thread in scratch memory, 202 us for the first
-// size above.)
+// Queue the two-pass form's horizontal pass.  Two rows per thread share the
+// weights, but one after the other's per-pixel work: while single rows leave
+// no more than HPASS_ROWS1 workgroups (six a CU) those are faster.  2500 to
+// 2500 columns, RGB, 1 / 2 / 4 rows: 30 rows 11.9 / 15.0 / 21.0 us, 120 rows
+// 14.8 / 17.1 / 23.4, 300 rows 24.3 / 21.7 / 25.4, 1500 rows 83.6 / 72.4 /
+// 83.9.  (Floating-point samples may not be finite, so those plans keep to the
+// list's own entries; the generic per-pixel work is too large to repeat for
+// several rows: with both in one kernel it kept 1936 bytes per thread in
+// scratch memory, 202 us for the first size above.)
+#define HPASS_ROWS1 1536
+
 void enqueue_hpass(const DevPlan &D, hipStream_t st)
 {
 	EmitSimple E;
 	const int nx = (D.out_w + 255) / 256;
-	if (D.h_shared && !D.in_float && emit_simple_ctx(D, E))
-		hipLaunchKernelGGL(hpass_rows_kernel, dim3(nx, (D.out_h + HP_ROWS - 1) / HP_ROWS), dim3(256), 0, st, D);
-	else
+	if (!D.h_shared || D.in_float || !emit_simple_ctx(D, E))
 		hipLaunchKernelGGL(hpass_kernel, dim3(nx, D.out_h), dim3(256), 0, st, D);
+	else if ((long long)nx * D.out_h <= HPASS_ROWS1)
+		hipLaunchKernelGGL(hpass_rows_kernel<1>, dim3(nx, D.out_h), dim3(256), 0, st, D);
+	else
+		hipLaunchKernelGGL(hpass_rows_kernel<2>, dim3(nx, (D.out_h + 1) / 2), dim3(256), 0, st, D);
 }
 
 // ---- fused band kernel ------------------------------------------------------

@@ -284,5 +284,25 @@ def test_alone_shapes(scenario):
     scenario("s_alone_shapes")
 
 
+def s_hpass_rows(M):
+    """The two-pass form's horizontal pass: a row per thread while that gives at
+    most six workgroups a CU, then two."""
+    import cases
+    from imageworsener_amd import api
+    for ow, oh, rows in [(256, 1, 1), (256, 1536, 1), (256, 1537, 2), (257, 768, 1), (257, 769, 2), (4000, 100, 2)]:
+        job = api.image_job(np.zeros((20, 30, 3), np.uint8), 30, 20, cases.RGB, 8, canvas=(ow, oh),
+                            resize=api.resize_both("catrom"), options=[("amd:resample", "twopass")])
+        M.m.mock_clear_log()
+        j = M.lib.device_job(job)
+        j.run()
+        (_, name, grid), = M.launches("hpass")
+        assert "hpass_rows_kernelILi%dE" % rows in name and grid[:2] == (-(-ow // 256), -(-oh // rows)), (ow, oh, name, grid)
+        j.close()
+
+
+def test_hpass_rows(scenario):
+    scenario("s_hpass_rows")
+
+
 if __name__ == "__main__":
     globals()[sys.argv[2]](Mock(sys.argv[1]), *sys.argv[3:])
