@@ -2913,14 +2913,17 @@ struct EdrEdge {
 };
 
 // D[0] = -1, D[1 + k] = boundary k, then 4.0: every sample lies in some range.
-template <int NW>
-struct EdrLds {
+struct EdrTables {
 	double D[ED_LDS_TABLE + 4];
 	double lin[ED_LDS_TABLE + 2];
 	double lo[ED_LDS_TABLE + 1], hi[ED_LDS_TABLE + 1];  // level k's exact samples: [lo[k], hi[k])
 	unsigned short Q[1 + ED_NB];             // first guess of b: 0 below 0, then by s * ED_NB
 	unsigned short code[ED_LDS_TABLE + 1];   // output code per level
 	unsigned long long eps;                  // bits of the widest distance of an exact sample from its level
+};
+
+template <int NW>
+struct EdrLds : EdrTables {
 	EdrEdge edge[2][NW];
 	double hold[NW + 1][2];  // a wave's predecessor's state once it is fixed; [NW]: zero
 };
@@ -3283,8 +3286,38 @@ __global__ void __launch_bounds__(256) edr_interleave_kernel(const DevPlan *__re
 	for (int t = threadIdx.x; t < q * rows; t += 256) edr_interleave4(P, it.y + t / q, (t % q) * 4);
 }
 
-// One plane on the workgroup's first NW waves: rows of at most 64 * NW * SEG
-// pixels.
+// The plane's tables, by all EDR_THREADS threads (by the 64 that walk narrow
+// rows alone it took 64 us); ends with a barrier.
+__device__ __forceinline__ void edr_tables(const DevOChan &q, EdrTables &S)
+{
+	const int tid = threadIdx.x, Pq = q.P;
+	g_cf64 *T = (g_cf64 *)q.T, *U = (g_cf64 *)q.U, *M = (g_cf64 *)q.M, *lin = (g_cf64 *)q.lin;
+	if (tid == 0) S.eps = 0;
+	__syncthreads();
+	double eps = 0.0;
+	for (int k = tid; k <= Pq; k += EDR_THREADS) {
+		// The top level's exact samples end at 1.0 (U[P] is infinite).
+		S.lo[k] = k ? T[k - 1] : 0.0;
+		S.hi[k] = U[k];
+		S.lin[k] = lin[k];
+		eps = fmax(eps, fmax(fabs(S.lo[k] - lin[k]), fabs((k < Pq ? U[k] : 1.0) - lin[k])));
+		S.code[k] = (unsigned short)(0.5 + ((g_cf64 *)q.code)[k]);
+	}
+	atomicMax(&S.eps, (unsigned long long)__double_as_longlong(eps));
+	for (int k = tid; k < Pq + 3; k += EDR_THREADS) {
+		double d = k == 0 ? -1.0 : 4.0;
+		if (k > 0 && k <= Pq) d = fmin(T[k - 1], fmax(k > 1 ? T[k - 2] : 0.0, fmax(U[k - 1], M[k - 1])));
+		S.D[k] = d;
+	}
+	// The level below the bin's middle: its upper boundary is the nearest.
+	if (tid == 0) S.Q[0] = 0;
+	for (int k = tid; k < ED_NB; k += EDR_THREADS)
+		S.Q[1 + k] = (unsigned short)(level_in(q.lin, 1, Pq, (k + 0.5) / (double)ED_NB) - 1);
+	__syncthreads();
+}
+
+// One plane on the workgroup's first NW waves, its tables in place: rows of at
+// most 64 * NW * SEG pixels.
 template <bool M1, int SEG, int NW>
 __device__ __forceinline__ void edr_plane(const DevPlan &P, int o, EdrLds<NW> &S)
 {
@@ -3292,8 +3325,6 @@ __device__ __forceinline__ void edr_plane(const DevPlan &P, int o, EdrLds<NW> &S
 	constexpr int NT = 64 * NW;
 	const int tid = threadIdx.x;
 	const DevOChan &q = P.oc[o];
-	const int Pq = q.P;
-	g_cf64 *T = (g_cf64 *)q.T, *U = (g_cf64 *)q.U, *M = (g_cf64 *)q.M, *lin = (g_cf64 *)q.lin;
 
 	EdrCtx c;
 	c.m = c_ed_matrix[(q.subtype >= 0 && q.subtype <= 7) ? q.subtype : 0];
@@ -3308,29 +3339,8 @@ __device__ __forceinline__ void edr_plane(const DevPlan &P, int o, EdrLds<NW> &S
 	c.n = max(0, min(SEG, c.W - c.x0));
 	c.par = 0;
 
-	if (tid == 0) S.eps = 0;
 	if (tid < 2) S.hold[NW][tid] = 0.0;
 	for (int t = tid; t < (int)(sizeof(S.edge) / sizeof(double)); t += NT) (&S.edge[0][0].first[0])[t] = 0.0;
-	__syncthreads();
-	double eps = 0.0;
-	for (int k = tid; k <= Pq; k += NT) {
-		// The top level's exact samples end at 1.0 (U[P] is infinite).
-		S.lo[k] = k ? T[k - 1] : 0.0;
-		S.hi[k] = U[k];
-		S.lin[k] = lin[k];
-		eps = fmax(eps, fmax(fabs(S.lo[k] - lin[k]), fabs((k < Pq ? U[k] : 1.0) - lin[k])));
-		S.code[k] = (unsigned short)(0.5 + ((g_cf64 *)q.code)[k]);
-	}
-	atomicMax(&S.eps, (unsigned long long)__double_as_longlong(eps));
-	for (int k = tid; k < Pq + 3; k += NT) {
-		double d = k == 0 ? -1.0 : 4.0;
-		if (k > 0 && k <= Pq) d = fmin(T[k - 1], fmax(k > 1 ? T[k - 2] : 0.0, fmax(U[k - 1], M[k - 1])));
-		S.D[k] = d;
-	}
-	// The level below the bin's middle: its upper boundary is the nearest.
-	if (tid == 0) S.Q[0] = 0;
-	for (int k = tid; k < ED_NB; k += NT)
-		S.Q[1 + k] = (unsigned short)(level_in(q.lin, 1, Pq, (k + 0.5) / (double)ED_NB) - 1);
 	__syncthreads();
 	c.eps_hi = (unsigned int)(S.eps >> 32) + 1u;
 
@@ -3365,6 +3375,7 @@ __global__ void __launch_bounds__(EDR_THREADS) errdiff_rows_kernel(const DevPlan
 	const int2 pl = planes[blockIdx.x];
 	const DevPlan &P = plans[pl.x];
 	const int W = P.out_w, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	edr_tables(P.oc[pl.y], *(EdrTables *)lds);
 	// The widest shape's code first: behind the others 3072-px rows took 9.7 us
 	// instead of 8.7.
 	if (W > 2048) {
