@@ -1231,7 +1231,7 @@ __device__ __forceinline__ void band_span(const DevWeights &dv, int a, int b, in
 // then).
 // Bound by the table gathers, then the FP64 sums: with the tables in LDS and
 // only the plan's own channels looked up (five gathers per pixel before,
-// whatever the channels), 4000x3000 RGB to 750 rows: 159 -> 88 us; 16-bit
+// whatever the channels), 4000x3000 RGB to 750 rows: 159 -> 84 us; 16-bit
 // (tables in L2), 1500 to 375 rows: 180 -> 138 us; the fused kernel for 3072
 // squared of grey 475 -> 390 us, 1023x767 floats (through colour_in before)
 // 135 -> 55 us, 640x480 RGB to 320x240 65 -> 52 us.
@@ -2892,9 +2892,9 @@ __global__ void __launch_bounds__(ED_THREADS) errdiff_kernel(const DevPlan *__re
 // over as many waves as give each its own SIMD: segments of 4 pixels up to
 // 1024 wide, of 8 beyond (16 pixels on 4 waves do not fit the registers:
 // 3072-wide rows 10.0 us against 8.7).  Measured per row, errdiff_kernel ->
-// this kernel: Floyd-Steinberg 1000 pixels 16.7 -> 4.0 us, 2500 pixels
-// 22.2 -> 5.6 us, 200 pixels 12.7 -> 2.9 us; Jarvis-Judice-Ninke to 4 levels,
-// 3072 pixels, 23.1 -> 8.7 us.
+// this kernel: Floyd-Steinberg 1000 pixels 16.7 -> 3.7 us, 2500 pixels
+// 22.2 -> 5.7 us, 200 pixels 12.7 -> 2.8 us; Jarvis-Judice-Ninke to 4 levels,
+// 3072 pixels, 23.1 -> 8.8 us.
 //
 // The samples come segment-transposed (ed_sample_at), so that a wave's loads
 // are consecutive, and the codes go out planar over the samples already
