@@ -779,7 +779,8 @@ struct BandRows {
 // order of the operands in the machine code).
 // load(c, r, x): sample x of intermediate row r.  Columns whose list lies
 // inside the row read four samples at a time (load.four), so that a cache line
-// is asked for once per four taps.  Then the rows' pixels one by one.
+// is asked for once per four taps.  BY_OUT: the list lies by output (a batch's
+// bands; else as DevPlan::h_by_tap says).  Then the rows' pixels one by one.
 template <int RR, bool SKIP, bool BY_OUT, class Emit, class Load>
 __device__ __forceinline__ void hrows(const DevPlan &P, const Emit &E, int i, int j0, int n, Load load)
 {

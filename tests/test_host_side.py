@@ -121,7 +121,7 @@ def s_tune_alone(M):
         return int(last[-1][1].split("band_kernelILi")[1][0]), last[-1][2][0], timed
 
     job = cases.c0_job()
-    assert bands(job) == (1, 240, 0)  # the rule of band_rows_alone
+    assert bands(job) == (1, 240, 0)  # shape_alone's
     M.m.mock_event_ms(cb)
     tuned = dict(job, options=[("amd:tune", "1")])
     for f in (4, 2):
